@@ -316,7 +316,7 @@ int hexa_moe_depth_ws_bytes(const hexa_moe_depth_desc* d, int64_t* forward_bytes
  * idx [T][k] int32, thr [T] (load-importance only, else NULL) and stats (GShard: me[E], ce[E], l_aux = 2E+1 floats;
  * load-importance: importance, load, their two gradients, l_aux = 4E+1 floats) are outputs the backward needs.
  * With wg == NULL the routing decision is the caller's: idx is read ([T][k] int32) and logits / scores / thr /
- * stats / noise are ignored.
+ * stats / noise are ignored; with idx == NULL as well, `route` holds the caller's decision already (hexa_route_build).
  * Then: route = hexa_route_build(idx); y1 = x.W1^T + b1 and y2 = gelu(y1) ([k][T][hidden], saved for the backward);
  * y [T][d_out] = sum over slots of y2.W2 + b2.  Biases may be NULL.
  * plan (may be NULL): HEXA_ESTMM_PLAN_INTS(num_experts) ints that receive the work plan of the backward's ESTMM

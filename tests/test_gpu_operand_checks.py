@@ -74,3 +74,36 @@ def test_what_an_activation_returns_is_checked(dev, change, monkeypatch):
     monkeypatch.setitem(ACTS, "odd", lambda t: change(F.gelu(t)))
     with pytest.raises(RuntimeError, match="hexa_moe"):
         _run(o, "odd", False)
+
+
+@pytest.mark.parametrize("act", list(ACTS))
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.int16, torch.uint8, torch.bool])
+def test_a_decision_in_another_type_is_refused(dev, act, dtype):
+    o = _operands(dev)
+    o["chosen"] = o["chosen"].to(dtype)
+    with pytest.raises(TypeError, match="int32 or int64"):
+        _run(o, act, False)
+
+
+@pytest.mark.parametrize("act", list(ACTS))
+def test_a_decision_is_read_in_its_own_type_and_strides(dev, act):
+    """Top-1, with ids that are no expert's: an int64 id whose low 32 bits name an expert is not that expert's."""
+    def run(chosen):
+        o = _operands(dev)
+        o["chosen"] = chosen
+        ws = [o[n].requires_grad_(True) for n in ("w1", "w2", "b1", "b2")]
+        y = _run(o, act, False)
+        y.backward(o["x"])
+        return [y.detach()[kept]] + [w.grad for w in ws]
+
+    ids = _operands(dev)["chosen"][:, :1].clone()
+    kept = torch.ones(T, dtype=torch.bool, device=dev)
+    kept[[3, 4, T - 1]] = False
+    low = torch.where(kept[:, None], ids, torch.full_like(ids, -1)).to(torch.int32)
+    want = run(low)
+    high = torch.where(kept[:, None], ids, ids + (1 << 32))
+    wide = torch.full((2, T + 1), 99, dtype=torch.int64, device=dev)
+    wide[1, :T] = high[:, 0]
+    for chosen in (high, wide[1:, :T].t(), low.expand(T, 4)[:, 2:3]):
+        for a, b in zip(run(chosen), want):
+            assert torch.equal(a, b)
