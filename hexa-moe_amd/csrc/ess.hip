@@ -99,13 +99,14 @@ template <typename T>
 __global__ __launch_bounds__(256) void sum_slots_kernel(SumSlotsK p) { sum_slots_body<T>(p, blockIdx.x); }
 
 template <typename T>
-int launch_sum_slots_t(void* out, const void* ws, int64_t n, int nws, const void* extra, int dt, hipStream_t st) {
-    if (n == 0 || (nws == 0 && !extra)) return HEXA_OK;
-    if (n % Vec16<T>::N) HEXA_FAIL(HEXA_ERR_UNSUPPORTED, "sum_slots: size must be a multiple of the vector width");
-    int64_t blocks = (n / Vec16<T>::N + 255) / 256;
+int launch_sum_slots_t(SumSlotsK p, int dt, hipStream_t st) {
+    if (p.n == 0 || (p.nws == 0 && !p.extra)) return HEXA_OK;
+    if ((p.offsets ? p.N : p.n) % Vec16<T>::N) HEXA_FAIL(HEXA_ERR_UNSUPPORTED, "sum_slots: rows must be multiples of the vector width");
+    int64_t blocks = (p.n / Vec16<T>::N + 255) / 256;
     if (blocks > 256 * 16) blocks = 256 * 16;
+    p.blocks = (int)blocks;
     SmallTask t;
-    t.kind = TASK_SUM_SLOTS; t.sum_slots = SumSlotsK{out, ws, n, nws, extra, (int)blocks}; t.blocks = (int)blocks;
+    t.kind = TASK_SUM_SLOTS; t.sum_slots = p; t.blocks = (int)blocks;
     if (!defer_task(defer_targets().sum_slots, t, dt)) {
         hipLaunchKernelGGL((sum_slots_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, st, t.sum_slots);
         HEXA_CHECK_LAUNCH("sum_slots");
@@ -115,10 +116,15 @@ int launch_sum_slots_t(void* out, const void* ws, int64_t n, int nws, const void
 
 }  // namespace
 
-int launch_sum_slots(void* out, const void* ws, int64_t n, int nws, int dt, hipStream_t st, const void* extra) {
-    if (dt == HEXA_F32) return launch_sum_slots_t<float>(out, ws, n, nws, extra, dt, st);
-    if (dt == HEXA_BF16) return launch_sum_slots_t<__bf16>(out, ws, n, nws, extra, dt, st);
-    return launch_sum_slots_t<_Float16>(out, ws, n, nws, extra, dt, st);
+static int launch_sum_slots_d(const SumSlotsK& p, int dt, hipStream_t st) {
+    if (dt == HEXA_F32) return launch_sum_slots_t<float>(p, dt, st);
+    return dt == HEXA_BF16 ? launch_sum_slots_t<__bf16>(p, dt, st) : launch_sum_slots_t<_Float16>(p, dt, st);
+}
+int launch_sum_slots(void* out, const void* ws, const RouteView& r, int N, bool accumulate, int dt, hipStream_t st, const void* extra) {
+    return launch_sum_slots_d(SumSlotsK{out, ws, (int64_t)r.T * N, r.k - 1, extra, 0, r.offsets, r.token_ids, r.T, r.E, N, accumulate ? 1 : 0}, dt, st);
+}
+int launch_add(void* out, const void* extra, int64_t n, int dt, hipStream_t st) {
+    return launch_sum_slots_d(SumSlotsK{out, nullptr, n, 0, extra, 0, nullptr, nullptr, 0, 0, 0, 1}, dt, st);
 }
 
 // out (+)= the sum of `parts` partial results of n values each, in their order

@@ -315,7 +315,7 @@ int launch_ffn16_fused(void* y1, void* y2, void* y, const void* x, const void* w
     if (units == 0) return HEXA_OK;
     const int rc = act_dt == HEXA_BF16 ? launch_ffn_d<__bf16>(p, (int)units, st) : launch_ffn_d<_Float16>(p, (int)units, st);
     if (rc) return rc;
-    if (r.k > 1) return launch_sum_slots(y, slot_ws, (int64_t)r.T * d_out, r.k - 1, act_dt, st);
+    if (r.k > 1) return launch_sum_slots(y, slot_ws, r, d_out, false, act_dt, st);
     return HEXA_OK;
 }
 

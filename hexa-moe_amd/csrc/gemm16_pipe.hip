@@ -721,7 +721,7 @@ int launch_esmm16_pipe(const EsmmArgs& a, hipStream_t st) {
     else rc = io ? launch_pipe_a<_Float16, true>(pk, grid, act, a.colsum != nullptr, st)
                  : launch_pipe_a<_Float16, false>(pk, grid, act, a.colsum != nullptr, st);
     if (rc) return rc;
-    if (p.ws) return launch_sum_slots(a.out, a.slot_ws, (int64_t)a.r.T * a.out_dim, a.r.k - 1, a.out_dt, st, a.sum_extra);
+    if (p.ws) return launch_sum_slots(a.out, a.slot_ws, a.r, a.out_dim, a.accumulate, a.out_dt, st, a.sum_extra);
     if (a.colsum) return launch_colsum_fold(a, p.mt_ub, HEXA_TILE_ROWS, p.ntn, C::BN, st);
     return HEXA_OK;
 }

@@ -550,7 +550,7 @@ int launch_esmm32(const EsmmArgs& a, hipStream_t st) {
                               : (io ? launch_esmm32_t<true, false, Deep>(p, st) : launch_esmm32_t<false, false, Deep>(p, st));
         if (rc) return rc;
     }
-    if (p.ws) return launch_sum_slots(a.out, a.slot_ws, (int64_t)a.r.T * a.out_dim, a.r.k - 1, HEXA_F32, st, a.sum_extra);
+    if (p.ws) return launch_sum_slots(a.out, a.slot_ws, a.r, a.out_dim, a.accumulate, HEXA_F32, st, a.sum_extra);
     return HEXA_OK;
 }
 

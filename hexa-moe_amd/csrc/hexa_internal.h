@@ -151,7 +151,9 @@ int estmm32_parts(int T, int k, int E, int m_dim, int n_dim);   // parts the fp3
 int launch_fold(void* out, const float* ws, long n, int parts, int dt, int accumulate, hipStream_t st);
 int launch_ess(const EssArgs& a, hipStream_t s);
 int launch_ess_noalloc(EssArgs a, hipStream_t s);
-int launch_sum_slots(void* out, const void* ws, int64_t n, int nws, int dt, hipStream_t s, const void* extra = nullptr);
+// out [T][N] += the other slots' results in ws ([k-1][T][N]) + extra; accumulate: out held something before slot 0's product
+int launch_sum_slots(void* out, const void* ws, const RouteView& r, int N, bool accumulate, int dt, hipStream_t s, const void* extra = nullptr);
+int launch_add(void* out, const void* extra, int64_t n, int dt, hipStream_t s);   // out += extra
 // routing front end of the depth call: the router also counts, the counting sort's scan launch also finishes the loss,
 // its scatter launch also makes the ESTMM plan (see router.hip, route.hip)
 bool router_hist_supported(int E);

@@ -228,10 +228,60 @@ __device__ __forceinline__ void ess_fold_body(const EssFoldK& p, int block) {
 
 // out[i] += ws[0][i] + ws[1][i] + ... in fp32, slot order (the deterministic reduction behind the one-launch slot
 // sum of ESMM).  `extra` (may be null): one more addend of out's shape, added last (the gate path's share of an
-// input gradient)
+// input gradient).  A (token, slot) that is in no list -- its expert id was no expert's -- left its row of ws, or of out,
+// as it was: where a list is short of T entries, sum_listed_slots adds the rows that were written (inlined: a call would
+// give every kernel with this task a stack).
+template <typename T>
+__device__ __forceinline__ void sum_listed_slots(const SumSlotsK& p, int block) {
+    constexpr int V = Vec16<T>::N;
+    T* out = reinterpret_cast<T*>(p.out);
+    const T* ws = reinterpret_cast<const T*>(p.ws);
+    const int64_t nv = p.n / V;
+    const int64_t stride = (int64_t)p.blocks * 256;
+    const int lane = threadIdx.x & 63;
+    // a wavefront looks its rows (consecutive ones) up in each slot's list, 64 entries at a time
+    for (int64_t i0 = (int64_t)block * 256 + (threadIdx.x - lane); i0 < nv; i0 += stride) {
+        const int64_t i = min(i0 + lane, nv - 1);
+        const int row = (int)(i * V / p.N);
+        const int lo = __builtin_amdgcn_readlane(row, 0), hi = __builtin_amdgcn_readlane(row, 63);
+        float acc[V];
+#pragma unroll
+        for (int j = 0; j < V; ++j) acc[j] = 0.f;
+        auto add = [&](const T* from) {
+            union { uint4 u; T e[V]; } w;
+            w.u = reinterpret_cast<const uint4*>(from)[i];
+#pragma unroll
+            for (int j = 0; j < V; ++j) acc[j] += Cvt<T>::to_f(w.e[j]);
+        };
+        for (int s = 0; s <= p.nws; ++s) {
+            const int count = p.offsets[(size_t)s * (p.E + 1) + p.E];
+            const int32_t* ids = p.token_ids + (size_t)s * p.T;
+            bool listed = s == 0 && p.accumulate;
+            for (int r0 = 0; r0 < count; r0 += 64) {
+                const int id = r0 + lane < count ? ids[r0 + lane] : -1;
+                for (unsigned long long m = __ballot(id >= lo && id <= hi); m; m &= m - 1)
+                    listed = listed || __builtin_amdgcn_readlane(id, __ffsll((long long)m) - 1) == row;
+            }
+            if (listed) add(s == 0 ? out : ws + (size_t)(s - 1) * p.n);
+        }
+        if (p.extra) add(reinterpret_cast<const T*>(p.extra));
+        union { uint4 u; T e[V]; } o;
+#pragma unroll
+        for (int j = 0; j < V; ++j) o.e[j] = Cvt<T>::from_f(acc[j]);
+        if (i0 + lane < nv) reinterpret_cast<uint4*>(out)[i] = o.u;
+    }
+}
+
 template <typename T>
 __device__ __forceinline__ void sum_slots_body(const SumSlotsK& p, int block) {
     constexpr int V = Vec16<T>::N;
+    if (p.offsets) {
+        int missing = 0;
+        for (int s0 = 0; s0 <= p.nws; s0 += 8)      // up to 8 list lengths in flight
+#pragma unroll
+            for (int q = 0; q < 8; ++q) missing |= p.T - p.offsets[(size_t)min(s0 + q, p.nws) * (p.E + 1) + p.E];
+        if (missing) return sum_listed_slots<T>(p, block);
+    }
     T* out = reinterpret_cast<T*>(p.out);
     const T* ws = reinterpret_cast<const T*>(p.ws);
     const int64_t nv = p.n / V;

@@ -128,6 +128,9 @@ int hexa_route_from_padded_lists(const int32_t* token_idx_list, const int32_t* e
  * With it, all slots run in ONE launch (slot 0 writes `out`, the others write slot_ws) followed by a
  * small reduction out += sum(slot_ws) in slot order; without it the slots run one launch after the
  * other, each adding into `out`.  Both orders are fixed, so results are reproducible either way.
+ * Rows of (token, slot) pairs that are in no list (ids outside [0, E) in the routing decision) are neither read nor
+ * written: they add nothing to a sum over slots, and with slot_ws a token without any pair gets 0 (accumulate: keeps what
+ * it had).
  * Replaces ESMM_TENSOR_CORE (torch/hexa_moe_ops.cpp:45-117) -> launch_esmm_accum_shared_tensor_{full,
  * mix,half} (include/hexa_moe.h:22-72, kernels/esmm_full.cu:249-300), and with w_layout OUT_IN the
  * ESMM task of FUSED_GRAD (kernels/fused_ops_full.cu:117-247). */
