@@ -240,7 +240,7 @@ __device__ __forceinline__ void sum_listed_slots(const SumSlotsK& p, int block) 
     const int64_t stride = (int64_t)p.blocks * 256;
     const int lane = threadIdx.x & 63;
     // a wavefront looks its rows (consecutive ones) up in each slot's list, 64 entries at a time
-    for (int64_t i0 = (int64_t)block * 256 + (threadIdx.x - lane); i0 < nv; i0 += stride) {
+    for (int64_t i0 = (int64_t)block * 256 + __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u); i0 < nv; i0 += stride) {
         const int64_t i = min(i0 + lane, nv - 1);
         const int row = (int)(i * V / p.N);
         const int lo = __builtin_amdgcn_readlane(row, 0), hi = __builtin_amdgcn_readlane(row, 63);
@@ -275,18 +275,20 @@ __device__ __forceinline__ void sum_listed_slots(const SumSlotsK& p, int block) 
 template <typename T>
 __device__ __forceinline__ void sum_slots_body(const SumSlotsK& p, int block) {
     constexpr int V = Vec16<T>::N;
+    const int lane = threadIdx.x & 63;
+    // the length of slot `lane`'s list (more than 64 slots: the shortest one's)
+    int len = p.T;
     if (p.offsets) {
-        int missing = 0;
-        for (int s0 = 0; s0 <= p.nws; s0 += 8)      // up to 8 list lengths in flight
-#pragma unroll
-            for (int q = 0; q < 8; ++q) missing |= p.T - p.offsets[(size_t)min(s0 + q, p.nws) * (p.E + 1) + p.E];
-        if (missing) return sum_listed_slots<T>(p, block);
+        len = p.offsets[(size_t)min(lane, p.nws) * (p.E + 1) + p.E];
+        if (p.nws >= 64)
+            for (int s = lane + 64; s <= p.nws; s += 64) len = min(len, p.offsets[(size_t)s * (p.E + 1) + p.E]);
     }
     T* out = reinterpret_cast<T*>(p.out);
     const T* ws = reinterpret_cast<const T*>(p.ws);
     const int64_t nv = p.n / V;
     const int64_t stride = (int64_t)p.blocks * 256;
-    for (int64_t i = (int64_t)block * 256 + threadIdx.x; i < nv; i += stride) {
+    for (int64_t i0 = (int64_t)block * 256 + __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u); i0 < nv; i0 += stride) {
+        const int64_t i = min(i0 + lane, nv - 1);
         union { uint4 u; T e[V]; } o, w;
         o.u = reinterpret_cast<const uint4*>(out)[i];
         float acc[V];
@@ -302,9 +304,14 @@ __device__ __forceinline__ void sum_slots_body(const SumSlotsK& p, int block) {
 #pragma unroll
             for (int j = 0; j < V; ++j) acc[j] += Cvt<T>::to_f(w.e[j]);
         }
+        // the lists' lengths are looked at here, before the first store and not before the first rows are on their way (with
+        // a wait for them at the kernel's start a layer's two sums took 2 us each longer, 18432 tokens, d 384); the assembly
+        // keeps the compiler from looking in front of the loop
+        asm volatile("" : "+v"(len));
+        if (__any(len != p.T)) return sum_listed_slots<T>(p, block);
 #pragma unroll
         for (int j = 0; j < V; ++j) o.e[j] = Cvt<T>::from_f(acc[j]);
-        reinterpret_cast<uint4*>(out)[i] = o.u;
+        if (i0 + lane < nv) reinterpret_cast<uint4*>(out)[i] = o.u;
     }
 }
 
