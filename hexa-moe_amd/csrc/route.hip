@@ -519,8 +519,9 @@ __global__ __launch_bounds__(256) void route_from_lists_kernel(const int32_t* __
     int32_t* tbase = off + (E + 1);
     int* tmp = tbase + (E + 1);
     const int s = blockIdx.x;
-    const int32_t* L = expert_idx_list + (size_t)s * T;
-    for (int e = threadIdx.x; e < E; e += 256) {
+    // (as unsigned: positions that were never assigned hold -1 and are at the end, behind every expert)
+    const uint32_t* L = reinterpret_cast<const uint32_t*>(expert_idx_list) + (size_t)s * T;
+    for (uint32_t e = threadIdx.x; e < (uint32_t)E; e += 256) {
         int lo = 0, hi = T;  // first position with L[pos] >= e
         while (lo < hi) { int mid = (lo + hi) >> 1; if (L[mid] < e) lo = mid + 1; else hi = mid; }
         int lb = lo;

@@ -98,8 +98,8 @@ int hexa_token_assign(int32_t* token_idx_list, int32_t* expert_idx_list,
                       int num_experts, int32_t* scratch, void* stream);
 
 /* Build a route blob from reference-style lists (k slots of exactly T entries each, grouped by
- * expert, no padding): what a caller holding token_idx_list / expert_idx_list from the two ops above
- * (pad = 1) passes on to the operators.  Replaces the host-side rebuild of expert_start_list in
+ * expert, no padding; where the routing held ids outside [0, E), the entries that hexa_token_assign left at -1 come last):
+ * what a caller holding token_idx_list / expert_idx_list from the two ops above (pad = 1) passes on to the operators.  Replaces the host-side rebuild of expert_start_list in
  * launch_fused_grad_* (kernels/fused_ops_full.cu:486-512). */
 int hexa_route_from_lists(const int32_t* token_idx_list, const int32_t* expert_idx_list, int num_tokens,
                           int top_k, int num_experts, int32_t* route, void* stream);

@@ -70,3 +70,42 @@ def test_sum_over_slots_takes_the_listed_rows(dev, dtype, accumulate, T, k, E, d
     assert float((got - want).norm() / want.norm()) < BOUND[dtype]
     none = off.all(1)
     assert torch.equal(y.cpu()[none], start[none])
+
+
+@pytest.mark.parametrize("dtype", list(BOUND))
+@pytest.mark.parametrize("T,k,E", [(1, 2, 2), (70, 1, 3), (130, 2, 3), (1500, 3, 70)])
+def test_the_reference_operators_take_lists_with_unassigned_ends(dev, dtype, T, k, E):
+    """TOKEN_COUNT and TOKEN_ASSIGN into lists of num_tokens entries, then the matmul operators on them."""
+    import hexa_moe_cuda as ext
+    d_in, d_out, full = 32, 64, dtype == torch.float32
+    ids, off = _decision(T, E, k, T + E)
+    if T > 1:
+        off[1], ids[1] = False, 0
+    g = gen(T + 1)
+    x, W = torch.randn(k, T, d_in, generator=g).to(dtype), uniform((E, d_in, d_out), d_in ** -0.5, g).to(dtype)
+    bias, start = uniform((E, d_out), 0.5, g).to(dtype), torch.randn(T, d_out, generator=g).to(dtype)
+    tok = torch.full((k * T,), -1, dtype=torch.int32, device=dev)
+    exp = torch.full((k * T,), -1, dtype=torch.int32, device=dev)
+    cum = torch.arange(0, (k + 1) * T, T, dtype=torch.int32, device=dev)
+    for s in range(k):
+        r = ids[:, s].to(torch.int32).contiguous().to(dev)
+        count, offsets = torch.zeros(E, dtype=torch.int32, device=dev), torch.zeros(E + 1, dtype=torch.int32, device=dev)
+        ext.TOKEN_COUNT(count, offsets, r, T, E)
+        ext.TOKEN_ASSIGN(tok[s * T:(s + 1) * T], exp[s * T:(s + 1) * T], offsets, r, T, E)
+    y = start.to(dev)
+    _poison(dev, (k - 1) * T * d_out * x.element_size() or 4)
+    ext.ESMM_TENSOR_CORE(y, x.to(dev), W.to(dev), bias.to(dev), tok, exp, cum, full, full, full, True, T, k, d_in, d_out, E)
+    want = _expected(x, W, bias, ids, off, start)
+    assert float((y.double().cpu() - want).norm() / want.norm()) < BOUND[dtype]
+    # the gradients of a layer d_out -> d_in with weights W: j_y [k,T,d_in], x [T,d_out]
+    j_x, j_w, j_b = start.to(dev), torch.zeros(E, d_in, d_out, dtype=dtype, device=dev), torch.zeros(E, d_in, dtype=dtype, device=dev)
+    rows = torch.randn(T, d_out, generator=g).to(dtype)
+    ext.FUSED_GRAD(j_b, j_x, j_w, x.to(dev), W.to(dev), rows.to(dev), tok, exp, cum, full, full, True, T, k, d_out, d_in, E)
+    want = _expected(x, W, torch.zeros_like(bias), ids, off, start)
+    assert float((j_x.double().cpu() - want).norm() / want.norm()) < BOUND[dtype]
+    for e in range(E):
+        at = [((ids[:, s] == e) & ~off[:, s]).nonzero()[:, 0] for s in range(k)]
+        dw = sum(x[s, a].double().t() @ rows[a].double() for s, a in enumerate(at))
+        db = sum(x[s, a].double().sum(0) for s, a in enumerate(at))
+        assert float((j_w[e].double().cpu() - dw).norm()) <= BOUND[dtype] * float(dw.norm()) + 1e-30
+        assert float((j_b[e].double().cpu() - db).norm()) <= BOUND[dtype] * float(db.norm()) + 1e-30
