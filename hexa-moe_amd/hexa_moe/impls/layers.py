@@ -92,10 +92,42 @@ def _need_gpu(x):
                            "and its input to a HIP device")
 
 
-def _two_halves(native, config, routing, x, wg, fc1_w, fc2_w, fc1_bias, fc2_bias, chosen, dtype=None):
+class _OneOperation(torch.autograd.Function):
+    """`call(*tensors)`, a tensor or a tuple of them, as one operation of a torch.jit trace.  The kernels write through raw
+    pointers, so of a call's own tensor operations a trace would keep allocations that nothing fills."""
+
+    @staticmethod
+    def forward(ctx, call, *tensors):
+        state = torch._C._get_tracing_state()
+        torch._C._set_tracing_state(None)
+        try:
+            with torch.set_grad_enabled(any(ctx.needs_input_grad)):
+                ctx.inputs = [t if t is None else t.detach().requires_grad_(need) for t, need in zip(tensors, ctx.needs_input_grad[1:])]
+                ctx.outputs = call(*ctx.inputs)
+            results = [o.detach() for o in ((ctx.outputs,) if torch.is_tensor(ctx.outputs) else ctx.outputs)]
+        finally:
+            torch._C._set_tracing_state(state)
+        ctx.set_materialize_grads(False)
+        results = [o.detach() for o in results]     # (the tracer expects to have seen what becomes the operation's result)
+        return results[0] if torch.is_tensor(ctx.outputs) else tuple(results)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        outputs = (ctx.outputs,) if torch.is_tensor(ctx.outputs) else ctx.outputs
+        inputs = [t for t in ctx.inputs if t is not None and t.requires_grad]
+        outputs, grads = zip(*[(o, g) for o, g in zip(outputs, grads) if g is not None])
+        found = iter(torch.autograd.grad(outputs, inputs, grads, allow_unused=True))
+        return (None, *(next(found) if t is not None and t.requires_grad else None for t in ctx.inputs))
+
+
+def _traceable(call, *tensors):
+    return call(*tensors) if torch._C._get_tracing_state() is None else _OneOperation.apply(call, *tensors)
+
+
+def _two_halves(native, config, stage, routing, x, wg, fc1_w, fc2_w, fc1_bias, fc2_bias, chosen, dtype=None):
     """A depth whose activation is the caller's: it is evaluated once, between the two halves, as an ordinary part of
     the autograd graph.  Returns (y, l_aux, idx)."""
-    y1, l_aux, idx, handle = native.depth_in(config.route_pool.core, config.stage, x, wg, fc1_w, fc1_bias, chosen, fc2_w, routing, dtype)
+    y1, l_aux, idx, handle = native.depth_in(config.route_pool.core, stage, x, wg, fc1_w, fc1_bias, chosen, fc2_w, routing, dtype)
     y2 = config.activation_fn(y1)
     if y2.dtype != y1.dtype:
         y2 = y2.to(y1.dtype)
@@ -116,9 +148,14 @@ class FusedMoE_Shared_CudaCore:
         chosen = indices if torch.is_tensor(indices) else torch.stack([i.reshape(-1) for i in indices], dim=1)
         native = _native.load()
         routing = native.Routing(chosen.shape[1], int(config.num_global_experts))
-        if is_plain_gelu(config.activation_fn):
-            return native.depth(config.route_pool.core, config.stage, x, None, fc1_w, fc2_w, fc1_bias, fc2_bias, chosen, routing, [], [], None)[0]
-        return _two_halves(native, config, routing, x, None, fc1_w, fc2_w, fc1_bias, fc2_bias, chosen)[0]
+        stage = config.stage
+
+        def call(x, chosen, fc1_w, fc2_w, fc1_bias, fc2_bias):
+            if is_plain_gelu(config.activation_fn):
+                return native.depth(config.route_pool.core, stage, x, None, fc1_w, fc2_w, fc1_bias, fc2_bias, chosen, routing, [], [], None)[0]
+            return _two_halves(native, config, stage, routing, x, None, fc1_w, fc2_w, fc1_bias, fc2_bias, chosen)[0]
+
+        return _traceable(call, x, chosen, fc1_w, fc2_w, fc1_bias, fc2_bias)
 
 
 class FusedMoEDepth:
@@ -135,16 +172,21 @@ class FusedMoEDepth:
         top_k, noise_scale, is_gshard, sigma = opts
         native = _native.load()
         routing = native.Routing(top_k, config.num_global_experts, noise_scale, sigma, is_gshard)
-        if is_plain_gelu(config.activation_fn):
-            fwd = bwd = ()
-            if FusedMoEDepth.events:
-                fwd, bwd = ([0 if e is None else e.cuda_event for e in FusedMoEDepth.events[d] or ()] for d in ("fwd", "bwd"))
-            y, l_aux, idx = native.depth(config.route_pool.core, config.stage, tokens_input, wg, fc1_w, fc2_w, fc1_bias, fc2_bias, None,
-                                         routing, fwd, bwd, dtype)
-        else:
-            y, l_aux, idx = _two_halves(native, config, routing, tokens_input, wg, fc1_w, fc2_w, fc1_bias, fc2_bias, None, dtype)
-        config.routing_ = idx
-        return y, l_aux
+        stage = config.stage
+
+        def call(tokens_input, wg, fc1_w, fc2_w, fc1_bias, fc2_bias):
+            if is_plain_gelu(config.activation_fn):
+                fwd = bwd = ()
+                if FusedMoEDepth.events:
+                    fwd, bwd = ([0 if e is None else e.cuda_event for e in FusedMoEDepth.events[d] or ()] for d in ("fwd", "bwd"))
+                y, l_aux, idx = native.depth(config.route_pool.core, stage, tokens_input, wg, fc1_w, fc2_w, fc1_bias, fc2_bias, None,
+                                             routing, fwd, bwd, dtype)
+            else:
+                y, l_aux, idx = _two_halves(native, config, stage, routing, tokens_input, wg, fc1_w, fc2_w, fc1_bias, fc2_bias, None, dtype)
+            config.routing_ = idx
+            return y, l_aux
+
+        return _traceable(call, tokens_input, wg, fc1_w, fc2_w, fc1_bias, fc2_bias)
 
 
 def topk_and_loss(scores, top_k, loss_fn=losses.gshard_loss):
