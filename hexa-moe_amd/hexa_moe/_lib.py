@@ -36,7 +36,12 @@ class DepthDesc(ctypes.Structure):
     """hexa_moe_depth_desc of include/hexa_moe_hip.h."""
     _fields_ = [(n, ctypes.c_int32) for n in ("num_tokens", "top_k", "num_experts", "d_in", "hidden", "d_out", "act_dt",
                                               "w_dt", "b1_dt", "b2_dt", "gw1_dt", "gw2_dt", "gb1_dt", "gb2_dt", "loss")] + \
-               [("noise_scale", ctypes.c_float), ("sigma", ctypes.c_float), ("part", ctypes.c_int32), ("wide_y", ctypes.c_int32), ("careful", ctypes.c_int32)]
+               [("noise_scale", ctypes.c_float), ("sigma", ctypes.c_float), ("reserved", ctypes.c_int32)]
+
+
+class DepthOpts(ctypes.Structure):
+    """hexa_moe_depth_opts of include/hexa_moe_hip.h."""
+    _fields_ = [(n, ctypes.c_int32) for n in ("size", "part", "wide_y", "careful")]
 
 
 # name -> (restype, argtypes); kept in one table so the export test can walk it
@@ -69,6 +74,9 @@ SIGNATURES = {
     "hexa_moe_depth_ws_bytes": (_i, [ctypes.POINTER(DepthDesc), ctypes.POINTER(_i64), ctypes.POINTER(_i64)]),
     "hexa_moe_depth_forward": (_i, [ctypes.POINTER(DepthDesc)] + [_vp] * 17 + [_vp, _i64, _vp, _i, _vp]),
     "hexa_moe_depth_backward": (_i, [ctypes.POINTER(DepthDesc)] + [_vp] * 21 + [_vp, _i64, _vp, _i, _vp]),
+    "hexa_moe_depth_part_ws_bytes": (_i, [ctypes.POINTER(DepthDesc), ctypes.POINTER(DepthOpts), ctypes.POINTER(_i64), ctypes.POINTER(_i64)]),
+    "hexa_moe_depth_part_forward": (_i, [ctypes.POINTER(DepthDesc), ctypes.POINTER(DepthOpts)] + [_vp] * 17 + [_vp, _i64, _vp, _i, _vp]),
+    "hexa_moe_depth_part_backward": (_i, [ctypes.POINTER(DepthDesc), ctypes.POINTER(DepthOpts)] + [_vp] * 21 + [_vp, _i64, _vp, _i, _vp]),
     "hexa_moe_depth_route_rounding": (_i, [ctypes.POINTER(DepthDesc)] + [_vp] * 16 + [_i64, _vp]),
     "hexa_round_weights": (_i, [_vp, _vp, _i64, _vp, _vp, _i64, _vp, _i, _i, _i, _i, _vp]),
     "hexa_last_error": (ctypes.c_char_p, []),

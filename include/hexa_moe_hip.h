@@ -19,6 +19,8 @@
 extern "C" {
 #endif
 
+/* Changes with what an existing entry point, struct or constant means; new entry points alone leave it as it is (version 9
+ * has gained hexa_round_weights, hexa_moe_depth_route_rounding and hexa_moe_depth_part_*). */
 #define HEXA_ABI_VERSION 9
 
 /* element types */
@@ -293,10 +295,16 @@ typedef struct hexa_moe_depth_desc {
     int32_t loss;
     float noise_scale; /* factor of `noise` in the logits (gate_noise / E while training, else 0) */
     float sigma;       /* load-importance only */
+    int32_t reserved;
+} hexa_moe_depth_desc;
+
+/* Options of hexa_moe_depth_part_*; those of hexa_moe_depth_forward and _backward are all 0. */
+typedef struct hexa_moe_depth_opts {
+    int32_t size;      /* sizeof(hexa_moe_depth_opts) as the caller knows it; what it does not know is 0 */
     int32_t part;      /* HEXA_PART_* (0: all) */
     int32_t wide_y;    /* 1: the forward stores y as fp32 (16-bit act_dt and top_k 1 only) */
     int32_t careful;   /* 1: GELU and GELU' of the fp32 product, not of the one rounded to act_dt */
-} hexa_moe_depth_desc;
+} hexa_moe_depth_opts;
 
 /* Which parts of the depth a call runs (0: all of them).  With an activation that the kernels do not fuse, the caller
  * evaluates it between a call of HEXA_PART_ROUTE | HEXA_PART_FC1 and one of HEXA_PART_FC2; with weights that it rounds
@@ -336,7 +344,7 @@ int hexa_moe_depth_forward(const hexa_moe_depth_desc* d, const void* x, const fl
                            void* y2, void* y, void* ws, int64_t ws_bytes, void* const* events, int num_events,
                            void* stream);
 
-/* HEXA_PART_ROUTE of hexa_moe_depth_forward for a caller with fp32 master weights: also rounds src1 [E][hidden][d_in] and
+/* HEXA_PART_ROUTE of hexa_moe_depth_part_forward for a caller with fp32 master weights: also rounds src1 [E][hidden][d_in] and
  * src2 [E][hidden][d_out] (either may be NULL, with its dst) to act_dt, as hexa_round_weights does but beside the front
  * end's own launches; with eight and more choices per expert, experts without tokens are rounded too.
  * x_src (may be NULL): fp32 tokens; x is then a buffer that receives them rounded to act_dt. */
@@ -358,6 +366,20 @@ int hexa_moe_depth_backward(const hexa_moe_depth_desc* d, const void* dy, const 
                             int32_t* plan, const void* y1, const void* y2, void* dx, float* dwg, void* dw1,
                             void* db1, void* dw2, void* db2, void* dy1, void* ws, int64_t ws_bytes, void* const* events,
                             int num_events, void* stream);
+
+/* The three calls above with options (NULL: none).  Pointers that belong to parts which are not asked for may be NULL. */
+int hexa_moe_depth_part_ws_bytes(const hexa_moe_depth_desc* d, const hexa_moe_depth_opts* opts, int64_t* forward_bytes, int64_t* backward_bytes);
+int hexa_moe_depth_part_forward(const hexa_moe_depth_desc* d, const hexa_moe_depth_opts* opts, const void* x, const float* wg, const float* noise,
+                                const void* fc1_w, const void* fc1_b, const void* fc2_w, const void* fc2_b, float* logits,
+                                float* scores, int32_t* idx, float* thr, float* stats, int32_t* route, int32_t* plan, void* y1,
+                                void* y2, void* y, void* ws, int64_t ws_bytes, void* const* events, int num_events,
+                                void* stream);
+int hexa_moe_depth_part_backward(const hexa_moe_depth_desc* d, const hexa_moe_depth_opts* opts, const void* dy, const float* grad_l_aux, const void* x,
+                                 const float* wg, const void* fc1_w, const void* fc2_w, const float* scores,
+                                 const int32_t* idx, const float* thr, const float* stats, const int32_t* route,
+                                 int32_t* plan, const void* y1, const void* y2, void* dx, float* dwg, void* dw1,
+                                 void* db1, void* dw2, void* db2, void* dy1, void* ws, int64_t ws_bytes, void* const* events,
+                                 int num_events, void* stream);
 
 /* fp32 master weights of one or two layers (n1 / n2 elements per expert, multiples of 8; n2 = 0: one) rounded to the
  * 16-bit type dt, for the experts to which `route` sends tokens; the other experts' copies are not written.

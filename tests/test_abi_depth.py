@@ -1,0 +1,50 @@
+"""The C ABI's depth descriptor is what version 9 says it is, whatever lies behind it; options travel apart from it."""
+import ctypes
+
+import pytest
+
+SIZES = (256, 2, 8, 64, 128, 64)
+TYPES = (2, 2, 0, 0, 0, 0, 0, 0)
+
+
+def _desc(reserved=0):
+    from hexa_moe import _lib
+    return _lib.DepthDesc(*SIZES, *TYPES, 0, 0.0, 0.0, reserved)
+
+
+def _bytes(fn, *args):
+    from hexa_moe import _lib
+    f, b = ctypes.c_int64(), ctypes.c_int64()
+    rc = getattr(_lib.load(), fn)(*args, ctypes.byref(f), ctypes.byref(b))
+    return rc, f.value, b.value
+
+
+def test_descriptor_of_version_9():
+    from hexa_moe import _lib
+    assert ctypes.sizeof(_lib.DepthDesc) == 72
+    want = _bytes("hexa_moe_depth_ws_bytes", ctypes.byref(_desc()))
+    assert want[0] == 0 and want[1] > 0 and want[2] > 0
+    # a caller's struct ends with `reserved`, which nobody had to clear, and is followed by whatever it is followed by
+    for fill in (0x01, 0x7f, 0xff):
+        memory = (ctypes.c_ubyte * 256)(*[fill] * 256)
+        ctypes.memmove(memory, bytes(_desc(reserved=int.from_bytes(bytes([fill] * 4), "little", signed=True))), 72)
+        assert _bytes("hexa_moe_depth_ws_bytes", ctypes.cast(memory, ctypes.POINTER(_lib.DepthDesc))) == want
+
+
+def test_options():
+    from hexa_moe import _lib
+    d, size = _desc(), ctypes.sizeof(_lib.DepthOpts)
+    whole = _bytes("hexa_moe_depth_ws_bytes", ctypes.byref(d))
+    ask = lambda *o: _bytes("hexa_moe_depth_part_ws_bytes", ctypes.byref(d), ctypes.byref(_lib.DepthOpts(*o)))      # noqa: E731
+    assert _bytes("hexa_moe_depth_part_ws_bytes", ctypes.byref(d), None) == whole
+    assert ask(size) == whole
+    assert ask(8, 7, 1, 1) == whole         # a caller that knows `part` only: what follows it is not looked at
+    assert ask(size, 7, 1, 0)[0] == -2      # wide_y is for top-1
+    assert ask(size, 8)[0] == -1            # no such part
+    for n in (0, 3, size + 4):
+        assert ask(n)[0] == -1
+
+
+@pytest.mark.parametrize("fn", ["hexa_moe_depth_part_ws_bytes", "hexa_moe_depth_ws_bytes"])
+def test_null_descriptor(fn):
+    assert _bytes(fn, *([None] * (2 if "part" in fn else 1)))[0] == -1
