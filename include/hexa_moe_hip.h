@@ -304,6 +304,7 @@ typedef struct hexa_moe_depth_opts {
     int32_t part;      /* HEXA_PART_* (0: all) */
     int32_t wide_y;    /* 1: the forward stores y as fp32 (16-bit act_dt and top_k 1 only) */
     int32_t careful;   /* 1: GELU and GELU' of the fp32 product, not of the one rounded to act_dt */
+    int32_t no_gate;   /* 1: wg is NULL in every call, and the workspaces leave the router's and the gate's share out */
 } hexa_moe_depth_opts;
 
 /* Which parts of the depth a call runs (0: all of them).  With an activation that the kernels do not fuse, the caller
@@ -319,7 +320,7 @@ typedef struct hexa_moe_depth_opts {
 #define HEXA_PART_FC2 4
 #define HEXA_PART_ALL 7
 
-/* Bytes of caller scratch the two calls need (either pointer may be NULL). */
+/* Bytes of caller scratch the two calls need (either pointer may be NULL); with options, those of the parts asked for. */
 int hexa_moe_depth_ws_bytes(const hexa_moe_depth_desc* d, int64_t* forward_bytes, int64_t* backward_bytes);
 
 /* Forward.  With wg (fp32 [E][d_in]) the call starts at the gate: logits = x.wg^T (fp32), scores / idx / l_aux as

@@ -40,6 +40,7 @@ def test_options():
     assert ask(size) == whole
     assert ask(8, 7, 1, 1) == whole         # a caller that knows `part` only: what follows it is not looked at
     assert ask(size, 7, 1, 0)[0] == -2      # wide_y is for top-1
+    assert ask(size, -1)[0] == -1
     assert ask(size, 8)[0] == -1            # no such part
     for n in (0, 3, size + 4):
         assert ask(n)[0] == -1
@@ -48,3 +49,26 @@ def test_options():
 @pytest.mark.parametrize("fn", ["hexa_moe_depth_part_ws_bytes", "hexa_moe_depth_ws_bytes"])
 def test_null_descriptor(fn):
     assert _bytes(fn, *([None] * (2 if "part" in fn else 1)))[0] == -1
+
+
+@pytest.mark.parametrize("no_gate", [0, 1])
+@pytest.mark.parametrize("act_dt", [0, 2])
+def test_a_part_takes_its_own_scratch(no_gate, act_dt):
+    """The backward's pieces: the first layer's half has the gate's and the column sums', each half its weight gradient's."""
+    from hexa_moe import _lib
+    T, k, E, d, h, size = 32768, 2, 64, 1024, 4096, 2 if act_dt else 4
+    desc = _lib.DepthDesc(T, k, E, d, h, d, act_dt, act_dt, *[0] * 6, 0, 0.0, 0.0, 0)
+    ask = lambda part: _bytes("hexa_moe_depth_part_ws_bytes", ctypes.byref(desc),      # noqa: E731
+                              ctypes.byref(_lib.DepthOpts(ctypes.sizeof(_lib.DepthOpts), part, 0, 0, no_gate)))
+    fwd, bwd = zip(*[ask(p)[1:] for p in (1, 2, 4, 7)])
+    slots = (k - 1) * T * d * size
+    assert fwd[1] <= 256 and fwd[2] == slots and fwd[3] == fwd[2] + (fwd[0] if not no_gate else 0)
+    if no_gate:
+        assert fwd[0] <= 256
+    plan = -(-(4 * E + 32) * 4 // 256) * 256
+    assert bwd[1] + bwd[2] - plan == bwd[3]
+    ess, partial = 8 * E * d * 4, 128 << 20      # of the weight gradient's scratch at most
+    assert bwd[2] <= plan + ess + partial
+    colsum = k * (T // 128 + E) * h * 4
+    gate = T * E * 4 + T * d * size + (T // 64 + 1) * E * d * 4
+    assert bwd[1] <= plan + colsum + partial + slots + (0 if no_gate else gate)

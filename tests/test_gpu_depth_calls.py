@@ -1,5 +1,7 @@
-"""A MoE depth through the tensor-level wrappers of the C ABI's depth calls (ops.DepthPlan, moe_depth_forward / _backward)
-against the module."""
+"""A MoE depth through the tensor-level wrappers of the C ABI's depth calls (ops.DepthPlan, moe_depth_forward / _backward),
+and in parts, against the module."""
+import ctypes
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -66,3 +68,48 @@ def test_wrappers_give_what_the_module_gives(dev, dtype, k):
                            torch.empty(d.plan.bwd_bytes, dtype=torch.uint8, device=dev))
     d.same(("y", "dx", "dwg", "dw1", "db1", "dw2", "db2"))
     assert float(d.stats[-1]) == float(d.want["l_aux"])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("k", [1, 2])
+@pytest.mark.parametrize("gated", [True, False])
+def test_parts_stay_inside_the_scratch_they_ask_for(dev, dtype, k, gated):
+    """Every part with exactly the bytes it asks for, in front of memory that has to stay as it is."""
+    from hexa_moe import _lib, ops
+    lib, d, p = _lib.load(), _Depth(dev, dtype, k), ops._ptr
+    d.forward()
+    want = {n: t.clone() for n, t in (("y", d.y), ("y1", d.y1), ("y2", d.y2))}
+    GUARD = 1 << 16
+
+    def run(part, backward, *args):
+        o = _lib.DepthOpts(ctypes.sizeof(_lib.DepthOpts), part, 0, 0, int(not gated))
+        sizes = [ctypes.c_int64(), ctypes.c_int64()]
+        _lib.check(lib.hexa_moe_depth_part_ws_bytes(ctypes.byref(d.plan.desc), ctypes.byref(o), *[ctypes.byref(s) for s in sizes]), "ws_bytes")
+        n = sizes[backward].value
+        ws = torch.full((n + GUARD,), 0xA5, dtype=torch.uint8, device=dev)
+        fn = lib.hexa_moe_depth_part_backward if backward else lib.hexa_moe_depth_part_forward
+        _lib.check(fn(ctypes.byref(d.plan.desc), ctypes.byref(o), *args, p(ws), n, None, 0, ops._stream()), "part")
+        assert bool((ws[n:] == 0xA5).all()), f"part {part} wrote behind its scratch"
+
+    w, g = d.w, d.grads
+    wg = w["wg"] if gated else None
+    for t in (d.y, d.y1, d.y2, d.scores, d.stats):
+        t.fill_(float("nan"))
+    run(1, 0, p(d.x), p(wg), None, None, None, None, None, p(d.logits), p(d.scores), p(d.idx), None, p(d.stats), p(d.blob), p(d.estmm_plan), None, None, None)
+    run(2, 0, p(d.x), None, None, p(w["w1"]), p(w["b1"]), None, None, None, None, None, None, None, p(d.blob), None, p(d.y1), None, None)
+    assert torch.equal(d.y1, want["y1"])
+    d.y2.copy_(want["y2"])
+    run(4, 0, None, None, None, None, None, p(w["w2"]), p(w["b2"]), None, None, None, None, None, p(d.blob), None, None, p(d.y2), p(d.y))
+    assert torch.equal(d.y, want["y"])
+    run(4, 1, p(d.dy), None, None, None, None, p(w["w2"]), None, None, None, None, p(d.blob), p(d.estmm_plan), None, p(d.y2), None, None, None, None,
+        p(g["dw2"]), p(g["db2"]), p(d.dy1))
+    d.same(("dw2", "db2"))
+    # the activation's derivative between the halves, as the caller would have it
+    y1 = d.y1.clone().requires_grad_(True)
+    F.gelu(y1).backward(d.dy1)
+    d.dy1.copy_(y1.grad)
+    run(2, 1, None, p(d.g_aux) if gated else None, p(d.x), p(wg), p(w["w1"]), None, p(d.scores), p(d.idx), None, p(d.stats), p(d.blob), p(d.estmm_plan),
+        None, None, p(g["dx"]), p(g["dwg"]) if gated else None, p(g["dw1"]), p(g["db1"]), None, None, p(d.dy1))
+    bound = 1e-5 if dtype == torch.float32 else 1e-2       # GELU' of a dy2 rounded in between
+    for n in ("dw1", "db1") + (("dx", "dwg") if gated else ()):
+        assert float((g[n].double() - d.want[n].double()).norm()) <= bound * float(d.want[n].double().norm()), n
