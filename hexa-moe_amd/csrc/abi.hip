@@ -267,10 +267,9 @@ extern "C" int hexa_esmm_ess_ws_floats(int T, int k, int out_dim, int E, int64_t
     return HEXA_OK;
 }
 
-extern "C" int hexa_esmm_gelu_bwd_ess(void* out, void* db, const void* x, const void* w, const void* y1,
-                                      const int32_t* route, int w_layout, int db_accumulate, int T, int k, int in_dim,
-                                      int out_dim, int E, int x_dt, int w_dt, int db_dt, float* ws, int64_t ws_floats,
-                                      void* stream) {
+int hexa::esmm_gelu_bwd_ess_call(void* out, void* db, const void* x, const void* w, const void* y1, const int32_t* route, int w_layout,
+                                 int db_accumulate, int T, int k, int in_dim, int out_dim, int E, int x_dt, int w_dt, int db_dt,
+                                 float* ws, int64_t ws_floats, void* stream, bool careful) {
     if (int rc = check_sizes("hexa_esmm_gelu_bwd_ess", T, k, E, in_dim, out_dim)) return rc;
     if (!out || !db || !x || !w || !y1 || !route) HEXA_FAIL(HEXA_ERR_ARG, "hexa_esmm_gelu_bwd_ess: null pointer");
     if (!is_dt(x_dt) || !is_dt(w_dt) || !is_dt(db_dt)) HEXA_FAIL(HEXA_ERR_ARG, "hexa_esmm_gelu_bwd_ess: unknown element type");
@@ -284,6 +283,7 @@ extern "C" int hexa_esmm_gelu_bwd_ess(void* out, void* db, const void* x, const 
         a.x_per_slot = 0; a.out_per_slot = 1;
         a.w_layout = w_layout; a.accumulate = 0;
         a.x_dt = x_dt; a.w_dt = w_dt; a.bias_dt = HEXA_F32; a.out_dt = x_dt; a.act = HEXA_ACT_GELU_BWD;
+        a.careful = careful;
         if (w_layout != HEXA_W_IN_OUT && w_layout != HEXA_W_OUT_IN)
             HEXA_FAIL(HEXA_ERR_ARG, "hexa_esmm_gelu_bwd_ess: bad w_layout %d", w_layout);
         if (esmm16_dma_colsum_supported(a)) {
@@ -292,10 +292,18 @@ extern "C" int hexa_esmm_gelu_bwd_ess(void* out, void* db, const void* x, const 
         }
     }
     // any other case: the two operators one after the other (same results up to the order of the sums)
-    int rc = hexa_esmm(out, x, w, nullptr, route, 0, w_layout, 0, T, k, in_dim, out_dim, E, x_dt, w_dt, HEXA_F32, x_dt,
-                       HEXA_ACT_GELU_BWD, const_cast<void*>(y1), nullptr, stream);
+    int rc = esmm_call(out, x, w, nullptr, route, 0, w_layout, 0, T, k, in_dim, out_dim, E, x_dt, w_dt, HEXA_F32, x_dt,
+                       HEXA_ACT_GELU_BWD, const_cast<void*>(y1), nullptr, nullptr, nullptr, stream, careful);
     if (rc) return rc;
     return hexa_ess(db, out, route, 1, db_accumulate, T, k, out_dim, E, x_dt, db_dt, ws, ws ? ws_floats : 0, stream);
+}
+
+extern "C" int hexa_esmm_gelu_bwd_ess(void* out, void* db, const void* x, const void* w, const void* y1,
+                                      const int32_t* route, int w_layout, int db_accumulate, int T, int k, int in_dim,
+                                      int out_dim, int E, int x_dt, int w_dt, int db_dt, float* ws, int64_t ws_floats,
+                                      void* stream) {
+    return esmm_gelu_bwd_ess_call(out, db, x, w, y1, route, w_layout, db_accumulate, T, k, in_dim, out_dim, E, x_dt, w_dt, db_dt, ws,
+                                  ws_floats, stream, false);
 }
 
 extern "C" int hexa_gelu_bwd(void* dy1, const void* dy2, const void* y1, int64_t n, int dt, void* stream) {
