@@ -59,15 +59,17 @@ struct EsmmArgs {
     // optional: also db[e][:] (+)= column sums of the expert's stored result rows (ESS of the result), through
     // per-tile partial sums in `colsum` (16-bit per-slot results on the fast path only)
     float* colsum = nullptr; void* db = nullptr; int db_dt = 0, db_accumulate = 0;
-    // GELU / GELU' of the fp32 product and not of the rounded one.  16-bit contractions that are no multiple of 32 always do
-    // (also in the sum over slots, see esmm16_slot_by_slot), and fp32 masters with few rows per expert ask for it: both once
-    // ran on the general kernels, which do the same (relative error of y against fp64, 2657 tokens, d 184, top-2, bf16:
-    // 2.95e-3; with the rounded product 3.64e-3).
+    // GELU / GELU' of the fp32 product and not of the rounded one, and the sum with an earlier result too.  16-bit contractions
+    // that are no multiple of 32 always do (also in the sum over slots, see esmm16_slot_by_slot), and fp32 masters with few
+    // rows per expert ask for it: both once ran on the general kernels, which do the same (relative error of y against fp64,
+    // 2657 tokens, d 184, top-2, bf16: 2.95e-3; with the rounded product 3.64e-3).
     bool careful = false;
     bool wide = false;   // the result, rounded to out_dt, is stored as fp32 (pipelined kernel only, see esmm16_wide_supported)
     // optional, with slot_ws on the fast path: one more tensor of the result's shape added by the slot sum
     const void* sum_extra = nullptr;
 };
+// the fp32 product goes into an activation or onto an earlier result
+inline bool esmm16_unrounded(const EsmmArgs& a) { return (a.careful || a.in_dim % 32 != 0) && (a.act != HEXA_ACT_NONE || a.accumulate); }
 // sums over slots where each slot's fp32 product joins the result, in launches of their own
 inline bool esmm16_slot_by_slot(const EsmmArgs& a) { return a.in_dim % 32 != 0 && !a.out_per_slot && a.r.k > 1; }
 struct EstmmArgs {

@@ -116,3 +116,27 @@ def _check(layer, fused, gate):
 def test_masters_used_for_few_rows(dev, fused, d, h):
     layer = _Layer(dev, torch.bfloat16, 60, d, h, 8, 1, True, "gelu")
     _check(layer, fused, False)
+
+
+@pytest.mark.parametrize("fused", [0, 2])
+@pytest.mark.parametrize("masters,d,h,act", [(False, 72, 264, "gelu"), (False, 64, 136, "gelu"), (False, 64, 264, "own"), (True, 64, 128, "gelu")])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gate_share_of_one_slot(dev, dtype, masters, d, h, act, fused):
+    """dx = the gate's share as it is stored + the fp32 product, rounded once (hidden sizes that are no multiple of 32, and
+    masters used for few rows)."""
+    _check(_Layer(dev, dtype, 60, d, h, 8, 1, masters, act), fused, True)
+
+
+def test_accumulated_product_of_a_ragged_contraction(dev):
+    """out += x . w where the contraction is no multiple of 32: the fp32 product joins what is there (328 is long enough for the
+    pipelined kernel, which would round it first)."""
+    from hexa_moe import _lib, ops
+    T, d_in, d_out, E = 500, 328, 136, 4
+    g = torch.Generator().manual_seed(1)
+    x, w = torch.randn(1, T, d_in, generator=g).to(torch.bfloat16), (torch.randn(E, d_in, d_out, generator=g) / d_in ** 0.5).to(torch.bfloat16)
+    old = torch.randn(T, d_out, generator=g).to(torch.bfloat16)
+    routing = torch.randint(0, E, (T, 1), generator=g)
+    out = ops.esmm(x.to(dev), w.to(dev), None, ops.route_build(routing.to(dev), E), True, _lib.HEXA_W_IN_OUT, out=old.clone().to(dev), accumulate=True)
+    product = torch.bmm(x[0].double()[:, None], w.double()[routing[:, 0]])[:, 0]
+    differ = (out.cpu() != (old.double() + product).to(torch.bfloat16)).double().mean().item()
+    assert differ < 0.01, differ
