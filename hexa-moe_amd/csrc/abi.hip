@@ -76,7 +76,7 @@ extern "C" int hexa_abi_version(void) { return HEXA_ABI_VERSION; }
 // add one more tensor (`sum_extra`): the same predicate esmm_call applies, for callers that must decide beforehand
 // where that addend is written.
 bool hexa::esmm_slot_sum_takes_extra(const int32_t* route, int w_layout, int T, int k, int in_dim, int out_dim, int E,
-                                     int x_dt, int w_dt, int out_dt, const void* slot_ws) {
+                                     int x_dt, int w_dt, int out_dt, const void* slot_ws, bool careful) {
     if (T <= 0 || k <= 1 || !slot_ws || x_dt == HEXA_F32 || !dma_path_enabled()) return false;
     EsmmArgs a;
     a.out = nullptr; a.x = nullptr; a.w = nullptr; a.bias = nullptr; a.out_act = nullptr; a.slot_ws = const_cast<void*>(slot_ws);
@@ -85,6 +85,7 @@ bool hexa::esmm_slot_sum_takes_extra(const int32_t* route, int w_layout, int T, 
     a.x_per_slot = 1; a.out_per_slot = 0;
     a.w_layout = w_layout; a.accumulate = 0;
     a.x_dt = x_dt; a.w_dt = w_dt; a.bias_dt = HEXA_F32; a.out_dt = out_dt; a.act = HEXA_ACT_NONE;
+    a.careful = careful;
     return esmm16_dma_supported(a) && !esmm16_slot_by_slot(a);
 }
 

@@ -127,6 +127,55 @@ int launch_add(void* out, const void* extra, int64_t n, int dt, hipStream_t st) 
     return launch_sum_slots_d(SumSlotsK{out, nullptr, n, 0, extra, 0, nullptr, nullptr, 0, 0, 0, 1}, dt, st);
 }
 
+// out = the fp32 results of every slot, and `extra` (may be null), added in that order and rounded once.  A wavefront per row; rows
+// that a short list does not hold are looked up in it, as in sum_listed_slots.  For lists of a few hundred rows: bound by its launch.
+namespace {
+template <typename T>
+__global__ __launch_bounds__(256) void sum_wide_slots_kernel(T* __restrict__ out, const float* __restrict__ ws, const T* __restrict__ extra,
+                                                             const int32_t* __restrict__ offsets, const int32_t* __restrict__ token_ids, int rows,
+                                                             int k, int E, int N) {
+    const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (row >= rows) return;
+    unsigned listed = 0;
+    for (int s = 0; s < k; ++s) {
+        const int count = offsets[(size_t)s * (E + 1) + E];
+        bool found = count >= rows;
+        for (int r0 = 0; !found && r0 < count; r0 += 64)
+            found = __ballot(r0 + lane < count && token_ids[(size_t)s * rows + r0 + lane] == row) != 0;
+        listed |= found ? 1u << s : 0u;
+    }
+    for (int c = lane * 8; c < N; c += 64 * 8) {
+        float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < k; ++s) {
+            if (!(listed >> s & 1)) continue;
+            const float4* from = reinterpret_cast<const float4*>(ws + ((size_t)s * rows + row) * N + c);
+            const float4 a = from[0], b = from[1];
+            acc[0] += a.x; acc[1] += a.y; acc[2] += a.z; acc[3] += a.w;
+            acc[4] += b.x; acc[5] += b.y; acc[6] += b.z; acc[7] += b.w;
+        }
+        union { uint4 u; T e[8]; } o;
+        if (extra) {
+            o.u = *reinterpret_cast<const uint4*>(extra + (size_t)row * N + c);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[j] += Cvt<T>::to_f(o.e[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o.e[j] = Cvt<T>::from_f(acc[j]);
+        *reinterpret_cast<uint4*>(out + (size_t)row * N + c) = o.u;
+    }
+}
+}  // namespace
+int launch_sum_wide_slots(void* out, const float* ws, const void* extra, const RouteView& r, int N, int dt, hipStream_t st) {
+    if (N % 8 || r.k > WIDE_SLOTS_MAX || (dt != HEXA_BF16 && dt != HEXA_F16)) HEXA_FAIL(HEXA_ERR_UNSUPPORTED, "sum_wide_slots: rows of 8 16-bit values, up to 32 slots");
+    const dim3 grid(div_up(r.T, 4));
+    if (dt == HEXA_BF16)
+        hipLaunchKernelGGL((sum_wide_slots_kernel<__bf16>), grid, dim3(256), 0, st, (__bf16*)out, ws, (const __bf16*)extra, r.offsets, r.token_ids, r.T, r.k, r.E, N);
+    else
+        hipLaunchKernelGGL((sum_wide_slots_kernel<_Float16>), grid, dim3(256), 0, st, (_Float16*)out, ws, (const _Float16*)extra, r.offsets, r.token_ids, r.T, r.k, r.E, N);
+    HEXA_CHECK_LAUNCH("sum_wide_slots");
+    return HEXA_OK;
+}
+
 // out (+)= the sum of `parts` partial results of n values each, in their order
 int launch_fold(void* out, const float* ws, long n, int parts, int dt, int accumulate, hipStream_t st) {
     SmallTask f;

@@ -60,9 +60,9 @@ struct EsmmArgs {
     // per-tile partial sums in `colsum` (16-bit per-slot results on the fast path only)
     float* colsum = nullptr; void* db = nullptr; int db_dt = 0, db_accumulate = 0;
     // GELU / GELU' of the fp32 product and not of the rounded one, and the sum with an earlier result too.  16-bit contractions
-    // that are no multiple of 32 always do (also in the sum over slots, see esmm16_slot_by_slot), and fp32 masters with few
-    // rows per expert ask for it: both once ran on the general kernels, which do the same (relative error of y against fp64,
-    // 2657 tokens, d 184, top-2, bf16: 2.95e-3; with the rounded product 3.64e-3).
+    // that are no multiple of 32 always do, and fp32 masters with few rows per expert ask for it, both also in the sum over
+    // slots (see esmm16_slot_by_slot): they once ran on the general kernels, which do the same (relative error of y against
+    // fp64, 2657 tokens, d 184, top-2, bf16: 2.95e-3; with the rounded product 3.64e-3).
     bool careful = false;
     bool wide = false;   // the result, rounded to out_dt, is stored as fp32 (pipelined kernel only, see esmm16_wide_supported)
     // optional, with slot_ws on the fast path: one more tensor of the result's shape added by the slot sum
@@ -71,7 +71,7 @@ struct EsmmArgs {
 // the fp32 product goes into an activation or onto an earlier result
 inline bool esmm16_unrounded(const EsmmArgs& a) { return (a.careful || a.in_dim % 32 != 0) && (a.act != HEXA_ACT_NONE || a.accumulate); }
 // sums over slots where each slot's fp32 product joins the result, in launches of their own
-inline bool esmm16_slot_by_slot(const EsmmArgs& a) { return a.in_dim % 32 != 0 && !a.out_per_slot && a.r.k > 1; }
+inline bool esmm16_slot_by_slot(const EsmmArgs& a) { return (a.careful || a.in_dim % 32 != 0) && !a.out_per_slot && a.r.k > 1; }
 struct EstmmArgs {
     void* dw; const void* p; const void* q;   // dw[e][m][n] = sum_rows p[row][m] * q[row][n]
     RouteView r;
@@ -95,7 +95,7 @@ int esmm_gelu_bwd_ess_call(void* out, void* db, const void* x, const void* w, co
                            int db_accumulate, int T, int k, int in_dim, int out_dim, int E, int x_dt, int w_dt, int db_dt, float* ws,
                            int64_t ws_floats, void* stream, bool careful);
 bool esmm_slot_sum_takes_extra(const int32_t* route, int w_layout, int T, int k, int in_dim, int out_dim, int E, int x_dt,
-                               int w_dt, int out_dt, const void* slot_ws);
+                               int w_dt, int out_dt, const void* slot_ws, bool careful);
 int launch_esmm16(const EsmmArgs& a, hipStream_t s);
 int launch_esmm32(const EsmmArgs& a, hipStream_t s);
 // Tuning / testing knobs: 0 = automatic.  Each one starts from an environment variable (read once) and
@@ -158,6 +158,9 @@ int launch_ess(const EssArgs& a, hipStream_t s);
 int launch_ess_noalloc(EssArgs a, hipStream_t s);
 // out [T][N] += the other slots' results in ws ([k-1][T][N]) + extra; accumulate: out held something before slot 0's product
 int launch_sum_slots(void* out, const void* ws, const RouteView& r, int N, bool accumulate, int dt, hipStream_t s, const void* extra = nullptr);
+// out [T][N] (16-bit) = the slots' fp32 results in ws ([k][T][N]) + extra (of out's type, may be null), rounded once
+constexpr int WIDE_SLOTS_MAX = 32;
+int launch_sum_wide_slots(void* out, const float* ws, const void* extra, const RouteView& r, int N, int dt, hipStream_t s);
 int launch_add(void* out, const void* extra, int64_t n, int dt, hipStream_t s);   // out += extra
 // routing front end of the depth call: the router also counts, the counting sort's scan launch also finishes the loss,
 // its scatter launch also makes the ESTMM plan (see router.hip, route.hip)

@@ -72,8 +72,9 @@ class _Layer:
         torch.autograd.backward([y, l_aux], [dy.to(self.dev), torch.full_like(l_aux, aux)])
         return y.detach().cpu(), x.grad.cpu()
 
-    def want(self, gate_dx=None):
-        """(y, dx); gate_dx: the gate's share of dx, which the products join one after the other."""
+    def want(self, gate_dx, slot_by_slot):
+        """(y, dx), the slots' products and the gate's share of dx (gate_dx) added before they are rounded; with slot_by_slot
+        rounded as each joins."""
         rounded = lambda t: t.to(self.dtype).double()      # noqa: E731
         route = self.m.dispatch_params.routing_.long().cpu()
         w1, w2 = (rounded(p[0].detach().cpu()) for p in (self.m.batched_fc1_w, self.m.batched_fc2_w))
@@ -90,11 +91,13 @@ class _Layer:
             grad = phi(y1) + y1 * torch.exp(-0.5 * y1 * y1) / math.sqrt(2.0 * math.pi)
             dy1 = rounded((q if self.fused else rounded(q)) * grad)
             p2, r = torch.bmm(y2[:, None], w2[e])[:, 0], torch.bmm(dy1[:, None], w1[e])[:, 0]
-            y, dx = rounded(p2 if y is None else y + p2), rounded(r if dx is None else dx + r)
+            y, dx = p2 if y is None else y + p2, r if dx is None else dx + r
+            if slot_by_slot:
+                y, dx = rounded(y), rounded(dx)
         return y.to(self.dtype), dx.to(self.dtype)
 
 
-def _check(layer, fused, gate):
+def _check(layer, fused, gate, slot_by_slot=False):
     """As good as every value is the one expected.  fp32 sums differ from 64 bits by some 2^-22, which moves a value over a
     rounding boundary of bf16 once in thousands, and one element of y1 or dy1 that was moved so moves a few of its row's: below
     1 % in all.  One more rounding on the way changes a fifth of the values and more."""
@@ -106,7 +109,7 @@ def _check(layer, fused, gate):
         y, dx = layer.run(layer.dy, 50.0 if gate else 0.0)
     finally:
         _lib.check(lib.hexa_set_option(b"backward_fused", 0), "hexa_set_option")
-    for name, got, want in zip(("y", "dx"), (y, dx), layer.want(gate_dx)):
+    for name, got, want in zip(("y", "dx"), (y, dx), layer.want(gate_dx, slot_by_slot)):
         differ = (got != want).double().mean().item()
         assert differ < 0.03, (name, differ)
 
@@ -140,3 +143,46 @@ def test_accumulated_product_of_a_ragged_contraction(dev):
     product = torch.bmm(x[0].double()[:, None], w.double()[routing[:, 0]])[:, 0]
     differ = (out.cpu() != (old.double() + product).to(torch.bfloat16)).double().mean().item()
     assert differ < 0.01, differ
+
+
+@pytest.mark.parametrize("fused", [0, 2])
+@pytest.mark.parametrize("gate", [False, True])
+@pytest.mark.parametrize("masters,d,h,k,act", [(True, 64, 128, 2, "gelu"), (True, 64, 128, 2, "own"), (True, 520, 264, 3, "gelu"),
+                                               (True, 72, 136, 2, "own"), (False, 72, 136, 2, "gelu"), (False, 64, 264, 3, "own")])
+def test_slots(dev, masters, d, h, k, act, gate, fused):
+    """Masters used for few rows: the slots' fp32 products are added and rounded once.  Hidden sizes that are no multiple of 32:
+    each joins the rounded sum of those before it."""
+    _check(_Layer(dev, torch.bfloat16, 60, d, h, 12, k, masters, act), fused, gate, slot_by_slot=not masters)
+
+
+@pytest.mark.parametrize("bad", [-1, 6])
+def test_slots_without_an_expert(dev, bad):
+    """Ids of no expert: the (token, slot) adds nothing, and a token without any slot gets zeros."""
+    from types import SimpleNamespace
+
+    from hexa_moe.impls import layers
+    T, d, h, E, k = 70, 64, 96, 6, 2
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(T, d, generator=g).to(torch.bfloat16).to(dev).requires_grad_(True)
+    w1, w2 = ((torch.randn(E, h, d, generator=g) / 8).to(dev).requires_grad_(True) for _ in range(2))
+    dy = torch.randn(T, d, generator=g).to(torch.bfloat16).to(dev)
+    routing = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)])
+    routing[::3, 0] = bad
+    routing[::4, 1] = bad
+    config = SimpleNamespace(num_global_experts=E, routing_=routing.to(dev), activation_fn=torch.nn.functional.gelu, stage=0,
+                             route_pool=layers.RoutePool())
+    y = layers.FusedMoE_Shared_CudaCore.apply(config, x, w1, w2, None, None)
+    y.backward(dy)
+    xr = x.detach().double().cpu().requires_grad_(True)
+    r1, r2 = (w.detach().to(torch.bfloat16).double().cpu() for w in (w1, w2))
+    want = torch.zeros(T, d, dtype=torch.float64)
+    for s in range(k):
+        for e in range(E):
+            rows = (routing[:, s] == e).nonzero()[:, 0]
+            want = want.index_add(0, rows, torch.nn.functional.gelu(xr[rows] @ r1[e].t()) @ r2[e])
+    want.backward(dy.double().cpu())
+    for got, ref in ((y, want), (x.grad, xr.grad)):
+        got, ref = got.detach().double().cpu(), ref.detach()
+        assert (got - ref).norm() <= 6.8e-3 * ref.norm()      # roundings as in test_gpu_backward_fused.py
+        none = (routing == bad).all(1)
+        assert none.any() and (got[none] == 0).all()
