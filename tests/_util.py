@@ -69,3 +69,20 @@ def make_linear(T, d_in, d_out, E, k, seed, dtype, m2s):
     W = uniform((E, d_in, d_out), b, g).to(dtype)
     bias = uniform((E, d_out), b, g).to(dtype)
     return x, W, bias
+
+
+def layer_fp64(x, routing, wg, W1, W2, b1, b2, dy, aux):
+    """One MoE layer with GELU and the GShard loss for a given decision, forward and backward through autograd in 64 bits on
+    the CPU: (y, l_aux, [dx, dwg, dW1, dW2, db1, db2]) for the gradients dy of y and aux of l_aux (absent biases: None)."""
+    from oracle import hexa_oracle as O
+    x, wg, W1, W2, b1, b2 = (None if t is None else t.detach().double().cpu().requires_grad_(True) for t in (x, wg, W1, W2, b1, b2))
+    routing = routing.long().cpu()
+    l_aux = O.gshard_loss(torch.softmax(x @ wg.t(), dim=1), routing)
+    y = torch.zeros(x.shape[0], W2.shape[2], dtype=torch.float64)
+    for s in range(routing.shape[1]):
+        for e in range(W1.shape[0]):
+            rows = (routing[:, s] == e).nonzero()[:, 0]
+            h = x[rows] @ W1[e].t() + (0 if b1 is None else b1[e])
+            y = y.index_add(0, rows, 0.5 * h * torch.erfc(-h / math.sqrt(2.0)) @ W2[e] + (0 if b2 is None else b2[e]))
+    torch.autograd.backward([y, l_aux], [dy.detach().double().cpu(), torch.full_like(l_aux, aux)])
+    return y.detach(), l_aux.detach(), [None if t is None else t.grad for t in (x, wg, W1, W2, b1, b2)]

@@ -49,3 +49,31 @@ def test_rounded_on_the_way(dev, dtype, act, T, d, E, k, offset):
     # rounded like y16, or not rounded at all: within the rounding of a 16-bit value (fp16: of its subnormals)
     ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
     assert ((y - y16.float()).abs() <= ulp * y16.float().abs() + 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,d,E,k", [(2304, 384, 32, 1), (65, 264, 5, 1), (500, 128, 8, 2)])
+def test_against_fp64(dev, dtype, T, d, E, k):
+    """The layer in 64 bits for the tokens and weights as they are rounded.  Four roundings in a chain, as in
+    test_gpu_backward_fused.py."""
+    from _util import layer_fp64, rel_err
+    from hexa_moe import moe as hmoe
+    torch.manual_seed(4)
+    m = hmoe.MoE_Cascaded(gate_type={"type": "top", "k": k, "gate_noise": 0.0, "fp32_gate": True}, model_dim_list=[d], moe_idx_list=[0],
+                          num_global_experts=E, total_depth=1, data_centric=True, activation_fn=F.gelu)
+    for p in m.parameters():
+        torch.nn.init.uniform_(p.data, -0.08, 0.08)
+    m = m.to(dev)
+    x = torch.randn(T, d, device=dev).requires_grad_(True)
+    with torch.autocast("cuda", dtype=dtype):
+        y, l_aux = m(0, x)
+    dy = torch.randn(T, d, device=dev).to(dtype)
+    torch.autograd.backward([y, l_aux], [dy.to(y.dtype), torch.ones_like(l_aux)])
+    params = [m.gates[0].wg.weight, m.batched_fc1_w[0], m.batched_fc2_w[0], m.batched_fc1_bias[0], m.batched_fc2_bias[0]]
+    w = [params[0], params[1].to(dtype), params[2].to(dtype), *params[3:]]
+    y_ref, aux_ref, grads = layer_fp64(x.to(dtype), m.dispatch_params.routing_, *w, dy, 1.0)
+    assert abs(l_aux.item() - aux_ref.item()) <= 1e-5 * abs(aux_ref.item())
+    most = 6.8e-3 if dtype == torch.bfloat16 else 8.5e-4
+    names = ("y", "dx", "dwg", "dW1", "dW2", "db1", "db2")
+    errs = {n: rel_err(a.grad if n != "y" else a, b)[0] for n, a, b in zip(names, [y, x] + params, [y_ref] + grads)}
+    assert all(e <= most for e in errs.values()), errs
