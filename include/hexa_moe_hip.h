@@ -303,7 +303,8 @@ typedef struct hexa_moe_depth_opts {
     int32_t size;      /* sizeof(hexa_moe_depth_opts) as the caller knows it; what it does not know is 0 */
     int32_t part;      /* HEXA_PART_* (0: all) */
     int32_t wide_y;    /* 1: the forward stores y as fp32 (16-bit act_dt and top_k 1 only) */
-    int32_t careful;   /* 1: GELU, GELU' and the sums into y and dx take the fp32 product, not the one rounded to act_dt */
+    int32_t careful;   /* 1: GELU, GELU' and the sums into y and dx take the fp32 product, not the one rounded to act_dt (top_k > 1:
+                        * with workspaces that hold an fp32 result of every slot) */
     int32_t no_gate;   /* 1: wg is NULL in every call, and the workspaces leave the router's and the gate's share out */
 } hexa_moe_depth_opts;
 

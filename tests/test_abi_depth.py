@@ -72,3 +72,16 @@ def test_a_part_takes_its_own_scratch(no_gate, act_dt):
     colsum = k * (T // 128 + E) * h * 4
     gate = T * E * 4 + T * d * size + (T // 64 + 1) * E * d * 4
     assert bwd[1] <= plan + colsum + partial + slots + (0 if no_gate else gate)
+
+
+@pytest.mark.parametrize("act_dt,careful", [(0, 1), (2, 0), (2, 1)])
+def test_scratch_of_slots_that_are_added_unrounded(act_dt, careful):
+    """16-bit tokens with the option: one fp32 result a slot; otherwise a result of the tokens' type for each slot but the first."""
+    from hexa_moe import _lib
+    T, k, E, d, h = 512, 3, 64, 256, 512
+    desc = _lib.DepthDesc(T, k, E, d, h, d, act_dt, act_dt, *[0] * 6, 0, 0.0, 0.0, 0)
+    ask = lambda c: _bytes("hexa_moe_depth_part_ws_bytes", ctypes.byref(desc),      # noqa: E731
+                           ctypes.byref(_lib.DepthOpts(ctypes.sizeof(_lib.DepthOpts), 7, 0, c, 0)))
+    (rc, fwd, bwd), (rc0, fwd0, bwd0) = ask(careful), ask(0)
+    more = T * d * (k * 4 - (k - 1) * 2) if careful and act_dt else 0
+    assert rc == rc0 == 0 and (fwd - fwd0, bwd - bwd0) == (more, more)
