@@ -1,30 +1,34 @@
-// ESMM and ESTMM in true fp32 on gfx950: v_mfma_f32_32x32x2_f32 (fp32 multiply, fp32 accumulate).  Unlike the
-// reference, which rounds fp32 operands to fp16 before its WMMA (kernels/esmm_full.cu:128-130,167-169), nothing is
-// rounded, so results agree with an fp32 matmul to ~1e-6.
+// ESMM and ESTMM for fp32 operands on gfx950, on the bf16 matrix pipes and as exact as on the fp32 ones.  Unlike the reference,
+// which rounds fp32 operands to fp16 before its WMMA (kernels/esmm_full.cu:128-130,167-169), nothing is rounded away.
 //
-// What bounds these kernels is the matrix pipeline: one such MFMA is 64 cycles for 4096 flop (131-145 TFLOP/s over the
-// chip from registers, the clock falling with random operands).  A 64 x 64 tile's 32 contraction indices are 1024 cycles
-// of each SIMD against 16 KB copied, so copies and LDS reads have time -- if they do not stand between the MFMAs:
-//   * four wavefronts multiply (32 x 32 each) and four copy: tiles stream into LDS with the asynchronous copy
-//     (global_load_lds_dwordx4), two or three stages, one barrier per stage;
-//   * a multiplying wavefront reads half a stage while the MFMAs of the other half run, also across that barrier;
-//   * tiles are small and three or four workgroups share a CU, so that one's start and end meet another's MFMAs and
-//     256 CUs finish together; all routing slots of a slot-summed result run in one launch; an ESTMM with few tiles is
-//     cut along its token lists.
-// Measured at 9216 tokens, 384 -> 1536, 8 experts, top-2 (21.7 GFLOP a launch; before: 128 x 128 tiles through registers,
-// two barriers per 16 indices, one launch per slot): fc1 + GELU 257 -> 237 us, fc2 465 -> 199, dW 446 -> 227, dy1 348 -> 242,
-// dx 479 -> 197, and at 2048 tokens, 128 -> 512 28 -> 11, 58 -> 16, 92 -> 18 us.  128 x 64 tiles, copies issued between the
-// MFMAs by the multiplying wavefronts, and one persistent workgroup pair per CU were measured too: 0 to 15 % slower.
+// A fp32 value is the sum of three bf16 values, exactly: h = bf16(x), m = bf16(x - h), l = x - h - m (8 + 8 + 8 bits of
+// significand, each rounded to nearest).  A product is then h h' + (h m' + m h') + (m m' + h l' + l h') and three terms below
+// 2^-24 of it that are left out; each is exact in the matrix pipe's fp32.  v_mfma_f32_32x32x16_bf16 takes 32 cycles for 16
+// contraction indices where v_mfma_f32_32x32x2_f32 takes 64 for two, so the six terms are 192 cycles against 512.
+// Error against 64 bits, in brackets v_mfma_f32_32x32x2_f32, on 64 x 64 and 128 x 128 tiles: 448 products a result 2.2e-7 (3.8e-7)
+// and 968 4.7e-7 (5.6e-7), lists of a few entries 5.4e-8 (6.3e-8); lower in each of 24 layers of 100 to 9000 tokens, 64 to 968 wide.
+// GELU and GELU' are gelu_full's, as exact as through erff.
 //
-// LDS tile formats (a stage holds 32 contraction indices):
-//   KC  contraction index fastest in memory: [row][32 k], 128 B per row.  The MFMA takes one contraction index per
-//       half-wavefront, and WHICH two indices it pairs is free: lanes 0..31 take k = 8g + j and lanes 32..63
-//       k = 8g + 4 + j, so a lane's four indices of a group are one ds_read_b128.  16-byte piece p of a row sits at
-//       position p ^ ((row >> 1) & 7): sixteen consecutive rows cover all 64 banks.
-//   KS  contraction index slowest in memory: [32 k][W columns].  Lanes read single floats, two rows of k per
-//       ds_read2st64_b32.  Piece ch of row k sits at ch ^ (8 * ((k >> 2) & 1)): the two half-wavefronts, four rows of k
-//       apart, use different halves of the banks.
-// The copy engine places lane i at LDS offset 16*i, so both swizzles choose which piece a lane fetches.
+// What the split has to be careful with, it leaves to the fp32 pipe: a stage of operands that holds a magnitude of 2^63 and
+// more (whose terms could overflow where the product does not), an infinity (0 times infinity in a term) or eight neighbours
+// that are all below 2^-100 (whose l would be a denormal bf16 value short of bits) is written to LDS unsplit and multiplied by
+// v_mfma_f32_32x32x2_f32.  A NaN is one in either way.
+//
+// Values are split once per workgroup, on their way from registers to LDS (6.5 vector instructions a value, about half the
+// MFMA cycles of a 128 x 128 tile), not once per wavefront that reads them; rows are fetched into registers a stage ahead.
+// One set of planes and two barriers a stage: 48 KB a workgroup, so that two of eight or three of four wavefronts share a CU and
+// one's split and barriers meet another's MFMAs.
+// What bounds them: matrix and vector instructions, which overlap in part only (a launch without the split, or without the MFMAs,
+// takes 0.9 and 0.6 of its time; without fetches 0.95).  At 9216 tokens, 384 -> 1536, 8 experts, top-2 (21.7 GFLOP a launch; before:
+// v_mfma_f32_32x32x2_f32 fed by asynchronous copies, at 64 % of its pipe's rate), kernel times inside a training step: fc1 + GELU
+// 245 -> 170 us, fc2 211 -> 136, dW 234 -> 143 and a fold of 19, dy1 248 -> 171, the step 1.44 -> 1.03 ms; 2048 rows, 8 experts:
+// 128 -> 512 10.3 -> 9.7, 512 -> 128 15.5 -> 14.6.  Fetching two stages ahead, one barrier a stage with two sets of planes (one
+// workgroup a CU), and splitting between a stage's MFMAs were measured too: 0 to 20 % slower.
+//
+// LDS tile formats, three planes (h, m, l) of each operand, a stage holds KD contraction indices:
+//   KC  contraction index fastest in memory: [row][KD], fragments by ds_read_b128 (frag_kc)
+//   KS  contraction index slowest in memory: [KD][W columns], fragments by ds_read_b64_tr_b16
+// 16-byte pieces are permuted inside a row so that neither the writes nor the reads meet on a bank.
 //
 // Replaces esmm_shared_tensor_kernel_vectorized_accum_full (kernels/esmm_full.cu:58-246) and the
 // ESMM / ESTMM tasks of fused_grad_*_kernel_vectorized_full (kernels/fused_ops_full.cu:117-371).
@@ -36,126 +40,231 @@
 namespace hexa {
 namespace {
 
-constexpr int KD = 32;                  // contraction indices per stage
-constexpr int NT = 512;                 // 2 x 2 wavefronts that multiply and four that copy
 typedef __attribute__((ext_vector_type(4))) float f32x4;
-typedef __attribute__((ext_vector_type(2))) float f32x2;
+typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
 
-constexpr int BM = 64, BN = 64;         // workgroup tile: one 32 x 32 block per multiplying wavefront
-constexpr int OPERAND_BYTES = 64 * KD * 4, STAGE_BYTES = 2 * OPERAND_BYTES;
-constexpr int R_CPW = 2, CPW = 4;       // copies per wavefront and stage: two of each operand
-// stages, and the wavefronts per SIMD the registers are sized for
-template <int STAGES_, int WAVES_> struct Depth { static constexpr int STAGES = STAGES_, WAVES = WAVES_; };
-using Deep = Depth<3, 6>;               // 48 KB: three workgroups per CU
-using Many = Depth<2, 8>;               // 32 KB: four
-
-// LDS reads in inline assembly: the compiler would order plain ones behind the copies in flight (see dma_common.h);
-// not usable before frag_fence().
-__device__ __forceinline__ f32x4 lds_read_f4(unsigned addr) {
-    f32x4 r;
-    asm volatile("ds_read_b128 %0, %1" : "=v"(r) : "v"(addr));
-    return r;
-}
-template <int A, int B> __device__ __forceinline__ f32x2 lds_read_2f(unsigned addr) {   // units of 256 bytes
-    f32x2 r;
-    asm volatile("ds_read2st64_b32 %0, %1 offset0:%2 offset1:%3" : "=v"(r) : "v"(addr), "n"(A), "n"(B));
-    return r;
-}
-
-// One 32-wide block of an operand for half a stage (HALF 0: k = 0..15, HALF 1: k = 16..31): at(g, j) is this lane's value
-// for k = 16 HALF + 8g + 4(lane >> 5) + j.
-struct FragKC {
-    f32x4 v[2];
-    // lane part of the address of group g of a stage
-    static __device__ __forceinline__ unsigned lane_addr(int lane, int g) {
-        const int row = lane & 31;
-        return row * 128 + (((2 * g + (lane >> 5)) ^ ((row >> 1) & 7)) << 4);
-    }
-    template <int HALF> __device__ __forceinline__ void read(const unsigned (&la)[4], unsigned base) {
-#pragma unroll
-        for (int g = 0; g < 2; ++g) v[g] = lds_read_f4(la[2 * HALF + g] + base);
-    }
-    __device__ __forceinline__ void pin() {
-#pragma unroll
-        for (int g = 0; g < 2; ++g) asm volatile("" : "+v"(v[g]));
-    }
-    __device__ __forceinline__ float at(int g, int j) const { return v[g][j]; }
+// Workgroup tile: WR x WF wavefronts, every one multiplies RB x FB blocks of 32 x 32; KD contraction indices per stage, of which
+// KG groups of wavefronts take a part each (and add their sums at the end).  WAVES: wavefronts per SIMD the registers are sized
+// for (three planes of both operands: 48 KB of LDS).
+template <int WR_, int WF_, int KG_, int RB_, int FB_, int KD_, int WAVES_> struct Tile {
+    static constexpr int WR = WR_, WF = WF_, KG = KG_, NT = 64 * WR_ * WF_ * KG_, RB = RB_, FB = FB_, KD = KD_, WAVES = WAVES_;
+    static constexpr int BM = 32 * RB_ * WR_, BN = 32 * FB_ * WF_, KSTEPS = KD_ / 16 / KG_;
+    static constexpr int R_PLANE = BM * KD * 2, F_PLANE = BN * KD * 2, F_AT = 3 * R_PLANE, BYTES = F_AT + 3 * F_PLANE;
+    static constexpr int RO = BM * KD / 8 / NT, FO = BN * KD / 8 / NT;      // octets a thread fetches and splits in a stage
+    static_assert(RO * NT * 8 == BM * KD && FO * NT * 8 == BN * KD, "whole octets per thread");
+    static_assert(KG <= 2 && (KG - 1) * WR * WF * RB * FB * 4096 <= BYTES, "one other group's sums fit into the planes");
 };
-struct FragKS {                   // 64 columns per row of k: 256 bytes
-    f32x2 v[2][2];
-    static __device__ __forceinline__ unsigned lane_addr(int lane, int col0) {
-        const int kh = lane >> 5, col = col0 + (lane & 31);
-        return kh * 4 * 256 + ((((col >> 2) ^ (8 * kh)) << 4) | ((col & 3) << 2));
-    }
-    template <int HALF> __device__ __forceinline__ void read(unsigned addr) {
-        constexpr int K0 = 16 * HALF;
-        v[0][0] = lds_read_2f<K0, K0 + 1>(addr);      v[0][1] = lds_read_2f<K0 + 2, K0 + 3>(addr);
-        v[1][0] = lds_read_2f<K0 + 8, K0 + 9>(addr);  v[1][1] = lds_read_2f<K0 + 10, K0 + 11>(addr);
-    }
-    __device__ __forceinline__ void pin() {
+using Wide = Tile<2, 4, 1, 2, 1, 32, 4>;
+using Deep = Tile<2, 2, 2, 1, 1, 64, 4>;
+
+// Eight neighbouring values of an operand: along the contraction (KC) or across it (KS).
+struct Octet { f32x4 a, b; };
+
+__device__ __forceinline__ float bits_f(unsigned u) { return __uint_as_float(u); }
+__device__ __forceinline__ float largest(float m, float a, float b) {      // of |a|, |b| and m; a NaN is passed over
+    float r;
+    asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
+    return r;
+}
+// the planes of eight values; whether they are to be multiplied as they are instead
+__device__ __forceinline__ bool split(const Octet& v, u32x4& h, u32x4& m, u32x4& l) {
+    const float x[8] = {v.a.x, v.a.y, v.a.z, v.a.w, v.b.x, v.b.y, v.b.z, v.b.w};
+    float big = 0.f;
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            asm volatile("" : "+v"(v[g][0]));
-            asm volatile("" : "+v"(v[g][1]));
+    for (int q = 0; q < 4; ++q) {
+        const float a = x[2 * q], b = x[2 * q + 1];
+        big = largest(big, a, b);
+        const unsigned hw = pack2<__bf16>(a, b);
+        const float ra = a - bits_f(hw << 16), rb = b - bits_f(hw & 0xffff0000u);
+        const unsigned mw = pack2<__bf16>(ra, rb);
+        h[q] = hw;
+        m[q] = mw;
+        l[q] = pack2<__bf16>(ra - bits_f(mw << 16), rb - bits_f(mw & 0xffff0000u));
+    }
+    constexpr unsigned LOW = 0x0d800000u, HIGH = 0x5f000000u;       // 2^-100, 2^63
+    const unsigned u = __float_as_uint(big);
+    return u - LOW >= HIGH - LOW && u != 0;
+}
+// the same eight values unsplit: their upper and lower halves in the planes of h and m
+__device__ __forceinline__ void halves(const Octet& v, u32x4& hi, u32x4& lo) {
+    const float x[8] = {v.a.x, v.a.y, v.a.z, v.a.w, v.b.x, v.b.y, v.b.z, v.b.w};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const unsigned a = __float_as_uint(x[2 * q]), b = __float_as_uint(x[2 * q + 1]);
+        hi[q] = (a >> 16) | (b & 0xffff0000u);
+        lo[q] = (a & 0xffffu) | (b << 16);
+    }
+}
+
+// Where piece `oct` (eight values) of row r of an operand sits in a plane of width W, and which pieces a lane handles: octet i
+// of thread tid is piece piece_of(tid) of row row_of(tid, i).
+template <bool KS, int W, int KD, int NT = 64> struct Place {
+    static constexpr int PPR = KS ? W / 8 : KD / 8, ROWS = NT / PPR;
+    static __device__ __forceinline__ int row_of(int tid, int i) { return tid / PPR + i * ROWS; }
+    static __device__ __forceinline__ int piece_of(int tid) { return tid % PPR; }
+    static __device__ __forceinline__ int swizzle(int row) {
+        if (!KS) return kc_swizzle<KD>(row);
+        return W == 64 ? ((row >> 1) & 1) << 2 : (row & 3) << 2;     // the four rows a transposing read touches: other banks
+    }
+    static __device__ __forceinline__ int at(int row, int piece) { return row * PPR * 16 + ((piece ^ swizzle(row)) << 4); }
+};
+
+typedef __attribute__((address_space(3))) s16x4* lds_s16x4_t;
+// the 32 x 16 fragment of a plane: rows col0 .. col0 + 31, contraction indices 16 ks + 8 (lane >> 5) + 0..7
+template <bool KS, int W, int KD> __device__ __forceinline__ u32x4 fragment(const char* plane, int col0, int ks, int lane) {
+    if constexpr (!KS) {
+        return frag_kc<u32x4, KD>(plane, col0, ks, lane);
+    } else {
+        const int grp = lane >> 4, s = lane & 15;
+        const int col = col0 + (grp & 1) * 16 + (s & 3) * 4, k = ks * 16 + (grp >> 1) * 8 + (s >> 2);
+        union { u32x4 v; s16x4 h[2]; } r;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            const char* p = plane + Place<true, W, KD>::at(k + 4 * half, col >> 3) + (col & 7) * 2;
+            r.h[half] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(__attribute__((address_space(3))) const void*)p);
+        }
+        return r.v;
+    }
+}
+__device__ __forceinline__ bf16x8 as_bf16(u32x4 v) {
+    union { u32x4 u; bf16x8 b; } c;
+    c.u = v;
+    return c.b;
+}
+__device__ __forceinline__ float whole(u32x4 hi, u32x4 lo, int j) {
+    return bits_f(j & 1 ? (hi[j >> 1] & 0xffff0000u) | (lo[j >> 1] >> 16) : (hi[j >> 1] << 16) | (lo[j >> 1] & 0xffffu));
+}
+
+// acc += F x R over the stage in LDS.  A lane ends up with row lane % 32 of R and, per group of four registers, 4 consecutive
+// columns of F, from either instruction.
+template <typename C, bool F_KS, bool R_KS>
+__device__ __forceinline__ void multiply(const char* smem, int kg, int wr, int wf, int lane, f32x16 (&acc)[C::FB][C::RB]) {
+    // the smallest terms first: of the first 16 products only the last addition rounds the whole sum
+    constexpr int TERMS[6][2] = {{0, 2}, {2, 0}, {1, 1}, {0, 1}, {1, 0}, {0, 0}};
+#pragma unroll
+    for (int step = 0; step < C::KSTEPS; ++step) {
+        const int ks = kg * C::KSTEPS + step;
+        u32x4 r[C::RB][3];
+#pragma unroll
+        for (int i = 0; i < C::RB; ++i)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) r[i][q] = fragment<R_KS, C::BM, C::KD>(smem + q * C::R_PLANE, (wr * C::RB + i) * 32, ks, lane);
+#pragma unroll
+        for (int j = 0; j < C::FB; ++j) {
+            u32x4 f[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) f[q] = fragment<F_KS, C::BN, C::KD>(smem + C::F_AT + q * C::F_PLANE, (wf * C::FB + j) * 32, ks, lane);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int t = 0; t < 6; ++t)
+#pragma unroll
+                for (int i = 0; i < C::RB; ++i) acc[j][i] = Mfma<__bf16>::run(as_bf16(f[TERMS[t][0]]), as_bf16(r[i][TERMS[t][1]]), acc[j][i]);
         }
     }
-    __device__ __forceinline__ float at(int g, int j) const { return v[g][j >> 1][j & 1]; }
-};
-// half a stage of both operands: a wavefront's columns (F) and rows (R)
-template <typename F, typename R> struct Half {
-    F f;
-    R r;
-    __device__ __forceinline__ void fence() {        // the reads have returned; nothing that uses them moves ahead of this
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        f.pin();
-        r.pin();
-    }
-    // acc (+)= F x R: a lane ends up with row lane%32 of R and, per group of four registers, 4 consecutive columns of F
-    __device__ __forceinline__ void multiply(f32x16& acc) const {
+}
+template <typename C, bool F_KS, bool R_KS>
+__device__ __forceinline__ void multiply_whole(const char* smem, int kg, int wr, int wf, int lane, f32x16 (&acc)[C::FB][C::RB]) {
+    for (int ks = kg * C::KSTEPS; ks < (kg + 1) * C::KSTEPS; ++ks) {
 #pragma unroll
-        for (int g = 0; g < 2; ++g)
+        for (int j = 0; j < C::FB; ++j) {
+            u32x4 f[2];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(f.at(g, k), r.at(g, k), acc, 0, 0, 0);
+            for (int q = 0; q < 2; ++q) f[q] = fragment<F_KS, C::BN, C::KD>(smem + C::F_AT + q * C::F_PLANE, (wf * C::FB + j) * 32, ks, lane);
+#pragma unroll
+            for (int i = 0; i < C::RB; ++i) {
+                u32x4 r[2];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) r[q] = fragment<R_KS, C::BM, C::KD>(smem + q * C::R_PLANE, (wr * C::RB + i) * 32, ks, lane);
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(whole(f[0], f[1], k), whole(r[0], r[1], k), acc[j][i], 0, 0, 0);
+            }
+        }
     }
-};
-// A multiplying wavefront's nk stages of a tile.  load0 / load1(h) issue the reads of the current stage's halves, advance()
-// makes the next stage the current one.  The half that follows is read while the MFMAs of the one before run, also across
-// the barrier behind which the next stage may be read (and this one overwritten).
-template <typename P, typename L0, typename L1, typename A>
-__device__ __forceinline__ void multiply_stages(int nk, bool busy, f32x16& acc, L0 load0, L1 load1, A advance) {
-    if (!busy) {
-        for (int kt = 0; kt < nk; ++kt) { barrier_nofence(); advance(); }
-        return;
-    }
-    P a, b;
-    barrier_nofence();
-    load0(a);
+}
+
+// The stages of a tile.  load(step, r, f) fetches a step's values into registers (the caller's addresses move on with it); the
+// values of a step are fetched while the step before is multiplied, and split and written while the CU's other workgroups
+// multiply.
+template <typename C, bool F_KS, bool R_KS, typename L>
+__device__ __forceinline__ void multiply_stages(int nk, bool busy, char* smem, int* sWhole, int tid, f32x16 (&acc)[C::FB][C::RB], L load) {
+    using PR = Place<R_KS, C::BM, C::KD, C::NT>;
+    using PF = Place<F_KS, C::BN, C::KD, C::NT>;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kg = wave / (C::WR * C::WF), wr = wave / C::WF % C::WR, wf = wave % C::WF;
+    Octet r[C::RO], f[C::FO];
+    auto each = [&](auto&& put) {
+#pragma unroll
+        for (int i = 0; i < C::RO; ++i) put(r[i], smem + PR::at(PR::row_of(tid, i), PR::piece_of(tid)), C::R_PLANE);
+#pragma unroll
+        for (int i = 0; i < C::FO; ++i) put(f[i], smem + C::F_AT + PF::at(PF::row_of(tid, i), PF::piece_of(tid)), C::F_PLANE);
+    };
+    if (nk > 0) load(0, r, f);
+    if (tid < 2) sWhole[tid] = 0;
     for (int kt = 0; kt < nk; ++kt) {
-        a.fence();
-        load1(b);
-        __builtin_amdgcn_sched_barrier(0);
-        a.multiply(acc);
-        __builtin_amdgcn_sched_barrier(0);
-        b.fence();
-        advance();
-        if (kt + 1 < nk) {
-            barrier_nofence();
-            load0(a);
+        __syncthreads();                                  // everyone is done reading the stage before
+        bool odd = false;
+        each([&](const Octet& v, char* to, int plane) {
+            u32x4 h, m, l;
+            odd |= split(v, h, m, l);
+            *reinterpret_cast<u32x4*>(to) = h;
+            *reinterpret_cast<u32x4*>(to + plane) = m;
+            *reinterpret_cast<u32x4*>(to + 2 * plane) = l;
+        });
+        // (one word for even and one for odd steps: the other one was last read before the barrier above)
+        if (tid == 0) sWhole[(kt + 1) & 1] = 0;
+        if (odd) sWhole[kt & 1] = 1;
+        __syncthreads();
+        if (__builtin_expect(__builtin_amdgcn_readfirstlane(sWhole[kt & 1]), 0)) {
+            // (the stage is multiplied here, and the planes are left as zeros for what follows: two ways of adding to the
+            // accumulators that meet behind a branch made the compiler copy them in every stage)
+            __syncthreads();
+            each([&](const Octet& v, char* to, int plane) {
+                u32x4 hi, lo;
+                halves(v, hi, lo);
+                *reinterpret_cast<u32x4*>(to) = hi;
+                *reinterpret_cast<u32x4*>(to + plane) = lo;
+                *reinterpret_cast<u32x4*>(to + 2 * plane) = u32x4{0u, 0u, 0u, 0u};
+            });
+            __syncthreads();
+            multiply_whole<C, F_KS, R_KS>(smem, kg, wr, wf, lane, acc);
+            __syncthreads();
+            each([&](const Octet&, char* to, int plane) {
+                *reinterpret_cast<u32x4*>(to) = u32x4{0u, 0u, 0u, 0u};
+                *reinterpret_cast<u32x4*>(to + plane) = u32x4{0u, 0u, 0u, 0u};
+            });
+            __syncthreads();
         }
-        __builtin_amdgcn_sched_barrier(0);
-        b.multiply(acc);
-        __builtin_amdgcn_sched_barrier(0);
+        if (kt + 1 < nk) load(kt + 1, r, f);
+        if (busy) multiply<C, F_KS, R_KS>(smem, kg, wr, wf, lane, acc);
     }
 }
 
-// which piece a lane fetches in wavefront copy c: KC (8 rows per copy), KS (4 rows of k per copy)
-__device__ __forceinline__ void kc32_lane(int c, int lane, int& row, int& piece) {
-    row = 8 * c + (lane >> 3);
-    piece = (lane & 7) ^ ((row >> 1) & 7);
-}
-__device__ __forceinline__ void ks32_lane(int c, int lane, int& kk, int& piece) {
-    kk = 4 * c + (lane >> 4);
-    piece = (lane & 15) ^ (8 * ((kk >> 2) & 1));
+// The groups' sums added, in the first one's accumulators; whether this wavefront is of that group.
+template <typename C> __device__ __forceinline__ bool combine(char* smem, int kg, int wave, int lane, f32x16 (&acc)[C::FB][C::RB]) {
+    if constexpr (C::KG > 1) {
+        f32x4* const at = reinterpret_cast<f32x4*>(smem) + (wave % (C::WR * C::WF)) * (C::RB * C::FB * 256) + lane;
+        __syncthreads();                                 // the planes have been read
+        if (kg > 0) {
+#pragma unroll
+            for (int b = 0; b < C::RB * C::FB; ++b)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const f32x16& v = acc[b / C::RB][b % C::RB];
+                    at[(b * 4 + g) * 64] = f32x4{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]};
+                }
+        }
+        __syncthreads();
+        if (kg > 0) return false;
+#pragma unroll
+        for (int b = 0; b < C::RB * C::FB; ++b)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const f32x4 v = at[(b * 4 + g) * 64];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc[b / C::RB][b % C::RB][4 * g + q] += v[q];
+            }
+    }
+    return true;
 }
 
 struct Esmm32K {
@@ -166,11 +275,11 @@ struct Esmm32K {
     int accumulate, act;
 };
 
-template <bool W_IN_OUT, bool WIDE, typename S>
-__global__ __launch_bounds__(NT, S::WAVES) void esmm32_kernel(Esmm32K p) {
-    constexpr int STAGES = S::STAGES, H = HEXA_TILE_ROWS / BM;   // H workgroup tiles per row tile of the routing
+template <bool W_IN_OUT, bool BIG, typename C>
+__global__ __launch_bounds__(C::NT, C::WAVES) void esmm32_kernel(Esmm32K p) {
+    constexpr int BM = C::BM, BN = C::BN, KD = C::KD, H = HEXA_TILE_ROWS / BM;   // H workgroup tiles per row tile of the routing
     extern __shared__ __attribute__((aligned(1024))) char smem[];
-    __shared__ int sTok[BM];
+    __shared__ int sTok[BM], sWhole[2];
 
     // Every XCD (workgroup ids go round-robin over the 8 of them) walks one contiguous eighth of the valid tiles,
     // column tiles fastest: an expert's weights are then fetched into one L2.
@@ -194,121 +303,101 @@ __global__ __launch_bounds__(NT, S::WAVES) void esmm32_kernel(Esmm32K p) {
     if (rows <= 0) return;
     const int n0 = nt * BN;
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave8 & 3, wr = wave >> 1, wf = wave & 1;
-    const bool copies = wave8 >= 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kg = wave / (C::WR * C::WF), wr = wave / C::WF % C::WR, wf = wave % C::WF;
     const int K = p.K, N = p.N;
     if (tid < BM) sTok[tid] = tid < rows ? p.token_ids[(size_t)s * p.T + row_start + tid] : -1;
     __syncthreads();
 
-    // Sources of this lane's copies: bases every lane shares plus 32-bit byte offsets (64-bit ones where an operand has
-    // 4 GiB and more): a copy whose address is one register beside a scalar pair disturbs the MFMAs of the SIMD's other
-    // wavefronts far less.  Lanes with nothing to fetch (rows past the tile's end, columns past N) re-read the first bytes
-    // of the tensor: what they produce is never stored.  Contraction indices past K come from a block of zeros, in both
-    // operands.
-    using Off = std::conditional_t<WIDE, size_t, unsigned>;
+    // Sources of this lane's values: bases every lane shares plus 32-bit byte offsets (64-bit ones where an operand has
+    // 4 GiB and more).  Lanes with nothing to fetch (rows past the tile's end, columns past N) read the first row or column:
+    // what they produce is never stored.  Contraction indices past K are zeros in both operands.
+    using Off = std::conditional_t<BIG, size_t, unsigned>;
+    using PR = Place<false, BM, KD, C::NT>;
+    using PF = Place<W_IN_OUT, BN, KD, C::NT>;
     const char* const xbase = reinterpret_cast<const char*>(p.x);
     const char* const wbase = reinterpret_cast<const char*>(p.w + (size_t)e * K * N);
-    Off off[CPW];
-    int kOf[CPW];                              // the stage's contraction index the lane fetches
+    Off offR[C::RO], offF[C::FO];
+    const int kR = PR::piece_of(tid) * 8;
+    const int n1 = n0 + PF::piece_of(tid) * 8, second = n1 + 4 < N ? 16 : 0;     // W_IN_OUT: where the octet's second half is
 #pragma unroll
-    for (int i = 0; i < CPW; ++i) {
-        int row, piece;
-        if (i < R_CPW) {
-            kc32_lane(wave + 4 * i, lane, row, piece);
-            const int tok = max(sTok[row], 0);
-            kOf[i] = piece * 4;
-            off[i] = (Off)((((size_t)p.x_slot_rows * s + tok) * K + piece * 4) * 4);
-        } else if (W_IN_OUT) {
-            ks32_lane(wave + 4 * (i - R_CPW), lane, row, piece);
-            const int n = n0 + piece * 4;
-            kOf[i] = row;
-            off[i] = (Off)(((size_t)row * N + (n < N ? n : 0)) * 4);
-        } else {
-            kc32_lane(wave + 4 * (i - R_CPW), lane, row, piece);
-            const int n = n0 + row;
-            kOf[i] = piece * 4;
-            off[i] = (Off)(((size_t)(n < N ? n : 0) * K + piece * 4) * 4);
-        }
+    for (int i = 0; i < C::RO; ++i) offR[i] = (Off)((((size_t)p.x_slot_rows * s + max(sTok[PR::row_of(tid, i)], 0)) * K + kR) * 4);
+#pragma unroll
+    for (int i = 0; i < C::FO; ++i) {
+        const int row = PF::row_of(tid, i);
+        if (W_IN_OUT) offF[i] = (Off)(((size_t)row * N + (n1 < N ? n1 : 0)) * 4);
+        else offF[i] = (Off)(((size_t)(n0 + row < N ? n0 + row : 0) * K + PF::piece_of(tid) * 8) * 4);
     }
     const Off stepF = W_IN_OUT ? (Off)KD * N * 4 : (Off)KD * 4;
-    const int nk = (K + KD - 1) / KD;
-    auto target = [&](int step, int i) {
-        return smem + (step % STAGES) * STAGE_BYTES + (i < R_CPW ? (wave + 4 * i) * 1024 : OPERAND_BYTES + (wave + 4 * (i - R_CPW)) * 1024);
-    };
-    auto copy = [&](int step, int i) {            // copy i of a step that lies inside the contraction
-        dma16((i < R_CPW ? xbase : wbase) + (size_t)off[i], target(step, i));
-        off[i] += i < R_CPW ? (Off)(KD * 4) : stepF;
-    };
-    auto issue = [&](int step) {
+    auto read4 = [](const char* base, Off off) { return *reinterpret_cast<const f32x4*>(base + (size_t)off); };
+    auto load = [&](int step, Octet (&r)[C::RO], Octet (&f)[C::FO]) {
         const int left = K - step * KD;
+        if (left >= KD) {
 #pragma unroll
-        for (int i = 0; i < CPW; ++i) {
-            if (left >= KD) copy(step, i);
-            else dma16(kOf[i] < left ? (i < R_CPW ? xbase : wbase) + (size_t)off[i] : reinterpret_cast<const char*>(g_zero_block), target(step, i));
+            for (int i = 0; i < C::RO; ++i) { r[i].a = read4(xbase, offR[i]); r[i].b = read4(xbase, offR[i] + 16); }
+#pragma unroll
+            for (int i = 0; i < C::FO; ++i) { f[i].a = read4(wbase, offF[i]); f[i].b = read4(wbase, offF[i] + (W_IN_OUT ? second : 16)); }
+        } else {
+            const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < C::RO; ++i) {
+                r[i].a = zero; r[i].b = zero;
+                if (kR < left) r[i].a = read4(xbase, offR[i]);
+                if (kR + 4 < left) r[i].b = read4(xbase, offR[i] + 16);
+            }
+#pragma unroll
+            for (int i = 0; i < C::FO; ++i) {
+                const int k = W_IN_OUT ? PF::row_of(tid, i) : PF::piece_of(tid) * 8;
+                f[i].a = zero; f[i].b = zero;
+                if (k < left) f[i].a = read4(wbase, offF[i]);
+                if (k + (W_IN_OUT ? 0 : 4) < left) f[i].b = read4(wbase, offF[i] + (W_IN_OUT ? second : 16));
+            }
         }
+#pragma unroll
+        for (int i = 0; i < C::RO; ++i) offR[i] += KD * 4;
+#pragma unroll
+        for (int i = 0; i < C::FO; ++i) offF[i] += stepF;
     };
 
-    if (copies) {
-#pragma unroll
-        for (int st = 0; st < STAGES - 1; ++st)
-            if (st < nk) issue(st);
-        for (int kt = 0; kt < nk; ++kt) {
-            wait_groups<CPW, STAGES - 2>(min(nk - 1 - kt, STAGES - 2));
-            barrier_nofence();      // the copies of step kt are in LDS, and everyone is done reading step kt - 1
-            if (kt + STAGES - 1 < nk) issue(kt + STAGES - 1);
-        }
-        return;
-    }
+    f32x16 acc[C::FB][C::RB];
+    zero_acc(acc);
+    const bool busy = wr * 32 * C::RB < rows && n0 + wf * 32 * C::FB < N;     // the others have no row or no column of the tile
+    multiply_stages<C, W_IN_OUT, false>((K + KD - 1) / KD, busy, smem, sWhole, tid, acc, load);
+    if (!combine<C>(smem, kg, wave, lane, acc) || !busy) return;
 
-    f32x16 acc;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
-    const bool busy = wr * 32 < rows && n0 + wf * 32 < N;     // the others have no row or no column of the tile
-    const unsigned lds0 = lds_addr(smem);
-    unsigned la[4], ksF = 0, stage_at = lds0;
-#pragma unroll
-    for (int g = 0; g < 4; ++g) la[g] = FragKC::lane_addr(lane, g);
-    if (W_IN_OUT) ksF = FragKS::lane_addr(lane, wf * 32);
-    using Pair = Half<std::conditional_t<W_IN_OUT, FragKS, FragKC>, FragKC>;
-    auto load = [&](Pair& h, auto half) {
-        constexpr int HALF = decltype(half)::value;
-        h.r.template read<HALF>(la, stage_at + wr * 32 * 128);
-        if constexpr (W_IN_OUT) h.f.template read<HALF>(ksF + stage_at + OPERAND_BYTES);
-        else h.f.template read<HALF>(la, stage_at + OPERAND_BYTES + wf * 32 * 128);
-    };
-    multiply_stages<Pair>(nk, busy, acc, [&](Pair& h) { load(h, std::integral_constant<int, 0>()); },
-                          [&](Pair& h) { load(h, std::integral_constant<int, 1>()); },
-                          [&]() { stage_at = stage_at + STAGE_BYTES == lds0 + STAGES * STAGE_BYTES ? lds0 : stage_at + STAGE_BYTES; });
-    if (!busy) return;
-
-    const int tok = sTok[wr * 32 + (lane & 31)];
-    if (tok < 0) return;
     const bool to_ws = p.ws != nullptr && s > 0;
     float* const outp = to_ws ? p.ws : p.out;
     const bool accumulate = p.accumulate && !to_ws;
     const size_t row0 = to_ws ? (size_t)p.T * (s - 1) : (size_t)p.out_slot_rows * s;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        const int n = n0 + wf * 32 + 8 * g + 4 * (lane >> 5);
-        if (n >= N) continue;
-        float4 v = make_float4(acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]);
-        if (p.bias) {
-            const float4 b = *reinterpret_cast<const float4*>(p.bias + (size_t)e * N + n);
-            v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w;
+    for (int i = 0; i < C::RB; ++i) {
+        const int tok = sTok[(wr * C::RB + i) * 32 + (lane & 31)];
+        if (tok < 0) continue;
+#pragma unroll
+        for (int j = 0; j < C::FB; ++j) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int n = n0 + (wf * C::FB + j) * 32 + 8 * g + 4 * (lane >> 5);
+                if (n >= N) continue;
+                float4 v = make_float4(acc[j][i][4 * g], acc[j][i][4 * g + 1], acc[j][i][4 * g + 2], acc[j][i][4 * g + 3]);
+                if (p.bias) {
+                    const float4 b = *reinterpret_cast<const float4*>(p.bias + (size_t)e * N + n);
+                    v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w;
+                }
+                const size_t off = (row0 + tok) * N + n;
+                if (p.act == HEXA_ACT_GELU_BWD) {
+                    const float4 y = *reinterpret_cast<const float4*>(p.out_act + off);
+                    v.x *= gelu_grad_full(y.x); v.y *= gelu_grad_full(y.y); v.z *= gelu_grad_full(y.z); v.w *= gelu_grad_full(y.w);
+                }
+                float4* dst = reinterpret_cast<float4*>(outp + off);
+                if (accumulate) {
+                    const float4 old = *dst;
+                    v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
+                }
+                *dst = v;
+                if (p.act == HEXA_ACT_GELU)
+                    *reinterpret_cast<float4*>(p.out_act + off) = make_float4(gelu_full(v.x), gelu_full(v.y), gelu_full(v.z), gelu_full(v.w));
+            }
         }
-        const size_t off = (row0 + tok) * N + n;
-        if (p.act == HEXA_ACT_GELU_BWD) {
-            const float4 y = *reinterpret_cast<const float4*>(p.out_act + off);
-            v.x *= gelu_grad_erf(y.x); v.y *= gelu_grad_erf(y.y); v.z *= gelu_grad_erf(y.z); v.w *= gelu_grad_erf(y.w);
-        }
-        float4* dst = reinterpret_cast<float4*>(outp + off);
-        if (accumulate) {
-            const float4 old = *dst;
-            v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
-        }
-        *dst = v;
-        if (p.act == HEXA_ACT_GELU)
-            *reinterpret_cast<float4*>(p.out_act + off) = make_float4(gelu_erf(v.x), gelu_erf(v.y), gelu_erf(v.z), gelu_erf(v.w));
     }
 }
 
@@ -321,14 +410,11 @@ struct Estmm32K {
     long total;
 };
 
-constexpr int RING = 8;      // steps whose token ids are in LDS (32 each)
-
-template <bool WIDE, typename S>
-__global__ __launch_bounds__(NT, S::WAVES) void estmm32_kernel(Estmm32K p) {
-    constexpr int STAGES = S::STAGES, LEAD = STAGES - 1;
-    static_assert(2 * LEAD <= RING, "ids are fetched LEAD steps ahead of the copies that need them");
+template <bool BIG, typename C>
+__global__ __launch_bounds__(C::NT, C::WAVES) void estmm32_kernel(Estmm32K p) {
+    constexpr int BM = C::BM, BN = C::BN, KD = C::KD;
     extern __shared__ __attribute__((aligned(1024))) char smem[];
-    __shared__ int sIds[RING * 32], sLoad[256], sExpert;
+    __shared__ int sLoad[256], sExpert, sWhole[2];
 
     const long logical = logical_tile(blockIdx.x, p.group);
     if (logical >= p.total) return;
@@ -337,8 +423,7 @@ __global__ __launch_bounds__(NT, S::WAVES) void estmm32_kernel(Estmm32K p) {
     const int rank = unit / p.parts, part = unit - rank * p.parts;
     const int m0 = (rem / p.ntn) * BM, n0 = (rem % p.ntn) * BN;
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave8 & 3, wr = wave >> 1, wf = wave & 1;
-    const bool copies = wave8 >= 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kg = wave / (C::WR * C::WF), wr = wave / C::WF % C::WR, wf = wave % C::WF;
     const int M = p.M, N = p.N, E = p.E;
 
     // Heaviest expert first (workgroups are dispatched in id order), up to 256 experts; beyond that by index.
@@ -369,148 +454,128 @@ __global__ __launch_bounds__(NT, S::WAVES) void estmm32_kernel(Estmm32K p) {
     const int nk = (int)((long)all_steps * (part + 1) / p.parts) - step0;
     if (p.parts == 1 && p.accumulate && nk == 0) return;
 
-    if (copies) {
-        struct Cursor { int s, r, end; };           // position in the list of slot s
-        auto seek = [&](Cursor c) {
-            while (c.s < p.k && c.r >= c.end) {
-                ++c.s;
-                if (c.s < p.k) { c.r = begin(c.s); c.end = end(c.s); }
-            }
-            return c;
-        };
-        auto advance = [&](Cursor c) { c.r += KD; return seek(c); };
-        Cursor start{0, begin(0), end(0)};
-        start = seek(start);
-        for (int skip = step0; skip > 0 && start.s < p.k;) {
-            const int here = (start.end - start.r + KD - 1) / KD, take = min(here, skip);
-            start.r += take * KD;
-            skip -= take;
-            start = seek(start);
+    struct Cursor { int s, r, end; };           // position in the list of slot s
+    auto seek = [&](Cursor c) {
+        while (c.s < p.k && c.r >= c.end) {
+            ++c.s;
+            if (c.s < p.k) { c.r = begin(c.s); c.end = end(c.s); }
         }
-        // the stage's token a lane fetches from and the byte in its row (columns past the result's edge re-read the row's
-        // first bytes: what they produce is never stored)
-        using Off = std::conditional_t<WIDE, size_t, unsigned>;
-        int tokOf[CPW];
-        unsigned colOf[CPW];
-#pragma unroll
-        for (int i = 0; i < CPW; ++i) {
-            int piece;
-            if (i < R_CPW) ks32_lane(wave + 4 * i, lane, tokOf[i], piece);
-            else ks32_lane(wave + 4 * (i - R_CPW), lane, tokOf[i], piece);
-            const int col = (i < R_CPW ? m0 : n0) + piece * 4;
-            colOf[i] = col < (i < R_CPW ? M : N) ? (unsigned)col * 4 : 0u;
-        }
-        const Off pitchP = (Off)M * 4, pitchQ = (Off)N * 4;
-        const unsigned ids_at = lds_addr(sIds);
-        const char* const zero = reinterpret_cast<const char*>(g_zero_block);
-        // every copying wavefront fetches the 32 ids of a step itself (the same words), so its own count of outstanding
-        // copies says when they are there
-        auto issue_ids = [&](int step, const Cursor& c) {
-            const int r = c.r + (lane & 31);
-            const void* src = c.s < p.k && r < c.end ? (const void*)(p.token_ids + (size_t)c.s * p.T + r) : (const void*)zero;
-            if (lane < 32) __builtin_amdgcn_global_load_lds((glb_ptr_t)src, (lds_ptr_t)(sIds + (step % RING) * 32), 4, 0, 0);
-        };
-        auto issue = [&](int step, const Cursor& c) {
-            char* base = smem + (step % STAGES) * STAGE_BYTES;
-            int tok[CPW];
-#pragma unroll
-            for (int i = 0; i < CPW; ++i) tok[i] = lds_read_i32(ids_at + ((step % RING) * 32 + tokOf[i]) * 4);
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            const char* const pb = reinterpret_cast<const char*>(p.pm) + (size_t)p.p_slot_rows * c.s * pitchP;
-            const char* const qb = reinterpret_cast<const char*>(p.qm) + (size_t)p.q_slot_rows * c.s * pitchQ;
-            const int left = c.end - c.r;
-#pragma unroll
-            for (int i = 0; i < CPW; ++i) {
-                int t = tok[i];
-                asm volatile("" : "+v"(t));
-                char* to = base + (i < R_CPW ? (wave + 4 * i) * 1024 : OPERAND_BYTES + (wave + 4 * (i - R_CPW)) * 1024);
-                const char* from = (i < R_CPW ? pb : qb) + (size_t)((Off)(unsigned)t * (i < R_CPW ? pitchP : pitchQ) + colOf[i]);
-                if (left >= KD) dma16((i < R_CPW ? pb : qb) + (size_t)((Off)(unsigned)t * (i < R_CPW ? pitchP : pitchQ) + colOf[i]), to);
-                else dma16(tokOf[i] < left ? from : zero, to);
-            }
-        };
-        if (nk > 0) {
-            // groups of CPW + 1 copies: the rows of a step, then the ids LEAD steps further on
-            Cursor ids = start, rows = start;
-            for (int st = 0; st < LEAD; ++st) { issue_ids(st, ids); ids = advance(ids); }
-            wait_vmcnt<0>();
-#pragma unroll
-            for (int st = 0; st < LEAD; ++st) {
-                if (st < nk) {
-                    issue(st, rows); rows = advance(rows);
-                    issue_ids(st + LEAD, ids); ids = advance(ids);
-                }
-            }
-            for (int kt = 0; kt < nk; ++kt) {
-                wait_groups<CPW + 1, LEAD - 1>(min(nk - 1 - kt, LEAD - 1));
-                barrier_nofence();
-                if (kt + LEAD < nk) {
-                    issue(kt + LEAD, rows); rows = advance(rows);
-                    issue_ids(kt + 2 * LEAD, ids); ids = advance(ids);
-                }
-            }
-        }
-        return;
+        return c;
+    };
+    Cursor ids = seek(Cursor{0, begin(0), end(0)});
+    for (int skip = step0; skip > 0 && ids.s < p.k;) {
+        const int here = (ids.end - ids.r + KD - 1) / KD, take = min(here, skip);
+        ids.r += take * KD;
+        skip -= take;
+        ids = seek(ids);
     }
 
-    f32x16 acc;
+    // Token ids are fetched a step before the rows they name.  Columns past the result's edge re-read the first ones of a row:
+    // what they produce is never stored.  Rows past the end of a list are zeros in both operands.
+    using Off = std::conditional_t<BIG, size_t, unsigned>;
+    using PR = Place<true, BM, KD, C::NT>;
+    using PF = Place<true, BN, KD, C::NT>;
+    int idR[C::RO], idF[C::FO];
+    Cursor rows = ids;
+    auto fetch_ids = [&]() {
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
-    const bool busy = m0 + wr * 32 < M && n0 + wf * 32 < N;
-    if (nk > 0) {
-        const unsigned lds0 = lds_addr(smem), laR = FragKS::lane_addr(lane, wr * 32), laF = FragKS::lane_addr(lane, wf * 32) + OPERAND_BYTES;
-        unsigned stage_at = lds0;
-        using Pair = Half<FragKS, FragKS>;
-        auto load = [&](Pair& h, auto half) {
-            constexpr int HALF = decltype(half)::value;
-            h.r.template read<HALF>(laR + stage_at);
-            h.f.template read<HALF>(laF + stage_at);
-        };
-        multiply_stages<Pair>(nk, busy, acc, [&](Pair& h) { load(h, std::integral_constant<int, 0>()); },
-                              [&](Pair& h) { load(h, std::integral_constant<int, 1>()); },
-                              [&]() { stage_at = stage_at + STAGE_BYTES == lds0 + STAGES * STAGE_BYTES ? lds0 : stage_at + STAGE_BYTES; });
-    }
-    const int m = m0 + wr * 32 + (lane & 31);
-    if (m >= M) return;
-
-    const bool whole = p.parts == 1;
-    float* const dst0 = (whole ? p.dw + (size_t)e * M * N : p.scratch + ((size_t)part * E + e) * M * N) + (size_t)m * N;
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        const int n = n0 + wf * 32 + 8 * g + 4 * (lane >> 5);
-        if (n >= N) continue;
-        float4 v = make_float4(acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]);
-        float4* dst = reinterpret_cast<float4*>(dst0 + n);
-        if (whole && p.accumulate) {
-            const float4 old = *dst;
-            v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
+        for (int i = 0; i < C::RO; ++i) {
+            const int r = ids.r + PR::row_of(tid, i);
+            idR[i] = ids.s < p.k && r < ids.end ? p.token_ids[(size_t)ids.s * p.T + r] : 0;
         }
-        *dst = v;
+#pragma unroll
+        for (int i = 0; i < C::FO; ++i) {
+            const int r = ids.r + PF::row_of(tid, i);
+            idF[i] = ids.s < p.k && r < ids.end ? p.token_ids[(size_t)ids.s * p.T + r] : 0;
+        }
+        rows = ids;
+        if (ids.s < p.k) { ids.r += KD; ids = seek(ids); }
+    };
+    const int mR = m0 + PR::piece_of(tid) * 8, nF = n0 + PF::piece_of(tid) * 8;
+    const unsigned colR = mR < M ? mR * 4u : 0u, colF = nF < N ? nF * 4u : 0u;
+    const unsigned secondR = mR + 4 < M ? 16u : 0u, secondF = nF + 4 < N ? 16u : 0u;
+    const Off pitchR = (Off)M * 4, pitchF = (Off)N * 4;
+    auto read4 = [](const char* base, Off off) { return *reinterpret_cast<const f32x4*>(base + (size_t)off); };
+    if (nk > 0) fetch_ids();
+    auto load = [&](int step, Octet (&r)[C::RO], Octet (&f)[C::FO]) {
+        const char* const pb = reinterpret_cast<const char*>(p.pm) + (size_t)p.p_slot_rows * rows.s * M * 4;
+        const char* const qb = reinterpret_cast<const char*>(p.qm) + (size_t)p.q_slot_rows * rows.s * N * 4;
+        const int left = rows.end - rows.r;
+        Off offR[C::RO], offF[C::FO];
+#pragma unroll
+        for (int i = 0; i < C::RO; ++i) offR[i] = (Off)(unsigned)idR[i] * pitchR + colR;
+#pragma unroll
+        for (int i = 0; i < C::FO; ++i) offF[i] = (Off)(unsigned)idF[i] * pitchF + colF;
+        if (left >= KD) {
+#pragma unroll
+            for (int i = 0; i < C::RO; ++i) { r[i].a = read4(pb, offR[i]); r[i].b = read4(pb, offR[i] + secondR); }
+#pragma unroll
+            for (int i = 0; i < C::FO; ++i) { f[i].a = read4(qb, offF[i]); f[i].b = read4(qb, offF[i] + secondF); }
+        } else {
+            const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < C::RO; ++i) {
+                r[i].a = zero; r[i].b = zero;
+                if (PR::row_of(tid, i) < left) { r[i].a = read4(pb, offR[i]); r[i].b = read4(pb, offR[i] + secondR); }
+            }
+#pragma unroll
+            for (int i = 0; i < C::FO; ++i) {
+                f[i].a = zero; f[i].b = zero;
+                if (PF::row_of(tid, i) < left) { f[i].a = read4(qb, offF[i]); f[i].b = read4(qb, offF[i] + secondF); }
+            }
+        }
+        if (step + 1 < nk) fetch_ids();
+    };
+
+    f32x16 acc[C::FB][C::RB];
+    zero_acc(acc);
+    const bool busy = m0 + wr * 32 * C::RB < M && n0 + wf * 32 * C::FB < N;
+    multiply_stages<C, true, true>(nk, busy, smem, sWhole, tid, acc, load);
+    if (!combine<C>(smem, kg, wave, lane, acc)) return;
+
+    const bool alone = p.parts == 1;
+    float* const dst0 = alone ? p.dw + (size_t)e * M * N : p.scratch + ((size_t)part * E + e) * M * N;
+#pragma unroll
+    for (int i = 0; i < C::RB; ++i) {
+        const int m = m0 + (wr * C::RB + i) * 32 + (lane & 31);
+        if (m >= M) continue;
+#pragma unroll
+        for (int j = 0; j < C::FB; ++j) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int n = n0 + (wf * C::FB + j) * 32 + 8 * g + 4 * (lane >> 5);
+                if (n >= N) continue;
+                float4 v = make_float4(acc[j][i][4 * g], acc[j][i][4 * g + 1], acc[j][i][4 * g + 2], acc[j][i][4 * g + 3]);
+                float4* dst = reinterpret_cast<float4*>(dst0 + (size_t)m * N + n);
+                if (alone && p.accumulate) {
+                    const float4 old = *dst;
+                    v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
+                }
+                *dst = v;
+            }
+        }
     }
 }
 
-template <bool IO, bool WIDE, typename S> int launch_esmm32_t(const Esmm32K& p, hipStream_t st) {
-    auto kernel = esmm32_kernel<IO, WIDE, S>;
-    constexpr int bytes = S::STAGES * STAGE_BYTES;
-    if (int rc = ensure_smem(kernel, bytes)) return rc;
-    const long tiles = (long)p.nslots * p.mt_ub * (HEXA_TILE_ROWS / BM) * p.ntn;
-    hipLaunchKernelGGL(kernel, dim3(round_up(tiles, 8)), dim3(NT), bytes, st, p);
+template <bool IO, bool BIG, typename C> int launch_esmm32_t(Esmm32K& p, hipStream_t st) {
+    p.ntn = div_up(p.N, C::BN);
+    const long tiles = (long)p.nslots * p.mt_ub * (HEXA_TILE_ROWS / C::BM) * p.ntn;
+    auto kernel = esmm32_kernel<IO, BIG, C>;
+    if (int rc = ensure_smem(kernel, C::BYTES)) return rc;
+    hipLaunchKernelGGL(kernel, dim3(round_up(tiles, 8)), dim3(C::NT), C::BYTES, st, p);
     HEXA_CHECK_LAUNCH("esmm32");
     return HEXA_OK;
 }
-
-template <bool WIDE> int launch_estmm32_t(Estmm32K& p, hipStream_t st) {
-    auto kernel = estmm32_kernel<WIDE, Deep>;
-    constexpr int bytes = Deep::STAGES * STAGE_BYTES;
-    if (int rc = ensure_smem(kernel, bytes)) return rc;
-    p.mtn = div_up(p.M, BM); p.ntn = div_up(p.N, BN);
+template <bool BIG, typename C> int launch_estmm32_t(Estmm32K& p, hipStream_t st) {
+    p.mtn = div_up(p.M, C::BM); p.ntn = div_up(p.N, C::BN);
     p.group = p.ntn;
     p.total = (long)p.E * p.parts * p.mtn * p.ntn;
-    hipLaunchKernelGGL(kernel, dim3(round_up(p.total, 8 * p.group)), dim3(NT), bytes, st, p);
+    auto kernel = estmm32_kernel<BIG, C>;
+    if (int rc = ensure_smem(kernel, C::BYTES)) return rc;
+    hipLaunchKernelGGL(kernel, dim3(round_up(p.total, 8 * p.group)), dim3(C::NT), C::BYTES, st, p);
     HEXA_CHECK_LAUNCH("estmm32");
     return HEXA_OK;
 }
-
 // whether byte offsets into rows x cols floats (and a stage beyond) need more than 32 bits
 bool too_large(size_t rows, size_t cols) { return (rows + 64) * cols * 4 >= ((size_t)1 << 32); }
 
@@ -525,7 +590,6 @@ int launch_esmm32(const EsmmArgs& a, hipStream_t st) {
     p.out = (float*)a.out; p.out_act = (float*)a.out_act;
     p.token_ids = a.r.token_ids; p.tile_info = a.r.tile_info; p.tile_count = a.r.tile_count;
     p.T = a.r.T; p.K = a.in_dim; p.N = a.out_dim; p.mt_ub = a.r.mt_ub;
-    p.ntn = div_up(a.out_dim, 64);
     p.x_slot_rows = a.x_per_slot ? a.r.T : 0;
     p.out_slot_rows = a.out_per_slot ? a.r.T : 0;
     p.act = a.act;
@@ -538,28 +602,42 @@ int launch_esmm32(const EsmmArgs& a, hipStream_t st) {
         p.slot_begin = s;
         p.nslots = std::min(per_launch, a.r.k - s);
         p.accumulate = (a.accumulate || (sum && !p.ws && s > 0)) ? 1 : 0;
-        if ((long)p.mt_ub * p.ntn == 0) continue;
+        if (p.mt_ub == 0) continue;
         const bool io = a.w_layout == HEXA_W_IN_OUT;
-        const bool wide = too_large((size_t)a.r.T * (a.x_per_slot ? a.r.k : 1), a.in_dim) || too_large(a.in_dim, a.out_dim);
-        // With more tiles than three workgroups per CU take at once, four with two stages each hide more of each other's
-        // starts and ends (fc2-type launch: 199 against 219 us; equal for fc1); below that a tile is on its own and a
-        // third stage is worth 2 us of 18.
-        const bool many = (long)p.nslots * a.r.T / BM * p.ntn > 768;
-        const int rc = wide   ? (io ? launch_esmm32_t<true, true, Deep>(p, st) : launch_esmm32_t<false, true, Deep>(p, st))
-                       : many ? (io ? launch_esmm32_t<true, false, Many>(p, st) : launch_esmm32_t<false, false, Many>(p, st))
-                              : (io ? launch_esmm32_t<true, false, Deep>(p, st) : launch_esmm32_t<false, false, Deep>(p, st));
+        const bool big = too_large((size_t)a.r.T * (a.x_per_slot ? a.r.k : 1), a.in_dim) || too_large(a.in_dim, a.out_dim);
+        // 128 x 128 tiles where they come to one for most CUs and the lists fill them: 3000 rows, 1024 -> 2048, 4 experts 101
+        // against 125 us of 64 x 64 tiles, 23 x 8 tiles of its fc2 124 against 139, 8192 rows, 2048 -> 512 (64 x 4) 160 both; 64
+        // rows an expert 49 against 44, 4000 rows, 2048 -> 512 (31 x 4 tiles) 117 against 101
+        const bool wide = (long)p.nslots * a.r.T / 128 * div_up(a.out_dim, 128) >= 180 && a.r.T >= 100 * a.r.E;
+        auto go = [&](auto bg) {
+            constexpr bool BIG = decltype(bg)::value;
+            return wide ? (io ? launch_esmm32_t<true, BIG, Wide>(p, st) : launch_esmm32_t<false, BIG, Wide>(p, st))
+                        : (io ? launch_esmm32_t<true, BIG, Deep>(p, st) : launch_esmm32_t<false, BIG, Deep>(p, st));
+        };
+        const int rc = big ? go(std::true_type()) : go(std::false_type());
         if (rc) return rc;
     }
     if (p.ws) return launch_sum_slots(a.out, a.slot_ws, a.r, a.out_dim, a.accumulate, HEXA_F32, st, a.sum_extra);
     return HEXA_OK;
 }
 
-// Parts every expert's token list is cut into: with fewer than two 64 x 64 tiles per CU a launch is the walk over one
-// list, so lists of 256 and more entries are cut until there are four workgroups per CU (or 128 entries a part).
+// Tile and number of parts that every expert's token list is cut into.  Where 128 x 128 tiles come to two and more per CU they
+// take whole lists.  With fewer, a launch is the walk over its longest list: such tiles cut lists of a thousand entries and
+// more into parts, and below that 64 x 64 tiles until there are six workgroups per CU (or 128 entries a part).  Measured with
+// one part of 64 x 64 tiles against this: 18432 entries, 8 experts, 1536 x 384 195 -> 178 us, 8192, 4, 2048 x 512 156 -> 133,
+// 5000, 12, 800 x 200 72 -> 45; uncut 128 x 128 against 64 x 64 tiles at 12000, 32, 3072 x 768 402 against 537.
+static bool estmm32_wide(int T, int k, int E, int m_dim, int n_dim, int* parts) {
+    const long t128 = (long)E * div_up(m_dim, 128) * div_up(n_dim, 128), t64 = (long)E * div_up(m_dim, 64) * div_up(n_dim, 64);
+    const long avg = (long)T * k / std::max(1, E);
+    const bool cut = t128 < 512 && avg >= 256, wide = t128 >= 512 || (t128 >= 200 && avg >= 1024);
+    const long want = wide ? std::min<long>((768 + t128 - 1) / t128, avg / 256) : std::min<long>((1536 + t64 - 1) / t64, avg / 128);
+    *parts = cut ? (int)std::max<long>(1, std::min<long>(8, want)) : 1;
+    return wide;
+}
 int estmm32_parts(int T, int k, int E, int m_dim, int n_dim) {
-    const long tiles = (long)E * div_up(m_dim, 64) * div_up(n_dim, 64), avg = (long)T * k / std::max(1, E);
-    if (tiles >= 512 || avg < 256) return 1;
-    return (int)std::max<long>(1, std::min<long>(8, std::min<long>((1024 + tiles - 1) / tiles, avg / 128)));
+    int parts;
+    estmm32_wide(T, k, E, m_dim, n_dim, &parts);
+    return parts;
 }
 
 int launch_estmm32(const EstmmArgs& a, hipStream_t st) {
@@ -572,9 +650,13 @@ int launch_estmm32(const EstmmArgs& a, hipStream_t st) {
     p.p_slot_rows = a.p_per_slot ? a.r.T : 0;
     p.q_slot_rows = a.q_per_slot ? a.r.T : 0;
     p.accumulate = a.accumulate;
-    p.parts = a.scratch ? std::max(1, std::min(estmm32_parts(p.T, p.k, p.E, p.M, p.N), a.max_slots / p.E)) : 1;
-    const bool wide = too_large((size_t)p.T * (a.p_per_slot ? p.k : 1), p.M) || too_large((size_t)p.T * (a.q_per_slot ? p.k : 1), p.N);
-    if (int rc = wide ? launch_estmm32_t<true>(p, st) : launch_estmm32_t<false>(p, st)) return rc;
+    int parts;
+    const bool wide = estmm32_wide(p.T, p.k, p.E, p.M, p.N, &parts) && !(parts > 1 && !a.scratch);
+    p.parts = a.scratch ? std::max(1, std::min(parts, a.max_slots / p.E)) : 1;
+    const bool big = too_large((size_t)p.T * (a.p_per_slot ? p.k : 1), p.M) || too_large((size_t)p.T * (a.q_per_slot ? p.k : 1), p.N);
+    const int rc = big ? (wide ? launch_estmm32_t<true, Wide>(p, st) : launch_estmm32_t<true, Deep>(p, st))
+                       : (wide ? launch_estmm32_t<false, Wide>(p, st) : launch_estmm32_t<false, Deep>(p, st));
+    if (rc) return rc;
     return p.parts > 1 ? launch_fold(a.dw, a.scratch, (long)p.E * p.M * p.N, p.parts, HEXA_F32, a.accumulate, st) : HEXA_OK;
 }
 

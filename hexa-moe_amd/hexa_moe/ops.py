@@ -224,9 +224,15 @@ def esmm(x, w, bias, route, m2s, w_layout, out=None, out_dtype=None, accumulate=
 
 
 def estmm32_slots(T, k, E, out_dim, in_dim):
-    """Scratch slots ([out_dim, in_dim] floats each) an fp32 estmm call can use: results with few 64 x 64 tiles cut
-    every expert's list into up to 8 parts."""
-    return 8 * E if T * k >= 256 * E and E * -(-out_dim // 64) * -(-in_dim // 64) < 512 else 0
+    """Scratch slots ([out_dim, in_dim] floats each) an fp32 estmm call can use: results with few tiles cut every
+    expert's list into up to 8 parts (estmm32_wide of gemm32.hip)."""
+    t128, t64 = (E * -(-out_dim // n) * -(-in_dim // n) for n in (128, 64))
+    avg = T * k // E
+    if t128 >= 512 or avg < 256:
+        return 0
+    parts = min(-(-768 // t128), avg // 256) if t128 >= 200 and avg >= 1024 else min(-(-1536 // t64), avg // 128)
+    parts = max(1, min(8, parts))
+    return parts * E if parts > 1 else 0
 
 
 def estmm(dy, x, route, dy_per_slot, x_per_slot, out=None, out_dtype=torch.float32, accumulate=False):
