@@ -54,7 +54,6 @@ using CfgP = Cfg<PIPE_WR, 2, PIPE_RB, 2, 3, 3, 64>;   // 128 x 128: 4 multiply w
 // - LUT_M_LO) + sign: the two 16-bit values of a 32-bit word are turned into two table addresses with packed 16-bit
 // arithmetic (four vector instructions per element instead of nine).  A piece with a value outside that range
 // (zeros, |x| >= 8, NaN) takes the polynomial: one wavefront-wide branch per 16-byte piece.
-constexpr unsigned LUT_M_HI = 0x4100;
 template <typename TC, int ACT, bool COLSUM> constexpr unsigned pipe_lut_lo() {
     // GELU' with column sums: fp32 entries next to the column-sum area leave room for magnitudes from 2^-14 only
     return ACT == HEXA_ACT_GELU_BWD && COLSUM ? 0x3880u : 0x3700u;
@@ -63,35 +62,6 @@ template <typename TC, int ACT, bool COLSUM> constexpr int pipe_lut_bytes() {
     constexpr int r = (int)(LUT_M_HI - pipe_lut_lo<TC, ACT, COLSUM>());
     return !std::is_same<TC, __bf16>::value ? 0 : ACT == HEXA_ACT_GELU ? 2 * r * 2 : ACT == HEXA_ACT_GELU_BWD ? 2 * r * 4 : 0;
 }
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ u16x2 as_u16x2(unsigned w) {
-    union { unsigned u; u16x2 v; } c;
-    c.u = w;
-    return c.v;
-}
-__device__ __forceinline__ unsigned as_u32(u16x2 v) {
-    union { unsigned u; u16x2 v; } c;
-    c.v = v;
-    return c.u;
-}
-// The table positions (as byte offsets, entries of 1 << SH bytes) of the two 16-bit values of w, packed in one word;
-// `far` collects the largest distance from the table's first magnitude (a magnitude below it wraps to a huge
-// one), so far >= the table's length says some value is outside.
-template <unsigned LO, int SH> __device__ __forceinline__ unsigned lut_offsets(unsigned w, u16x2& far) {
-    const u16x2 lo2 = {(unsigned short)LO, (unsigned short)LO};
-    const u16x2 u = as_u16x2(w & 0x7fff7fffu) - lo2;
-    far = __builtin_elementwise_max(far, u);
-    const u16x2 sh = {(unsigned short)(SH + 1), (unsigned short)(SH + 1)};
-    return as_u32(u << sh) | ((w >> (15 - SH)) & ((1u << SH) * 0x00010001u));
-}
-// (the 16-bit LDS loads that target one half of a register clear the other half on this chip, so two entries
-// are read into two registers and joined with one shift-or)
-template <int OFF> __device__ __forceinline__ unsigned lds_read_u16_async(unsigned addr) {
-    unsigned r;
-    asm volatile("ds_read_u16 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF));
-    return r;
-}
-
 struct PipeK {
     EsmmK e;
     int wg_per_xcd;       // workgroups per XCD (grid = 8 * wg_per_xcd)

@@ -127,11 +127,15 @@ bool esmm16_dma_colsum_supported(const EsmmArgs& a);
 bool esmm16_pipe_supported(const EsmmArgs& a);
 bool esmm16_wide_supported(const EsmmArgs& a);
 int launch_esmm16_pipe(const EsmmArgs& a, hipStream_t st);
+bool esmm16_big_supported(const EsmmArgs& a);
+int launch_esmm16_big(const EsmmArgs& a, hipStream_t st);
+bool estmm16_big_supported(const EstmmArgs& a);
+int launch_estmm16_big(const EstmmArgs& a, hipStream_t st);
 bool ffn16_fused_supported(int T, int k, int d_in, int hidden, int d_out, int act_dt, int w_dt, int b1_dt, int b2_dt);
 int launch_ffn16_fused(void* y1, void* y2, void* y, const void* x, const void* w1, const void* b1, const void* w2,
                        const void* b2, const RouteView& r, int d_in, int hidden, int d_out, int act_dt, int b1_dt,
                        int b2_dt, void* slot_ws, hipStream_t st);
-int launch_colsum_fold(const EsmmArgs& a, int mt_ub, int tile_rows, int ntn, int bn, hipStream_t st);
+int launch_colsum_fold(const EsmmArgs& a, int mt_ub, int tile_rows, int ntn, int bn, hipStream_t st, bool merged = false);
 int estmm_plan_cap_for(const RouteView& r, int out_dim, int in_dim);   // rows above which an expert's list is cut
 int launch_estmm_plan(int32_t* plan, const RouteView& r, int max_slots, int cap, hipStream_t st);
 int launch_estmm_fixup(const EstmmArgs& a, hipStream_t st);

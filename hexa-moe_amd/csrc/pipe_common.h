@@ -158,5 +158,36 @@ __device__ __forceinline__ void mma_stage_ahead(unsigned tileR, unsigned tileF, 
 template <typename TC> __device__ __forceinline__ float lo16(unsigned w) { return from_bits16<TC>(w & 0xffff); }
 template <typename TC> __device__ __forceinline__ float hi16(unsigned w) { return from_bits16<TC>(w >> 16); }
 
+// Tables of GELU and GELU' over the bf16 values from a lowest magnitude up to 8 (see gemm16_pipe.hip)
+constexpr unsigned LUT_M_HI = 0x4100;
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u16x2 as_u16x2(unsigned w) {
+    union { unsigned u; u16x2 v; } c;
+    c.u = w;
+    return c.v;
+}
+__device__ __forceinline__ unsigned as_u32(u16x2 v) {
+    union { unsigned u; u16x2 v; } c;
+    c.v = v;
+    return c.u;
+}
+// The table positions (as byte offsets, entries of 1 << SH bytes) of the two 16-bit values of w, packed in one word;
+// `far` collects the largest distance from the table's first magnitude (a magnitude below it wraps to a huge
+// one), so far >= the table's length says some value is outside.
+template <unsigned LO, int SH> __device__ __forceinline__ unsigned lut_offsets(unsigned w, u16x2& far) {
+    const u16x2 lo2 = {(unsigned short)LO, (unsigned short)LO};
+    const u16x2 u = as_u16x2(w & 0x7fff7fffu) - lo2;
+    far = __builtin_elementwise_max(far, u);
+    const u16x2 sh = {(unsigned short)(SH + 1), (unsigned short)(SH + 1)};
+    return as_u32(u << sh) | ((w >> (15 - SH)) & ((1u << SH) * 0x00010001u));
+}
+// (the 16-bit LDS loads that target one half of a register clear the other half on this chip, so two entries
+// are read into two registers and joined with one shift-or)
+template <int OFF> __device__ __forceinline__ unsigned lds_read_u16_async(unsigned addr) {
+    unsigned r;
+    asm volatile("ds_read_u16 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF));
+    return r;
+}
+
 }  // namespace
 }  // namespace hexa

@@ -559,24 +559,29 @@ __device__ __forceinline__ void colsum_fold_body(const ColsumFoldK& p, int block
     __shared__ int sFirst[8], sCount[8];        // per slot: first tile of expert e, its number of tiles
     __shared__ int red[256];
     const int bx = block % p.gx, e = block / p.gx, tid = threadIdx.x;
-    for (int s = 0; s < p.nslots; ++s) {
-        const int32_t* off = p.offsets + (size_t)s * (p.E + 1);
+    const int runs = p.merged ? 1 : p.nslots;
+    for (int s = 0; s < runs; ++s) {
+        auto tiles_of = [&](int x) {
+            int n = 0;
+            for (int q = s; q < (p.merged ? p.nslots : s + 1); ++q) n += p.offsets[(size_t)q * (p.E + 1) + x + 1] - p.offsets[(size_t)q * (p.E + 1) + x];
+            return (n + p.tile_rows - 1) / p.tile_rows;
+        };
         int before = 0;
-        for (int x = tid; x < e; x += 256) before += (off[x + 1] - off[x] + p.tile_rows - 1) / p.tile_rows;
+        for (int x = tid; x < e; x += 256) before += tiles_of(x);
         red[tid] = before;
         __syncthreads();
         for (int w = 128; w > 0; w >>= 1) {
             if (tid < w) red[tid] += red[tid + w];
             __syncthreads();
         }
-        if (tid == 0) { sFirst[s] = red[0]; sCount[s] = (off[e + 1] - off[e] + p.tile_rows - 1) / p.tile_rows; }
+        if (tid == 0) { sFirst[s] = red[0]; sCount[s] = tiles_of(e); }
         __syncthreads();
     }
     const int n = bx * 256 + tid;
     if (n >= p.N) return;
     const int nt = n / p.bn, nl = n - nt * p.bn;
     float sum = 0.f;
-    for (int s = 0; s < p.nslots; ++s) {
+    for (int s = 0; s < runs; ++s) {
         const int first = sFirst[s], last = min(first + sCount[s], p.mt_ub);
         // eight loads in flight per trip (a busy expert has a dozen tiles; one load per trip would pay the
         // memory latency a dozen times); the additions stay in tile order

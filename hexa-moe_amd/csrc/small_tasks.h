@@ -26,6 +26,7 @@ struct FixupK { void* dw; const int* plan; const float* scratch; int E; long mn;
 struct ColsumFoldK {
     void* db; const float* colsum; const int32_t* offsets;
     int E, mt_ub, tile_rows, ntn, bn, N, nslots, db_dt, accumulate, gx;
+    int merged;      // tiles run over an expert's lists of all slots, one behind the other
 };
 struct SumSlotsK {
     void* out; const void* ws; int64_t n; int nws; const void* extra; int blocks;
