@@ -68,10 +68,10 @@ template <int OFF = 0> __device__ __forceinline__ int lds_read_u8(unsigned addr)
     return r;
 }
 __device__ __forceinline__ void lds_write_u8(unsigned addr, int v) { asm volatile("ds_write_b8 %0, %1" ::"v"(addr), "v"(v) : "memory"); }
-// 16-byte store to an address of each lane's own
+// 16-byte store to an address of each lane's own (s_nop: see global_store128 of pipe_common.h)
 __device__ __forceinline__ void global_store128(char* at, u32x4 v, bool streaming) {
-    if (streaming) asm volatile("global_store_dwordx4 %0, %1, off nt" ::"v"(at), "v"(v) : "memory");
-    else asm volatile("global_store_dwordx4 %0, %1, off" ::"v"(at), "v"(v) : "memory");
+    if (streaming) asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 1" ::"v"(at), "v"(v) : "memory");
+    else asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" ::"v"(at), "v"(v) : "memory");
 }
 
 // a copy's wait: at most N (and EXTRA stores, where `lax`) younger operations may be outstanding
