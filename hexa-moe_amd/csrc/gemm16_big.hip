@@ -1,5 +1,5 @@
-// ESMM and ESTMM for bf16 / fp16 on gfx950 with 256 x 256 tiles, for products large enough to fill the chip with them (the
-// rules are use_big's in gemm16_dma.hip; the sums are those of the 128 x 128 kernels, in the same order).
+// ESMM for bf16 / fp16 on gfx950 with 256 x 256 tiles, for products large enough to fill the chip with them (the rule is
+// use_big in gemm16_dma.hip; the sums are those of the 128 x 128 kernels, in the same order).
 //
 // What bounds the 128 x 128 kernels there is the way of the operands, not the matrix pipes: a 128 x 128 x 64 stage reads
 // 32 KB from L2 and 64 KB from LDS for 2.1 MFLOP, and the CU's copy path (64 B a clock) is busy 64 to 72 % of the time.  A 256 x
@@ -13,9 +13,9 @@
 //
 // Measured: 8192 x 8192 x 8192 in bf16 1322 TFLOP/s in this schedule (1113 by the vendor's library on the same card); a
 // stage takes 1.4 to 1.6 us per round of 256 tiles.  32768 rows, top-2 of 64 experts with a skewed load, 1024 -> 4096: plain 888 us
-// before, 615 now; + GELU 1028, 740; fc2 787, 640; times GELU' with column sums 1010, 780; ESTMM 885 and 920 before, 735
-// and 730 now.  What is left there is the results' way out (537 MB each, 100 us and more of them) with nothing to multiply
-// in the meantime: a tile's accumulators hold half of the registers, so the next tile cannot begin before they are stored.
+// before, 615 now; + GELU 1028, 740; fc2 787, 640; times GELU' with column sums 1010, 780.  What is left there is the
+// results' way out (537 MB each, 100 us and more of them) with nothing to multiply in the meantime: a tile's accumulators
+// hold half of the registers, so the next tile cannot begin before they are stored.
 #include <algorithm>
 #include <type_traits>
 #include <utility>
@@ -581,296 +581,6 @@ __global__ __launch_bounds__(512, 2) void esmm16_big_kernel(BigK p) {
     }
 }
 
-// ------------------------------------------------------------------------------------------------------------------------
-// ESTMM: dw[e][m][n] = sum over the expert's (slot, token) list of P[row][m] * Q[row][n], one 256 x 256 block per workgroup
-// (not persistent: the units differ in length, and the dispatcher hands out the longest first).  Both operands are read
-// across their rows (transposing LDS reads); the rows are gathered by token id, whose 64 per step are fetched four steps
-// ahead by the wavefronts in turn.  Blocks of one expert are walked with all column blocks (up to 8) of a row block on one XCD.
-// ------------------------------------------------------------------------------------------------------------------------
-struct BigEstmmK {
-    const void* pm; const void* qm; void* dw;
-    const int32_t* token_ids; const int32_t* offsets;
-    const int* plan; float* scratch;          // units of the balanced plan (small_bodies.h); partial results of cut lists
-    int T, k, E, M, N, mtn, ntn, p_slot_rows, q_slot_rows, accumulate, stream_dw, group;
-    long total;
-};
-
-template <typename TC, bool OUT32>
-__global__ __launch_bounds__(512, 2) void estmm16_big_kernel(BigEstmmK p) {
-    using V = typename Mfma<TC>::V;
-    constexpr int BM = 256, BN = 256, BK = 64, HALF = BigHalf::HALF, STAGE = BigHalf::STAGE, IDS = 4;   // stages whose ids are in LDS
-    extern __shared__ __attribute__((aligned(1024))) char smem[];
-    const unsigned lds0 = lds_addr(smem);
-    int* const sIds = reinterpret_cast<int*>(smem + 2 * STAGE);
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave >> 2, wf = wave & 3;
-    const int M = p.M, N = p.N, T = p.T;
-
-    // the item: a unit (an expert's list or a part of it, heaviest expert first) and a block of its result
-    const long logical = logical_tile(blockIdx.x, p.group);
-    if (logical >= p.total) return;
-    const int per_e = p.mtn * p.ntn;
-    const int rank = (int)(logical / per_e), rem = (int)(logical - (long)rank * per_e);
-    const int m0 = (rem / p.ntn) * BM, n0 = (rem % p.ntn) * BN;
-    // (one round of loads for the plan, one for the lists' ends, one for the first token ids: each is a trip to memory in which
-    // nothing else runs)
-    int* const sUnit = sIds;                    // expert, part, parts, scratch slot, units; then the ends of its lists
-    if (tid == 0) sUnit[4] = p.plan[4 * p.E];
-    for (int r = tid; r < p.E; r += 512) {
-        const int u0 = p.plan[2 * p.E + r], n = p.plan[p.E + r], x = p.plan[r], at = p.plan[3 * p.E + r];
-        if (rank >= u0 && rank < u0 + n) {
-            sUnit[0] = x; sUnit[1] = rank - u0; sUnit[2] = n; sUnit[3] = at;
-            for (int s = 0; s < p.k; ++s) {
-                sUnit[8 + 2 * s] = p.offsets[(size_t)s * (p.E + 1) + x];
-                sUnit[9 + 2 * s] = p.offsets[(size_t)s * (p.E + 1) + x + 1];
-            }
-        }
-    }
-    __syncthreads();
-    if (rank >= sUnit[4]) return;
-    const int e = __builtin_amdgcn_readfirstlane(sUnit[0]), part = __builtin_amdgcn_readfirstlane(sUnit[1]);
-    const int nparts = __builtin_amdgcn_readfirstlane(sUnit[2]), slot = __builtin_amdgcn_readfirstlane(sUnit[3]);
-    struct Cursor { int s, r, end; };           // position in the list of slot s
-    auto walk = [&](auto begin, auto end, Cursor c) {
-        while (c.s < p.k && c.r >= c.end) {
-            ++c.s;
-            if (c.s < p.k) { c.r = begin(c.s); c.end = end(c.s); }
-        }
-        return c;
-    };
-    // its steps of 64 list entries, slot after slot (the last step of a slot's list may be partial)
-    int nk = 0;
-    Cursor rows{0, 0, 0};
-    {
-        auto begin = [&](int s) { return __builtin_amdgcn_readfirstlane(sUnit[8 + 2 * s]); };
-        auto end = [&](int s) { return __builtin_amdgcn_readfirstlane(sUnit[9 + 2 * s]); };
-        int all_steps = 0;
-        for (int s = 0; s < p.k; ++s) all_steps += (end(s) - begin(s) + BK - 1) / BK;
-        const int step0 = (int)((long)all_steps * part / nparts);
-        nk = (int)((long)all_steps * (part + 1) / nparts) - step0;
-        rows = walk(begin, end, Cursor{0, begin(0), end(0)});
-        for (int skip = step0; skip > 0 && rows.s < p.k;) {
-            const int here = (rows.end - rows.r + BK - 1) / BK, take = min(here, skip);
-            rows.r += take * BK;
-            skip -= take;
-            rows = walk(begin, end, rows);
-        }
-    }
-    __syncthreads();
-    auto advance = [&](Cursor c) {
-        if (c.s < p.k) {
-            c.r += BK;
-            c = walk([&](int s) { return p.offsets[(size_t)s * (p.E + 1) + e]; }, [&](int s) { return p.offsets[(size_t)s * (p.E + 1) + e + 1]; }, c);
-        }
-        return c;
-    };
-    if (nk == 0 && p.accumulate && slot < 0) return;
-    // ---- copies -------------------------------------------------------------------------------------------------------------
-    Cursor ids = rows;
-    const char* const zero = reinterpret_cast<const char*>(g_zero_block);
-    // the 64 token ids of a step, by one wavefront
-    auto id_of = [&](const Cursor& c) {
-        const int r = c.r + lane;
-        return c.s < p.k && r < c.end ? (const void*)(p.token_ids + (size_t)c.s * T + r) : (const void*)zero;
-    };
-    for (int st = 0; st < IDS; ++st) {
-        if (wave == st) sIds[st * 64 + lane] = *reinterpret_cast<const int*>(id_of(ids));
-        ids = advance(ids);
-    }
-    __syncthreads();
-    int kk, ch;
-    ks_lane<128>(wave, lane, kk, ch);           // this lane's copies fetch entries kk and kk + 32 of a step, column piece ch of a half
-    unsigned colA[2], colB[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int m = m0 + h * 128 + ch * 8, n = n0 + (2 * (ch >> 2) + h) * 32 + (ch & 3) * 8;
-        colA[h] = m < M ? (unsigned)m * 2u : 0u;      // (past the result's edge: the row's first bytes; what they produce is not stored)
-        colB[h] = n < N ? (unsigned)n * 2u : 0u;
-    }
-    const unsigned pitchA = (unsigned)M * 2u, pitchB = (unsigned)N * 2u;
-    int cs = 0;                                 // the step the copies are for
-    unsigned cbuf = 0, offA[2] = {0, 0}, offB[2] = {0, 0};
-    const char* pb = nullptr; const char* qb = nullptr;
-    int left = 0;
-    auto set_rows = [&]() {
-        int t[2];
-        t[0] = lds_read_i32(lds0 + 2 * STAGE + ((cs & (IDS - 1)) * 64 + kk) * 4);
-        t[1] = lds_read_i32(lds0 + 2 * STAGE + ((cs & (IDS - 1)) * 64 + kk + 32) * 4);
-        lds_wait();
-        pb = reinterpret_cast<const char*>(p.pm) + (size_t)p.p_slot_rows * rows.s * pitchA;
-        qb = reinterpret_cast<const char*>(p.qm) + (size_t)p.q_slot_rows * rows.s * pitchB;
-        left = rows.end - rows.r;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            asm volatile("" : "+v"(t[j]));
-            offA[j] = __umul24((unsigned)t[j], pitchA);
-            offB[j] = __umul24((unsigned)t[j], pitchB);
-        }
-        rows = advance(rows);
-    };
-    auto issue = [&](int half, const char* base, const unsigned (&off)[2], unsigned col) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            char* to = smem + cbuf + half * HALF + (wave + 8 * j) * 1024;
-            if (left >= BK) dma16(base + (size_t)(off[j] + col), to);
-            else dma16(kk + 32 * j < left ? base + (size_t)(off[j] + col) : zero, to);     // the last step of a list
-        }
-    };
-    auto first_part = [&]() {                   // B0, A0, B1 of the next step
-        set_rows();
-        issue(2, qb, offB, colB[0]); issue(0, pb, offA, colA[0]); issue(3, qb, offB, colB[1]);
-    };
-    auto second_part = [&]() {
-        issue(1, pb, offA, colA[1]);
-        cbuf ^= STAGE;
-        ++cs;
-    };
-
-    // ---- fragments ------------------------------------------------------------------------------------------------------------
-    unsigned sa[2], sb;
-    {
-        const int grp = lane >> 4, sl = lane & 15, k = (grp >> 1) * 8 + (sl >> 2);
-        auto at = [&](int col) { return lds0 + k * 256 + (((col >> 3) ^ ((k & 3) << 2)) << 4) + (col & 7) * 2; };
-        const int c = (grp & 1) * 16 + (sl & 3) * 4;
-        sa[0] = at(wr * 64 + c); sa[1] = at(wr * 64 + 32 + c); sb = 2 * HALF + at(wf * 32 + c);
-    }
-    unsigned rbuf = 0;
-    union Frag { V v; u32x4 q; s16x4 h[2]; };
-    Frag a[2][4], b0[4], b1[4];
-    auto read = [&](auto oc, unsigned at, Frag (&f)[4]) {
-        static_for<4>([&](auto kc) {
-            constexpr int ks = decltype(kc)::value, OFF = decltype(oc)::value + ks * 4096;
-            Frag& g = f[ks];
-            const unsigned addr = at;
-            asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(g.h[0]) : "v"(addr), "n"(OFF));
-            asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(g.h[1]) : "v"(addr), "n"(OFF + 1024));
-        });
-    };
-    auto pin = [&](Frag (&f)[4]) {
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) asm volatile("" : "+v"(f[ks].q));
-    };
-    f32x16 acc[2][2][2];
-#pragma unroll
-    for (int x = 0; x < 8; ++x)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[x >> 2][(x >> 1) & 1][x & 1][v] = 0.f;
-    auto mma = [&](auto hac, auto hbc, Frag (&b)[4]) {
-        constexpr int ha = decltype(hac)::value, hb = decltype(hbc)::value;
-        __builtin_amdgcn_sched_barrier(0);
-        if (m0 + ha * 128 + wr * 64 >= M || n0 + (2 * wf + hb) * 32 >= N) return;      // nothing of this block is stored
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-            for (int i = 0; i < 2; ++i) acc[ha][hb][i] = Mfma<TC>::run(b[ks].v, a[i][ks].v, acc[ha][hb][i]);
-        __builtin_amdgcn_s_setprio(0);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, 1>;
-    using AT_A1 = std::integral_constant<int, HALF>;
-
-    if (nk > 0) {
-        first_part(); second_part();
-        if (nk > 1) { first_part(); wait_vmcnt<8>(); }
-        else wait_vmcnt<0>();
-        barrier_nofence();
-        if (wr == 1) barrier_nofence();        // the second group runs half a step behind the first
-        for (int kt = 0; kt < nk; ++kt) {
-            read(I0(), sa[0] + rbuf, a[0]);
-            read(I0(), sa[1] + rbuf, a[1]);
-            read(I0(), sb + rbuf, b0);
-            read(AT_A1(), sb + rbuf, b1);
-            const bool one = kt + 1 < nk, two = kt + 2 < nk;
-            if (one) { second_part(); wait_vmcnt<8>(); }
-            else wait_vmcnt<0>();
-            lds_wait();
-            pin(a[0]); pin(a[1]); pin(b0); pin(b1);
-            barrier_nofence();
-            mma(I0(), I0(), b0);
-            mma(I0(), I1(), b1);
-            barrier_nofence();
-            read(AT_A1(), sa[0] + rbuf, a[0]);
-            read(AT_A1(), sa[1] + rbuf, a[1]);
-            if (two) {
-                first_part();
-                // (the ids of this step, which make room, were last read a step ago; these are needed in two)
-                if (wave == 0 && kt + IDS < nk) __builtin_amdgcn_global_load_lds((glb_ptr_t)id_of(ids), (lds_ptr_t)(sIds + (kt & (IDS - 1)) * 64), 4, 0, 0);
-                ids = advance(ids);
-                wait_vmcnt<8>();
-            } else {
-                wait_vmcnt<0>();
-            }
-            lds_wait();
-            pin(a[0]); pin(a[1]);
-            barrier_nofence();
-            mma(I1(), I1(), b1);
-            mma(I1(), I0(), b0);
-            barrier_nofence();
-            rbuf ^= STAGE;
-        }
-        if (wr == 0) barrier_nofence();
-    }
-    barrier_nofence();
-
-    // ---- result: a wavefront's 128 x 64 values, 32 rows at a time through its own 8 KB of the stages ------------------------------
-    constexpr int PITCH = 64 * 4 + 16;
-    char* const mine = smem + wave * 32 * PITCH;
-    typedef __attribute__((ext_vector_type(4))) float f4;
-    typedef __attribute__((ext_vector_type(2))) unsigned u2;
-    const bool accumulate = p.accumulate != 0;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        const int row0 = m0 + (b >> 1) * 128 + wr * 64 + (b & 1) * 32;
-        if (row0 >= M) continue;
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const f32x16& v = acc[b >> 1][u >> 2][b & 1];
-            const int g = u & 3;
-            *reinterpret_cast<float4*>(mine + (lane & 31) * PITCH + ((u >> 2) * 32 + 8 * g + 4 * (lane >> 5)) * 4) =
-                make_float4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const int m = row0 + q * 4 + (lane >> 4), n = n0 + wf * 64 + (lane & 15) * 4;
-            float4 v = *reinterpret_cast<const float4*>(mine + (q * 4 + (lane >> 4)) * PITCH + (lane & 15) * 16);
-            if (m >= M || n >= N) continue;
-            if (slot >= 0) {   // one part of a busy expert: fp32 partial result into its scratch slot
-                *reinterpret_cast<float4*>(p.scratch + ((size_t)(slot + part) * M + m) * N + n) = v;
-                continue;
-            }
-            const size_t off = ((size_t)e * M + m) * N + n;
-            if (OUT32) {
-                float4* dst = reinterpret_cast<float4*>(reinterpret_cast<float*>(p.dw) + off);
-                if (accumulate) { const float4 old = *dst; v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w; }
-                if (p.stream_dw) { const f4 w4 = {v.x, v.y, v.z, v.w}; __builtin_nontemporal_store(w4, reinterpret_cast<f4*>(dst)); }
-                else *dst = v;
-            } else {
-                uint2* dst = reinterpret_cast<uint2*>(reinterpret_cast<unsigned short*>(p.dw) + off);
-                if (accumulate) {
-                    const uint2 old = *dst;
-                    v.x += lo16<TC>(old.x); v.y += hi16<TC>(old.x); v.z += lo16<TC>(old.y); v.w += hi16<TC>(old.y);
-                }
-                const uint2 pk = pack4<TC>(v.x, v.y, v.z, v.w);
-                if (p.stream_dw) { const u2 w2 = {pk.x, pk.y}; __builtin_nontemporal_store(w2, reinterpret_cast<u2*>(dst)); }
-                else *dst = pk;
-            }
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    }
-}
-
-template <typename TC, bool OUT32> int launch_estmm_big_k(const BigEstmmK& p, hipStream_t st) {
-    auto kernel = estmm16_big_kernel<TC, OUT32>;
-    constexpr int bytes = 2 * BigHalf::STAGE + 1024;
-    if (int rc = ensure_smem(kernel, bytes)) return rc;
-    hipLaunchKernelGGL(kernel, dim3(round_up(p.total, 8 * p.group)), dim3(512), bytes, st, p);
-    HEXA_CHECK_LAUNCH("estmm16_big");
-    return HEXA_OK;
-}
-
 template <typename TC, bool IO, int ACT, bool COLSUM, bool TAIL>
 int launch_big_k(BigK& pk, int grid, hipStream_t st) {
     auto kernel = esmm16_big_kernel<TC, IO, ACT, COLSUM, TAIL>;
@@ -946,31 +656,6 @@ int launch_esmm16_big(const EsmmArgs& a, hipStream_t st) {
     if (pk.ws) return launch_sum_slots(a.out, a.slot_ws, a.r, a.out_dim, a.accumulate, a.out_dt, st, a.sum_extra);
     if (a.colsum) return launch_colsum_fold(a, (int)(total_ub / pk.ntn), HEXA_TILE_ROWS_L, pk.ntn, 256, st, true);
     return HEXA_OK;
-}
-
-bool estmm16_big_supported(const EstmmArgs& a) {
-    return a.plan && a.scratch && a.max_slots >= 2 && a.m_dim % 8 == 0 && a.n_dim % 8 == 0 && (a.dw_dt == a.pq_dt || a.dw_dt == HEXA_F32) &&
-           (size_t)a.r.T < ((size_t)1 << 24) && a.m_dim * 2 < (1 << 24) && a.n_dim * 2 < (1 << 24) &&
-           (size_t)a.r.T * a.m_dim * 2 < ((size_t)1 << 32) && (size_t)a.r.T * a.n_dim * 2 < ((size_t)1 << 32);
-}
-
-int launch_estmm16_big(const EstmmArgs& a, hipStream_t st) {
-    BigEstmmK p;
-    p.pm = a.p; p.qm = a.q; p.dw = a.dw; p.token_ids = a.r.token_ids; p.offsets = a.r.offsets; p.plan = a.plan; p.scratch = a.scratch;
-    p.T = a.r.T; p.k = a.r.k; p.E = a.r.E; p.M = a.m_dim; p.N = a.n_dim;
-    p.mtn = div_up(a.m_dim, 256); p.ntn = div_up(a.n_dim, 256);
-    p.p_slot_rows = a.p_per_slot ? a.r.T : 0;
-    p.q_slot_rows = a.q_per_slot ? a.r.T : 0;
-    p.accumulate = a.accumulate;
-    p.stream_dw = option(OPT_ESMM_STREAM) != 2;
-    p.group = std::min(p.ntn, 8);
-    const int units = a.r.E + (int)std::min<long>(a.max_slots - 1, (long)a.r.E * (PLAN_MAX_PARTS - 1));
-    p.total = (long)units * p.mtn * p.ntn;
-    if (p.total == 0) return HEXA_OK;
-    const bool o32 = a.dw_dt == HEXA_F32;
-    const int rc = a.pq_dt == HEXA_BF16 ? (o32 ? launch_estmm_big_k<__bf16, true>(p, st) : launch_estmm_big_k<__bf16, false>(p, st))
-                                        : (o32 ? launch_estmm_big_k<_Float16, true>(p, st) : launch_estmm_big_k<_Float16, false>(p, st));
-    return rc ? rc : launch_estmm_fixup(a, st);
 }
 
 }  // namespace hexa

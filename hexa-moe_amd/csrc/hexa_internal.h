@@ -129,8 +129,8 @@ bool esmm16_wide_supported(const EsmmArgs& a);
 int launch_esmm16_pipe(const EsmmArgs& a, hipStream_t st);
 bool esmm16_big_supported(const EsmmArgs& a);
 int launch_esmm16_big(const EsmmArgs& a, hipStream_t st);
-bool estmm16_big_supported(const EstmmArgs& a);
-int launch_estmm16_big(const EstmmArgs& a, hipStream_t st);
+bool estmm16_flow_supported(const EstmmArgs& a);
+int launch_estmm16_flow(const EstmmArgs& a, hipStream_t st);
 bool ffn16_fused_supported(int T, int k, int d_in, int hidden, int d_out, int act_dt, int w_dt, int b1_dt, int b2_dt);
 int launch_ffn16_fused(void* y1, void* y2, void* y, const void* x, const void* w1, const void* b1, const void* w2,
                        const void* b2, const RouteView& r, int d_in, int hidden, int d_out, int act_dt, int b1_dt,
