@@ -41,11 +41,19 @@ constexpr int FLOW_SORT_E = 256;       // experts that a workgroup sorts by itse
 struct FlowLds {
     static constexpr int HALF = 32 * 256, STAGE = 2 * HALF;       // 32 list entries x 128 columns of either operand
     static constexpr int IDS_AT = 2 * STAGE;
-    static constexpr int ITEMS_AT = IDS_AT + FLOW_IDS * 32 * 4;   // {expert, steps, row block | column block << 16, scratch slot or -1}
-    static constexpr int SEGS_AT = ITEMS_AT + FLOW_MAX_ITEMS * 16;   // {first id, ids, slot, row block | column block << 16}
+    static constexpr int ITEMS_AT = IDS_AT + FLOW_IDS * 32 * 4;   // {expert, steps, block (flow_block), scratch slot or -1}
+    static constexpr int SEGS_AT = ITEMS_AT + FLOW_MAX_ITEMS * 16;   // {first id, ids, slot, block (flow_block)}
     static constexpr int BYTES = SEGS_AT + FLOW_MAX_SEGS * 16;
     static_assert(4 * BYTES <= 160 * 1024, "four workgroups per CU");
 };
+
+// a block's row and column of blocks in one word, 16 bits each
+__host__ __device__ constexpr unsigned flow_block(int mb, int nb) { return (unsigned)mb | ((unsigned)nb << 16); }
+__host__ __device__ constexpr int flow_row_block(unsigned b) { return (int)(b & 0xffffu); }
+__host__ __device__ constexpr int flow_col_block(unsigned b) { return (int)(b >> 16); }
+constexpr int FLOW_MAX_DIM = 65536 * 128;
+static_assert(flow_row_block(flow_block(65535, 65535)) == 65535 && flow_col_block(flow_block(0, 65535)) == 65535 &&
+              flow_col_block(flow_block(65535, 32768)) == 32768, "16 unsigned bits each");
 
 struct FlowK {
     const void* pm; const void* qm; void* dw;
@@ -75,7 +83,7 @@ __device__ __forceinline__ void estmm16_flow_body(const FlowK& p, int block, cha
         const int rank = (int)(logical / per_e), rem = (int)(logical - (long)rank * per_e);
         // (the dimension with fewer blocks inside: a run shares the longer operand's columns)
         const int mb = p.mtn < p.ntn ? rem % p.mtn : rem / p.ntn, nb = p.mtn < p.ntn ? rem / p.mtn : rem % p.ntn;
-        sItem[j] = make_int4(-1, rank, mb | (nb << 16), -1);
+        sItem[j] = make_int4(-1, rank, (int)flow_block(mb, nb), -1);
     }
     __syncthreads();
     auto take = [&](int u0, int n, int e, int slot) {             // units u0 .. u0 + n - 1 are the parts of expert e
@@ -183,7 +191,7 @@ __device__ __forceinline__ void estmm16_flow_body(const FlowK& p, int block, cha
     auto set_columns = [&]() {
         pb = reinterpret_cast<const char*>(p.pm) + (size_t)(unsigned)(p.p_slot_rows * cd.rec.z) * pitchP;
         qb = reinterpret_cast<const char*>(p.qm) + (size_t)(unsigned)(p.q_slot_rows * cd.rec.z) * pitchQ;
-        const int m = (cd.rec.w & 0xffff) * BM + ch * 8, n = (cd.rec.w >> 16) * BN + ch * 8;
+        const int m = flow_row_block(cd.rec.w) * BM + ch * 8, n = flow_col_block(cd.rec.w) * BN + ch * 8;
         colP = m < M ? (unsigned)m * 2u : 0u;   // (past the result's edge: the row's first bytes; what they produce is not stored)
         colQ = n < N ? (unsigned)n * 2u : 0u;
     };
@@ -300,7 +308,7 @@ __device__ __forceinline__ void estmm16_flow_body(const FlowK& p, int block, cha
         // copies are issued behind the next step's barrier), 16 rows of 32 bits or 32 of 16 at a time.  The 16-byte pieces of a row
         // change places with the row's number, so that the lanes of a write, each in a row of its own, meet different banks.
         barrier_nofence();                      // every wavefront has read its fragments
-        const int m0 = (it.z & 0xffff) * BM + wr * 64, n0 = (it.z >> 16) * BN + wf * 64;
+        const int m0 = flow_row_block(it.z) * BM + wr * 64, n0 = flow_col_block(it.z) * BN + wf * 64;
         const bool whole = it.w < 0;
         const size_t per = (size_t)M * N;
         const unsigned stg = lds0 + ((g + 1) & 1) * L::STAGE + wave * 4096;

@@ -22,7 +22,7 @@ template <typename TC, bool OUT32> int launch_flow_k(const FlowK& p, int grid, h
 
 bool estmm16_flow_supported(const EstmmArgs& a) {
     if (!(a.m_dim % 8 == 0 && a.n_dim % 8 == 0 && (a.dw_dt == a.pq_dt || a.dw_dt == HEXA_F32) && a.r.k <= 8 &&
-          (size_t)a.r.T < ((size_t)1 << 24) && a.m_dim * 2 < (1 << 24) && a.n_dim * 2 < (1 << 24) &&
+          (size_t)a.r.T < ((size_t)1 << 24) && a.m_dim < FLOW_MAX_DIM && a.n_dim < FLOW_MAX_DIM &&
           (size_t)a.r.T * a.m_dim * 2 < ((size_t)1 << 32) && (size_t)a.r.T * a.n_dim * 2 < ((size_t)1 << 32) &&
           (size_t)a.m_dim * a.n_dim * 4 < ((size_t)1 << 32)))
         return false;

@@ -43,3 +43,21 @@ def test_estmm_flow(dev, T, E, k, m, n, skew, dtype):
             if T * m * n < 2e9:
                 want = O.estmm(dy.cpu().float(), x.cpu().float(), token_ids, offsets, wide_first, E)
                 assert_close(got[14][0], want, TOL[dtype], f"{wide_first} {out}")
+
+
+@pytest.mark.parametrize("wide_first", [True, False])
+def test_many_blocks_in_one_dimension(dev, wide_first):
+    """Block numbers of 32768 and more take the sign bit of the word that holds a block's row and column.  (The operands in fp32
+    give the reference: 32 products a result, each exact in fp32, summed in some order.)"""
+    from hexa_moe import ops
+    T, few, many = 32, 8, 32768 * 128 + 8
+    print(f"estmm flow: {many} {'rows' if wide_first else 'columns'} of the result", flush=True)
+    route = ops.route_build(torch.zeros((T, 1), dtype=torch.int64, device=dev), 1)
+    g = torch.Generator(device=dev).manual_seed(1)
+    a, b = (torch.randn(T, n, generator=g, device=dev, dtype=torch.bfloat16) for n in (few, many))
+    if wide_first:
+        a, b = b, a
+    got = ops.estmm(a[None], b, route, True, False)[0]
+    want = torch.matmul(a.float().t().contiguous(), b.float())
+    bound = 2 ** -24 * T * torch.matmul(a.float().abs().t().contiguous(), b.float().abs())
+    assert ((got - want).abs() <= 2 * bound).all()
