@@ -10,9 +10,12 @@
 // GELU and GELU' are gelu_full's, as exact as through erff.
 //
 // What the split has to be careful with, it leaves to the fp32 pipe: a stage of operands that holds a magnitude of 2^63 and
-// more (whose terms could overflow where the product does not), an infinity (0 times infinity in a term) or eight neighbours
-// that are all below 2^-100 (whose l would be a denormal bf16 value short of bits) is written to LDS unsplit and multiplied by
-// v_mfma_f32_32x32x2_f32.  A NaN is one in either way.
+// more (whose terms could overflow where the product does not), an infinity (0 times infinity in a term) or one value other than
+// zero below 2^-100 (whose l would be a denormal bf16 value short of bits; its neighbours may be another result column's, so
+// their size says nothing) is written to LDS unsplit and multiplied by v_mfma_f32_32x32x2_f32.  A NaN is one in either way.
+// Cost of the check: one vector instruction per two values, and two per value more in a stage where a wavefront holds a zero or a small
+// value (9216 tokens, 384 -> 1536, 8 experts, top-2, ESMM and ESTMM alone: 163 and 177 us; half of the values zeros 161 and 175; one in 10000
+// of 1e-33, so that most stages go to the fp32 pipe, 231 and 300; all of them 357 and 392).
 //
 // Values are split once per workgroup, on their way from registers to LDS (6.5 vector instructions a value, about half the
 // MFMA cycles of a 128 x 128 tile), not once per wavefront that reads them; rows are fetched into registers a stage ahead.
@@ -66,14 +69,21 @@ __device__ __forceinline__ float largest(float m, float a, float b) {      // of
     asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
     return r;
 }
-// the planes of eight values; whether they are to be multiplied as they are instead
-__device__ __forceinline__ bool split(const Octet& v, u32x4& h, u32x4& m, u32x4& l) {
+__device__ __forceinline__ float smallest(float m, float a, float b) {     // the same
+    float r;
+    asm("v_min3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
+    return r;
+}
+constexpr float SPLIT_LOW = 0x1p-100f, SPLIT_HIGH = 0x1p63f;
+struct Span { float low, high; };          // smallest and largest magnitude
+// the planes of eight values
+__device__ __forceinline__ void split(const Octet& v, u32x4& h, u32x4& m, u32x4& l, Span& span) {
     const float x[8] = {v.a.x, v.a.y, v.a.z, v.a.w, v.b.x, v.b.y, v.b.z, v.b.w};
-    float big = 0.f;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const float a = x[2 * q], b = x[2 * q + 1];
-        big = largest(big, a, b);
+        span.low = smallest(span.low, a, b);
+        span.high = largest(span.high, a, b);
         const unsigned hw = pack2<__bf16>(a, b);
         const float ra = a - bits_f(hw << 16), rb = b - bits_f(hw & 0xffff0000u);
         const unsigned mw = pack2<__bf16>(ra, rb);
@@ -81,9 +91,13 @@ __device__ __forceinline__ bool split(const Octet& v, u32x4& h, u32x4& m, u32x4&
         m[q] = mw;
         l[q] = pack2<__bf16>(ra - bits_f(mw << 16), rb - bits_f(mw & 0xffff0000u));
     }
-    constexpr unsigned LOW = 0x0d800000u, HIGH = 0x5f000000u;       // 2^-100, 2^63
-    const unsigned u = __float_as_uint(big);
-    return u - LOW >= HIGH - LOW && u != 0;
+}
+// the smallest magnitude other than zero, as bits of 2 |x| - 1, where a zero comes last
+__device__ __forceinline__ unsigned smallest_but_zero(unsigned m, const Octet& v) {
+    const float x[8] = {v.a.x, v.a.y, v.a.z, v.a.w, v.b.x, v.b.y, v.b.z, v.b.w};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) m = min(min(m, 2u * __float_as_uint(x[2 * q]) - 1u), 2u * __float_as_uint(x[2 * q + 1]) - 1u);
+    return m;
 }
 // the same eight values unsplit: their upper and lower halves in the planes of h and m
 __device__ __forceinline__ void halves(const Octet& v, u32x4& hi, u32x4& lo) {
@@ -202,14 +216,21 @@ __device__ __forceinline__ void multiply_stages(int nk, bool busy, char* smem, i
     if (tid < 2) sWhole[tid] = 0;
     for (int kt = 0; kt < nk; ++kt) {
         __syncthreads();                                  // everyone is done reading the stage before
-        bool odd = false;
+        Span span{1.f, 0.f};
         each([&](const Octet& v, char* to, int plane) {
             u32x4 h, m, l;
-            odd |= split(v, h, m, l);
+            split(v, h, m, l, span);
             *reinterpret_cast<u32x4*>(to) = h;
             *reinterpret_cast<u32x4*>(to + plane) = m;
             *reinterpret_cast<u32x4*>(to + 2 * plane) = l;
         });
+        // (zeros are common: rows behind a list's end, tokens' own; they are told from small values only where there are any)
+        bool odd = span.high >= SPLIT_HIGH;
+        if (__builtin_amdgcn_ballot_w64(span.low < SPLIT_LOW) != 0) {
+            unsigned low = ~0u;
+            each([&](const Octet& v, char*, int) { low = smallest_but_zero(low, v); });
+            odd |= low < 2u * __float_as_uint(SPLIT_LOW) - 1u;
+        }
         // (one word for even and one for odd steps: the other one was last read before the barrier above)
         if (tid == 0) sWhole[(kt + 1) & 1] = 0;
         if (odd) sWhole[kt & 1] = 1;
