@@ -227,8 +227,8 @@ def estmm32_slots(T, k, E, out_dim, in_dim):
     """Scratch slots ([out_dim, in_dim] floats each) an fp32 estmm call can use: results with few tiles cut every
     expert's list into up to 8 parts (estmm32_wide of gemm32.hip)."""
     t128, t64 = (E * -(-out_dim // n) * -(-in_dim // n) for n in (128, 64))
-    avg = T * k // E
-    if t128 >= 512 or avg < 256:
+    avg = T * k // max(1, E)
+    if t128 >= 512 or avg < 256 or t128 == 0:      # (the library refuses empty results)
         return 0
     parts = min(-(-768 // t128), avg // 256) if t128 >= 200 and avg >= 1024 else min(-(-1536 // t64), avg // 128)
     parts = max(1, min(8, parts))

@@ -180,3 +180,10 @@ def test_triton_sibling_surface_signatures():
     import torch
     with __import__("pytest").raises(RuntimeError):
         kernels.counter(torch.zeros(8, dtype=torch.int32), 4)       # CPU tensors are rejected: no fallback
+
+
+@pytest.mark.parametrize("out_dim,in_dim", [(0, 8), (8, 0), (0, 0)])
+def test_fp32_scratch_of_an_empty_result(out_dim, in_dim):
+    """Sizes the library refuses reach it: nothing divides by them on the way."""
+    from hexa_moe import ops
+    assert ops.estmm32_slots(600, 2, 2, out_dim, in_dim) == 0
