@@ -30,7 +30,7 @@ def test_estmm_flow(dev, T, E, k, m, n, skew, dtype):
         dy, x = dy.to(dev), x.to(dev)
         for out in (dtype, torch.float32):
             got = {}
-            for tile in (8, 14):
+            for tile in (8, 15):                             # (15: an error where the persistent kernel does not run)
                 _lib.check(lib.hexa_set_option(b"tile", tile), "hexa_set_option")
                 try:
                     dw = ops.estmm(dy, x, route, *per, out_dtype=out)
@@ -38,11 +38,11 @@ def test_estmm_flow(dev, T, E, k, m, n, skew, dtype):
                     torch.cuda.synchronize()
                 finally:
                     _lib.check(lib.hexa_set_option(b"tile", 0), "hexa_set_option")
-            for want, have in zip(got[8], got[14]):
+            for want, have in zip(got[8], got[15]):
                 assert torch.equal(have, want), (wide_first, out)
             if T * m * n < 2e9:
                 want = O.estmm(dy.cpu().float(), x.cpu().float(), token_ids, offsets, wide_first, E)
-                assert_close(got[14][0], want, TOL[dtype], f"{wide_first} {out}")
+                assert_close(got[15][0], want, TOL[dtype], f"{wide_first} {out}")
 
 
 @pytest.mark.parametrize("wide_first", [True, False])
