@@ -44,7 +44,7 @@ struct FlowLds {
     static constexpr int ITEMS_AT = IDS_AT + FLOW_IDS * 32 * 4;   // {expert, steps, block (flow_block), scratch slot or -1}
     static constexpr int SEGS_AT = ITEMS_AT + FLOW_MAX_ITEMS * 16;   // {first id, ids, slot, block (flow_block)}
     static constexpr int BYTES = SEGS_AT + FLOW_MAX_SEGS * 16;
-    static_assert(4 * BYTES <= 160 * 1024, "four workgroups per CU");
+    static_assert(4 * BYTES <= 160 * 1024, "four workgroups per CU where the kernel has no other LDS");
 };
 
 // a block's row and column of blocks in one word, 16 bits each
@@ -382,6 +382,8 @@ __device__ __forceinline__ void estmm16_flow_body(const FlowK& p, int block, cha
 }
 
 // the kernel's arguments; returns the grid (0: nothing to do)
+// (workgroups for four a CU.  The shared backward launches hold three, see backward16_kernel: there, behind the ESMM's workgroups, the
+// last quarter starts when others end.)
 inline int flow_args(const EstmmArgs& a, FlowK& p) {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8) cus = 256;

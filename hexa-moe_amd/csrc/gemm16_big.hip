@@ -9,7 +9,9 @@
 // apart, kept there by one barrier more for the second group: while one group multiplies, the other reads fragments
 // and issues copies.  A stage is two halves of 64 rows per wavefront, whose four kinds of copies (upper and lower rows, even
 // and odd columns) are issued where the half of the buffer they overwrite has been read by both groups, one stage ahead; waits
-// count the younger copies and the stores of the tile before (s_waitcnt vmcnt), so nothing is drained between tiles.
+// count the younger copies and the stores of the tile before (s_waitcnt vmcnt), so nothing is drained between the tiles of plain and
+// GELU launches.  GELU' waits for its block's y1 in every epilogue, and with it for the copies in front of it, which were issued
+// a stage before; its fp16 instances with column sums spill one register (an address, reloaded once a tile).
 //
 // Measured: 8192 x 8192 x 8192 in bf16 1322 TFLOP/s in this schedule (1113 by the vendor's library on the same card); a
 // stage takes 1.4 to 1.6 us per round of 256 tiles.  32768 rows, top-2 of 64 experts with a skewed load, 1024 -> 4096: plain 888 us

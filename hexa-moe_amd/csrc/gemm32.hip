@@ -19,8 +19,8 @@
 //
 // Values are split once per workgroup, on their way from registers to LDS (6.5 vector instructions a value, about half the
 // MFMA cycles of a 128 x 128 tile), not once per wavefront that reads them; rows are fetched into registers a stage ahead.
-// One set of planes and two barriers a stage: 48 KB a workgroup, so that two of eight or three of four wavefronts share a CU and
-// one's split and barriers meet another's MFMAs.
+// One set of planes and two barriers a stage: 48 KB and eight wavefronts a workgroup, so that two (by registers; three by LDS) share a
+// CU and one's split and barriers meet another's MFMAs.
 // What bounds them: matrix and vector instructions, which overlap in part only (a launch without the split, or without the MFMAs,
 // takes 0.9 and 0.6 of its time; without fetches 0.95).  At 9216 tokens, 384 -> 1536, 8 experts, top-2 (21.7 GFLOP a launch; before:
 // v_mfma_f32_32x32x2_f32 fed by asynchronous copies, at 64 % of its pipe's rate), kernel times inside a training step: fc1 + GELU
@@ -465,7 +465,7 @@ __global__ __launch_bounds__(C::NT, C::WAVES) void estmm32_kernel(Estmm32K p) {
         __syncthreads();
         e = __builtin_amdgcn_readfirstlane(sExpert);
     }
-    // The expert's steps of 32 list entries, slot after slot (the last step of a slot's list may be partial), and this
+    // The expert's steps of KD list entries, slot after slot (the last step of a slot's list may be partial), and this
     // workgroup's part of them.
     auto begin = [&](int s) { return p.offsets[(size_t)s * (E + 1) + e]; };
     auto end = [&](int s) { return p.offsets[(size_t)s * (E + 1) + e + 1]; };
@@ -647,6 +647,7 @@ int launch_esmm32(const EsmmArgs& a, hipStream_t st) {
 // more into parts, and below that 64 x 64 tiles until there are six workgroups per CU (or 128 entries a part).  Measured with
 // one part of 64 x 64 tiles against this: 18432 entries, 8 experts, 1536 x 384 195 -> 178 us, 8192, 4, 2048 x 512 156 -> 133,
 // 5000, 12, 800 x 200 72 -> 45; uncut 128 x 128 against 64 x 64 tiles at 12000, 32, 3072 x 768 402 against 537.
+// The parts' scratch is 84 MB a result at the most: less than 768 + 512 blocks of 128 x 128 floats, or 2 * 1536 of 64 x 64.
 static bool estmm32_wide(int T, int k, int E, int m_dim, int n_dim, int* parts) {
     const long t128 = (long)E * div_up(m_dim, 128) * div_up(n_dim, 128), t64 = (long)E * div_up(m_dim, 64) * div_up(n_dim, 64);
     const long avg = (long)T * k / std::max(1, E);

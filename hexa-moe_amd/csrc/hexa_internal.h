@@ -115,7 +115,7 @@ enum Opt {
     OPT_BATCH,          // HEXA_MOE_BATCH: 2 = every small kernel of the depth backward in a launch of its own, 1 = four batch launches instead of three
     OPT_FFN_FUSED,      // HEXA_MOE_FFN_FUSED: 1 = hexa_moe_depth_forward runs fc1, GELU and fc2 in one kernel where it is covered
     OPT_GATE_ROUTER,    // HEXA_MOE_GATE_ROUTER: 2 = hexa_moe_depth_forward runs the gate projection and the router as two launches
-    OPT_ESTMM_PIPE,     // HEXA_ESTMM_PIPE: 1 = the persistent ESTMM kernel wherever it applies (default: the one-item-per-workgroup kernel)
+    OPT_ESTMM_PIPE,     // HEXA_ESTMM_PIPE: 1 = the role-split ESTMM kernel (gemm16_estmm_pipe.hip) wherever it applies (default: estmm_flow.h)
     OPT_SIDE_STREAM,    // HEXA_MOE_SIDE_STREAM: the small kernels of hexa_moe_depth_backward on a second stream beside the matmul kernels: 1 = yes, 2 = no
     OPT_BACKWARD_FUSED, // HEXA_MOE_BACKWARD_FUSED: the independent products of a depth's backward in shared launches: 1 = wherever covered, 2 = never
     OPT_COUNT
@@ -139,7 +139,7 @@ int launch_colsum_fold(const EsmmArgs& a, int mt_ub, int tile_rows, int ntn, int
 int estmm_plan_cap_for(const RouteView& r, int out_dim, int in_dim);   // rows above which an expert's list is cut
 int launch_estmm_plan(int32_t* plan, const RouteView& r, int max_slots, int cap, hipStream_t st);
 int launch_estmm_fixup(const EstmmArgs& a, hipStream_t st);
-// whether a routing of this size goes to the persistent ESTMM kernel (the plan is made for the kernel that will run)
+// whether ESTMM goes to the role-split kernel (the plan is made for the kernel that will run)
 bool estmm_pipe_wanted(const RouteView& r);
 bool estmm16_pipe_supported(const EstmmArgs& a);
 int launch_estmm16_pipe(const EstmmArgs& a, hipStream_t st);

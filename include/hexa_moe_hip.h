@@ -120,7 +120,8 @@ int hexa_route_from_padded_lists(const int32_t* token_idx_list, const int32_t* e
  *   m2s == 0: x [T,in] shared by the slots, out [k,T,out]      (fc1 of the MoE FFN)
  *   m2s != 0: x [k,T,in] per slot,          out [T,out] = sum over slots (fc2; deterministic order)
  * w_layout selects w[E][in][out] or w[E][out][in]; bias [E][out] may be NULL.  x_dt is F32 (then w,
- * bias and out must be F32: true-fp32 MFMA path) or F16/BF16 (w may be the same 16-bit type or F32,
+ * bias and out must be F32: fp32 accuracy, by three exact bf16 terms of each operand or, where a value has none, the fp32
+ * matrix instruction) or F16/BF16 (w may be the same 16-bit type or F32,
  * fp32 accumulation; out may be that 16-bit type or F32).  accumulate != 0 adds into `out`.
  * act == HEXA_ACT_GELU additionally writes gelu(out) to out_act (same shape/dtype as out; m2s == 0).
  * act == HEXA_ACT_GELU_BWD multiplies the result by gelu'(y1), y1 read from out_act (same shape/dtype
@@ -145,15 +146,14 @@ int hexa_esmm(void* out, const void* x, const void* w, const void* bias, const i
  * dy_per_slot / x_per_slot say whether the operand is [k,T,*] (1) or [T,*] shared by the slots (0).
  * dt is the element type of dy and x (F32, F16 or BF16); dw_dt is F32 or dt.  Experts without tokens
  * get exact zeros (or are left untouched when accumulating).
- * plan / max_slots / scratch (optional).  With a plan from hexa_estmm_plan for the same
- * routing, max_slots and result size, the persistent kernel runs (up to 256 experts and 8 slots): one workgroup per
- * CU takes (expert, 128 x 128 block) items from a queue, longest first, so the load balances without cutting
- * experts; only an expert whose list is longer than a workgroup's share of the whole launch is cut into up to 8
+ * plan / max_slots / scratch (optional).  16-bit operands run on persistent workgroups, up to four per CU, that are dealt
+ * (expert, 128 x 128 block) items, the longest lists first.  With a plan from hexa_estmm_plan for the same routing, max_slots and
+ * result size, an expert whose list is longer than a workgroup's share of the launch is cut into up to 8
  * parts, whose fp32 partial results go through `scratch` (max_slots * out_dim * in_dim floats; max_slots < 2 or
- * scratch == NULL: nothing is cut) and are added in a fixed order, so results stay bit-reproducible.  The plan
- * also holds the queue's counters, which the call updates and leaves at zero: calls that share a plan must not
- * overlap (calls on one stream do not).  Without a plan one workgroup walks an expert's whole token list per
- * block and the kernel is as slow as the busiest expert.
+ * scratch == NULL: nothing is cut) and are added in a fixed order, so results stay bit-reproducible.  Without a plan
+ * one workgroup walks an expert's whole token list per block and a launch is as slow as the busiest expert.  (Option
+ * "estmm_pipe" = 1: one workgroup per CU takes the items from queues whose counters are in the plan; the call updates them and leaves
+ * them at zero, so calls that share a plan must not overlap then.)
  * fp32 operands need no plan: with max_slots >= 2 * num_experts and as much scratch, a launch with few result tiles cuts
  * every list into the same number of parts (up to 8, max_slots / num_experts at most), added in their order.
  * Replaces the ESTMM task of FUSED_GRAD (kernels/fused_ops_full.cu:248-371). */
@@ -164,7 +164,7 @@ int hexa_estmm(void* dw, const void* dy, const void* x, const int32_t* route, in
 /* Work plan of hexa_estmm for one routing: HEXA_ESTMM_PLAN_INTS(num_experts) ints (experts by decreasing load,
  * their parts, first work unit and first scratch slot, number of units, then the work queue's counters, zeroed).
  * out_dim / in_dim: the size of the result the plan is for (0, 0: unknown -- experts above 1.5x the mean load are
- * cut, the rule of the one-item-per-workgroup kernel).  Depends on the routing, max_slots and that size only, so
+ * cut).  Depends on the routing, max_slots and that size only, so
  * one plan serves every hexa_estmm call of a layer's backward whose results have the same number of 128 x 128
  * blocks.  No counterpart in the reference, whose ESTMM task walks each expert's list in one thread block
  * (kernels/fused_ops_full.cu:248-371). */
