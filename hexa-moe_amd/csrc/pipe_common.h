@@ -51,7 +51,6 @@ template <int N, typename F> __device__ __forceinline__ void static_for(F&& f) {
     static_for_impl(std::make_integer_sequence<int, N>{}, f);
 }
 __device__ __forceinline__ void lds_wait() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-// 16 bytes from base + off (a scalar base and a 32-bit lane offset: one address register per lane)
 // 16-byte store to base + off (a base every lane shares plus a 32-bit byte offset); `streaming` (uniform) adds the
 // non-temporal hint.  A store of more than 8 bytes reads its data for two wait states after its issue; the compiler keeps
 // vector instructions that overwrite it away from stores of its own, but does not look into inline assembly: s_nop 1.
@@ -59,6 +58,7 @@ __device__ __forceinline__ void global_store128(void* base, unsigned off, u32x4 
     if (streaming) asm volatile("global_store_dwordx4 %0, %1, %2 nt\n\ts_nop 1" ::"v"(off), "v"(v), "s"(base) : "memory");
     else asm volatile("global_store_dwordx4 %0, %1, %2\n\ts_nop 1" ::"v"(off), "v"(v), "s"(base) : "memory");
 }
+// 16 bytes from base + off (one address register per lane)
 __device__ __forceinline__ u32x4 global_load128_async(const void* base, unsigned off) {
     u32x4 r;
     asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(r) : "v"(off), "s"(base));

@@ -79,7 +79,7 @@ class Route:
     def estmm_plan(self, max_slots, out_dim=0, in_dim=0):
         """Work plan of estmm for this routing and result size (int32 [HEXA_ESTMM_PLAN_INTS]); made on first use,
         then shared by every estmm call on the routing whose result has as many 128 x 128 blocks.  The plan also
-        holds the work queue of the persistent kernel, so calls that use it must not overlap (one stream)."""
+        holds the work queue of the role-split kernel (option "estmm_pipe"), whose calls on one plan must not overlap (one stream)."""
         key = (int(max_slots), -(-int(out_dim) // 128) * -(-int(in_dim) // 128))
         plan = self._plans.get(key)
         if plan is None:
@@ -251,7 +251,7 @@ def estmm(dy, x, route, dy_per_slot, x_per_slot, out=None, out_dtype=torch.float
     plan = scratch = None
     slots = 0
     if x.dtype != torch.float32:
-        # a plan (made once per routing and result size) orders the work of the persistent kernel; with lists long
+        # a plan (made once per routing and result size) orders the work, longest lists first; with lists long
         # enough to be worth cutting it comes with scratch for up to 2E fp32 partial results, at most 256 MiB
         if T * k >= 128 * E and (out_dim * in_dim) % 4 == 0:
             slots = min(2 * E, (256 << 20) // (out_dim * in_dim * 4))
