@@ -91,6 +91,13 @@ template <int G, int MAXA> __device__ __forceinline__ void wait_groups(int ahead
     else wait_vmcnt<0>();
 }
 
+// the same with a group of N to N + SPAN copies (`more` above N), whatever this wavefront has to fetch
+template <int N, int SPAN, int MAXA> __device__ __forceinline__ void wait_groups_of(int more, int ahead) {
+    if constexpr (SPAN == 0) wait_groups<N, MAXA>(ahead);
+    else if (more == SPAN) wait_groups<N + SPAN, MAXA>(ahead);
+    else wait_groups_of<N, SPAN - 1, MAXA>(more, ahead);
+}
+
 // Workgroup barrier WITHOUT the memory fence of __syncthreads(): the fence would wait for every
 // outstanding copy (vmcnt(0)) and drain the pipeline.  Ordering is by hand: copies are awaited with
 // wait_vmcnt, LDS reads of the previous stage have been consumed by MFMAs before a wavefront arrives.

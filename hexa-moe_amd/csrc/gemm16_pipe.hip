@@ -104,9 +104,11 @@ __global__ __launch_bounds__(C::NT + 64 * (PIPE_COPY_WAVES + PIPE_STORE_WAVES)) 
     const EsmmK& p = pk.e;
     constexpr int BM = C::BM, BN = C::BN, STAGES = C::STAGES, NW = C::NW, BK = C::BKC;
     constexpr int CW = PIPE_COPY_WAVES, SW = PIPE_STORE_WAVES, NTS = 64 * SW, NT_ALL = C::NT + 64 * (CW + SW);
-    constexpr int R_CPW = C::R_COPIES / CW, F_CPW = C::F_COPIES / CW, CPW = R_CPW + F_CPW;   // copies per copy wavefront and stage
+    constexpr int R_CPW = C::R_COPIES / CW, F_CPW = C::F_COPIES / CW;   // copies per copy wavefront and stage
     static_assert(C::R_COPIES % CW == 0 && C::F_COPIES % CW == 0, "copies must divide evenly over the copy wavefronts");
     static_assert(BM <= 64 * CW, "at most one 64-id copy per copy wavefront");
+    static_assert(STAGES == 3, "the copy wavefronts wait for all but the last group");
+    static_assert(CW * (512 / BK) == 32 && C::RB <= 2, "a copy wavefront's i-th copy of rows belongs to row block i; one block or all of a wavefront's");
     constexpr int LUT = pipe_lut_bytes<TC, ACT, COLSUM>();
     constexpr unsigned LUT_LO = pipe_lut_lo<TC, ACT, COLSUM>(), LUT_R = LUT_M_HI - LUT_LO;
     using L = PipeLds<C, LUT, COLSUM>;
@@ -181,18 +183,26 @@ __global__ __launch_bounds__(C::NT + 64 * (PIPE_COPY_WAVES + PIPE_STORE_WAVES)) 
         zero_acc(acc);
         int stage = 0;
         for (int r = 0; r < ntiles; ++r) {
-            for (int kt = 0; kt < nk; ++kt) {
-                barrier_nofence();                       // the copies of this step have landed
-                const unsigned base = lds0 + L::STAGES_AT + stage * C::STAGE_BYTES;
-                mma_stage_ahead<TC, C, W_IN_OUT>(base, base + C::R_BYTES, wr, wf, lane, acc);
-                stage = stage + 1 == STAGES ? 0 : stage + 1;
-            }
+            auto steps = [&](auto nrb) {
+                constexpr int NRB = decltype(nrb)::value;
+                for (int kt = 0; kt < nk; ++kt) {
+                    barrier_nofence();                   // the copies of this step have landed
+                    const unsigned base = lds0 + L::STAGES_AT + stage * C::STAGE_BYTES;
+                    if constexpr (NRB > 0) mma_stage_ahead<TC, C, W_IN_OUT, false, NRB>(base, base + C::R_BYTES, wr, wf, lane, acc);
+                    stage = stage + 1 == STAGES ? 0 : stage + 1;
+                }
+            };
+            // (the row blocks wr, wr + WR, ... that hold rows)
+            const int blocks = (tile_rec(r).rows - 32 * wr + 32 * C::WR - 1) / (32 * C::WR);
+            if (blocks >= C::RB) steps(std::integral_constant<int, C::RB>());
+            else if (blocks > 0) steps(std::integral_constant<int, 1>());
+            else steps(std::integral_constant<int, 0>());
             barrier_nofence();                           // (A) the store wavefronts are done with the staging area
             // accumulators (+ bias, rounded) -> staging area
-            constexpr int RW = 32 * C::RB, FW = 32 * C::FB;
+            constexpr int FW = 32 * C::FB;
             const int nl0 = wf * FW + 4 * (lane >> 5);            // + j * 32 + 8 * gq
             const unsigned bias_at = lds0 + L::BIAS_AT + (r % 3) * L::BIAS_SLOT + nl0 * bias_esz;
-            const unsigned stg = lds0 + L::STAGING_AT + (wr * RW + (lane & 31)) * CP + nl0 * 2;   // + i * 32 * CP
+            const unsigned stg = lds0 + L::STAGING_AT + (wr * 32 + (lane & 31)) * CP + nl0 * 2;   // + i * 32 * WR * CP
             float bv[C::FB * 4][4];
 #pragma unroll
             for (int u = 0; u < C::FB * 4; ++u) { bv[u][0] = 0.f; bv[u][1] = 0.f; bv[u][2] = 0.f; bv[u][3] = 0.f; }
@@ -229,7 +239,7 @@ __global__ __launch_bounds__(C::NT + 64 * (PIPE_COPY_WAVES + PIPE_STORE_WAVES)) 
                 constexpr int u = decltype(jg)::value, j = u / 4, gq = u % 4;
                 static_for<C::RB>([&](auto ic) {
                     constexpr int i = decltype(ic)::value;
-                    lds_write64<i * 32 * CP + (j * 32 + 8 * gq) * 2>(
+                    lds_write64<i * 32 * C::WR * CP + (j * 32 + 8 * gq) * 2>(
                         stg, pack4<TC>(acc[j][i][4 * gq] + bv[u][0], acc[j][i][4 * gq + 1] + bv[u][1],
                                        acc[j][i][4 * gq + 2] + bv[u][2], acc[j][i][4 * gq + 3] + bv[u][3]));
                 });
@@ -251,10 +261,12 @@ __global__ __launch_bounds__(C::NT + 64 * (PIPE_COPY_WAVES + PIPE_STORE_WAVES)) 
         const char* const xbase = reinterpret_cast<const char*>(p.x);
         const char* wbase = reinterpret_cast<const char*>(p.w);
         unsigned srcR[R_CPW]; int stepR[R_CPW];
+        int copiesR = 0;                                 // of a tile's rows in blocks of 32, one copy per wavefront each
         unsigned srcF[F_CPW]; int stepF[F_CPW];
         auto set_sources = [&](int r) {   // this lane's copy sources for tile r (its token ids are in LDS)
             const Rec rec = tile_rec(r);
             const int e = rec.e, rows = rec.rows, s = rec.s, n0 = rec.nt * BN;
+            copiesR = (rows + 31) >> 5;
             wbase = reinterpret_cast<const char*>(p.w) + (size_t)e * K * N * 2;
             int rowi[R_CPW], kci[R_CPW], toki[R_CPW];
 #pragma unroll
@@ -294,6 +306,7 @@ __global__ __launch_bounds__(C::NT + 64 * (PIPE_COPY_WAVES + PIPE_STORE_WAVES)) 
             char* base = smem + L::STAGES_AT + stage * C::STAGE_BYTES;
 #pragma unroll
             for (int i = 0; i < R_CPW; ++i) {
+                if (i >= copiesR) break;
                 dma16(xbase + (size_t)srcR[i], base + (cw + CW * i) * 1024);
                 srcR[i] += stepR[i];
             }
@@ -310,6 +323,7 @@ __global__ __launch_bounds__(C::NT + 64 * (PIPE_COPY_WAVES + PIPE_STORE_WAVES)) 
             char* base = smem + L::STAGES_AT + stage * C::STAGE_BYTES;
 #pragma unroll
             for (int i = 0; i < R_CPW; ++i) {
+                if (i >= copiesR) break;
                 int row, kc;
                 kc_lane<BK>(cw + CW * i, lane, row, kc);
                 dma16(kc * 8 < ktail ? xbase + (size_t)srcR[i] : zero, base + (cw + CW * i) * 1024);
@@ -368,8 +382,8 @@ __global__ __launch_bounds__(C::NT + 64 * (PIPE_COPY_WAVES + PIPE_STORE_WAVES)) 
         long issued = STAGES - 1, g = 0;                 // steps whose copies have been issued; global step
         for (int r = 0; r < ntiles; ++r) {
             for (int kt = 0; kt < nk; ++kt, ++g) {
-                // the copies of step g have landed when at most the groups of the later steps are outstanding
-                wait_groups<CPW, STAGES - 2>((int)min(total_steps - 1 - g, (long)(STAGES - 2)));
+                // the copies of step g have landed when at most the group of the step behind it, the last one issued, is outstanding
+                wait_groups_of<F_CPW, R_CPW, STAGES - 2>(copiesR, (int)min(total_steps - 1 - g, (long)(STAGES - 2)));
                 // A tile's first step: the stage to refill was read in the previous tile's last step, which barrier
                 // (A) has closed, and the ring slots the next tile's token ids and bias go to were last used two tiles
                 // ago -- so these copies are issued BEFORE the step's barrier, while the multiply wavefronts are

@@ -71,24 +71,26 @@ __device__ __forceinline__ u32x4 global_load128_async(const void* base, unsigned
 // All reads are inline assembly and return in order: the wait before step ks allows exactly the reads of step
 // ks+1 to be outstanding, and every fragment passes through an empty statement behind that wait.
 template <int N> __device__ __forceinline__ void lds_wait_but() { asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory"); }
-template <typename TC, typename C, bool F_KS, bool R_KS = false>
+// NRB: row blocks of this wavefront that hold anything (block i of KC rows is tile row 32 * (wr + WR * i) on,
+// so that a tile of few rows keeps all wavefronts busy).
+template <typename TC, typename C, bool F_KS, bool R_KS = false, int NRB = C::RB>
 __device__ __forceinline__ void mma_stage_ahead(unsigned tileR, unsigned tileF, int wr, int wf, int lane, f32x16 (&acc)[C::FB][C::RB]) {
     using V = typename Mfma<TC>::V;
     constexpr int RW = 32 * C::RB, FW = 32 * C::FB, KD = C::BKC, NKS = KD / 16;
-    constexpr int READS = (R_KS ? 2 * C::RB : C::RB) + (F_KS ? 2 * C::FB : C::FB);      // LDS read instructions per contraction step
+    constexpr int READS = (R_KS ? 2 * NRB : NRB) + (F_KS ? 2 * C::FB : C::FB);      // LDS read instructions per contraction step
     union Frag { V v; u32x4 q; s16x4 h[2]; };
-    Frag f[2][C::FB], r[2][C::RB];
+    Frag f[2][C::FB], r[2][NRB];
     // what does not depend on the step: the row of a KC fragment and its swizzle, the column part of a KS one
-    unsigned rbase[C::RB]; int rsw[C::RB];
+    unsigned rbase[NRB]; int rsw[NRB];
     const int grp = lane >> 4, sl = lane & 15;
 #pragma unroll
-    for (int i = 0; i < C::RB; ++i) {
+    for (int i = 0; i < NRB; ++i) {
         if (R_KS) {
             const int col = wr * RW + i * 32 + (grp & 1) * 16 + (sl & 3) * 4;
             rbase[i] = tileR + (col & 7) * 2;
             rsw[i] = col >> 3;
         } else {
-            const int row = wr * RW + i * 32 + (lane & 31);
+            const int row = (wr + C::WR * i) * 32 + (lane & 31);
             rbase[i] = tileR + row * (2 * KD);
             rsw[i] = kc_swizzle<KD>(row);
         }
@@ -106,7 +108,7 @@ __device__ __forceinline__ void mma_stage_ahead(unsigned tileR, unsigned tileF, 
             fsw[j] = kc_swizzle<KD>(row);
         }
     }
-    auto read_step = [&](int ks, Frag (&fs)[C::FB], Frag (&rs)[C::RB]) {
+    auto read_step = [&](int ks, Frag (&fs)[C::FB], Frag (&rs)[NRB]) {
         const int kch = ks * 2 + (lane >> 5);
 #pragma unroll
         for (int j = 0; j < C::FB; ++j) {
@@ -122,7 +124,7 @@ __device__ __forceinline__ void mma_stage_ahead(unsigned tileR, unsigned tileF, 
             }
         }
 #pragma unroll
-        for (int i = 0; i < C::RB; ++i) {
+        for (int i = 0; i < NRB; ++i) {
             if (R_KS) {
                 const int k = ks * 16 + (grp >> 1) * 8 + (sl >> 2);
 #pragma unroll
@@ -148,11 +150,11 @@ __device__ __forceinline__ void mma_stage_ahead(unsigned tileR, unsigned tileF, 
 #pragma unroll
         for (int j = 0; j < C::FB; ++j) asm volatile("" : "+v"(f[cur][j].q));
 #pragma unroll
-        for (int i = 0; i < C::RB; ++i) asm volatile("" : "+v"(r[cur][i].q));
+        for (int i = 0; i < NRB; ++i) asm volatile("" : "+v"(r[cur][i].q));
 #pragma unroll
         for (int j = 0; j < C::FB; ++j)
 #pragma unroll
-            for (int i = 0; i < C::RB; ++i) acc[j][i] = Mfma<TC>::run(f[cur][j].v, r[cur][i].v, acc[j][i]);
+            for (int i = 0; i < NRB; ++i) acc[j][i] = Mfma<TC>::run(f[cur][j].v, r[cur][i].v, acc[j][i]);
     }
 }
 
