@@ -39,6 +39,13 @@
 namespace hexa {
 namespace {
 
+// Two row tiles of an expert side by side, all their column tiles one after the other: neighbours, which run at the same time on one
+// XCD, then share a column tile of weights and a row tile of tokens.  Against all column tiles of one row tile first, us a launch, fc1 + GELU | dy1
+// | dx: 4608 rows of 32 experts, 768 -> 3072 (4.7 MB of weights an expert, more than an L2) 55.5, 52.7 | 59.3, 59.1 | -; 18432 rows, top-2,
+// 384 -> 1536 87.5, 87.4 | 106.3, 103.2 | 66.5, 65.1.  Runs of four: 51.4 | 57.8 | - and 93.7 | 107.2 | 65.7.  Finding a tile takes two more trips
+// to memory at a workgroup's start (144 tokens of 32 experts: 48.9 us a pass without, 50.1 with), so lists of less than three quarters of a
+// row tile in the mean, which hardly ever have two, go without.
+constexpr int PIPE_ROW_RUN = 2;
 constexpr int PIPE_MAX_ROUNDS = 256;   // tiles one workgroup may walk (their records are kept in LDS)
 
 #ifndef PIPE_WR
@@ -65,6 +72,8 @@ template <typename TC, int ACT, bool COLSUM> constexpr int pipe_lut_bytes() {
 struct PipeK {
     EsmmK e;
     int wg_per_xcd;       // workgroups per XCD (grid = 8 * wg_per_xcd)
+    const int32_t* offsets; int E;   // of the route
+    int row_run;          // an expert's tiles are walked in runs of so many row tiles, rows fastest (1: column tiles fastest)
 };
 
 #ifndef PIPE_CW
@@ -126,7 +135,7 @@ __global__ __launch_bounds__(C::NT + 64 * (PIPE_COPY_WAVES + PIPE_STORE_WAVES)) 
     const int K = p.K, N = p.N, nk = TAIL ? K / BK + 1 : K / BK;
     const bool streaming = p.stream_out != 0;           // results leave with the non-temporal hint
 
-    // ---- this workgroup's walk: XCD x owns one contiguous eighth of the valid tiles (column tiles fastest);
+    // ---- this workgroup's walk: XCD x owns one contiguous eighth of the valid tiles (in the order of PIPE_ROW_RUN);
     // the workgroups of an XCD take its tiles round-robin, so at any time they share token rows and weights
     int cum[9];
     cum[0] = 0;
@@ -142,12 +151,24 @@ __global__ __launch_bounds__(C::NT + 64 * (PIPE_COPY_WAVES + PIPE_STORE_WAVES)) 
     int4* sInfo = reinterpret_cast<int4*>(smem + L::INFO_AT);   // {expert, first list position, rows | row tile << 10, slot << 24 | column tile}
     for (int i = tid; i < ntiles; i += NT_ALL) {
         const int logical = first + i * pk.wg_per_xcd;
-        const int mtg = logical / p.ntn, nt = logical - mtg * p.ntn;
+        int mtg = logical / p.ntn, nt = logical - mtg * p.ntn;
         int sl = 0;
 #pragma unroll
         for (int q = 1; q < 8; ++q) sl += (mtg >= cum[q] && q < p.nslots) ? 1 : 0;
         const int s = p.slot_begin + sl;
-        const int4 rec = p.tile_info[(size_t)s * p.mt_ub + (mtg - cum[sl])];
+        const int4* const slot_info = p.tile_info + (size_t)s * p.mt_ub;
+        int4 rec = slot_info[mtg - cum[sl]];
+        if (pk.row_run > 1) {
+            const int32_t* const off = pk.offsets + (size_t)s * (pk.E + 1) + rec.x;
+            const int base = mtg - (rec.y - off[0]) / BM;               // the expert's first row tile, and how many it has
+            const int m = min((off[1] - off[0] + BM - 1) / BM, cum[sl + 1] - base);
+            int l = logical - base * p.ntn;
+            const int run = l / (pk.row_run * p.ntn), rows = min(pk.row_run, m - run * pk.row_run);
+            l -= run * pk.row_run * p.ntn;
+            nt = l / rows;
+            mtg = base + run * pk.row_run + (l - nt * rows);
+            rec = slot_info[mtg - cum[sl]];
+        }
         sInfo[i] = make_int4(rec.x, rec.y, rec.z | ((mtg - cum[sl]) << 10), (s << 24) | nt);
     }
     if constexpr (LUT > 0) {
@@ -696,6 +717,8 @@ int launch_esmm16_pipe(const EsmmArgs& a, hipStream_t st) {
     if (p.total == 0) return HEXA_OK;
     pk.wg_per_xcd = (int)std::min<long>(std::max(1, compute_units() / 8), (p.total + 7) / 8);
     const int grid = 8 * pk.wg_per_xcd;
+    pk.offsets = a.r.offsets; pk.E = a.r.E;
+    pk.row_run = option(OPT_ESMM_GROUP) > 0 ? option(OPT_ESMM_GROUP) : (long)a.r.T * 4 >= 3L * C::BM * a.r.E ? PIPE_ROW_RUN : 1;
     const bool io = a.w_layout == HEXA_W_IN_OUT;
     if (a.wide && !io) HEXA_FAIL(HEXA_ERR_UNSUPPORTED, "esmm16_pipe: fp32 storage is for weights [in][out]");
     const int act = a.wide ? PIPE_ACT_WIDE : a.act;

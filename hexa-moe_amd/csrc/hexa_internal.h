@@ -106,7 +106,7 @@ enum Opt {
                         // whatever it covers; 2 = never, 1 = also when a tile shape is forced
     OPT_GENERAL,        // HEXA_MOE_GENERAL_KERNELS: 1 = general 16-bit kernels instead of the fast path
     OPT_ESMM_MAP,       // HEXA_ESMM_MAP: 2 = runs of tiles per XCD instead of one contiguous eighth of the tiles per XCD
-    OPT_ESMM_GROUP,     // HEXA_ESMM_GROUP: row tiles per XCD run
+    OPT_ESMM_GROUP,     // HEXA_ESMM_GROUP: row tiles per run (one-tile kernels with esmm_map = 2: of an XCD; pipelined kernel: side by side)
     OPT_ESTMM_GROUP,    // HEXA_ESTMM_GROUP: row tiles per XCD run
     OPT_ESMM_STREAM,    // HEXA_ESMM_STREAM: results stored with the streaming (non-temporal) hint: 0 = by the pipelined ESMM
                         // kernel and ESTMM's finished results, 1 = by the one-tile ESMM kernels as well, 2 = by none
