@@ -9,7 +9,7 @@ namespace {
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
 constexpr int GT = 32;          // tokens per workgroup (forward)
-constexpr int FWD_NB = 6;       // chunks of 8 contraction indices a wavefront of the forward kernel loads per trip
+constexpr int FWD_NB = 6;       // chunks of 16 contraction indices a wavefront of the forward kernels loads per trip
 constexpr int BWD_TB = 64;      // tokens per chunk of the backward tasks (and per dwg partial sum)
 
 __device__ __forceinline__ f32x16 zero16() {
@@ -49,9 +49,31 @@ template <int N> struct LoadN<float, N> {
         }
     }
 };
+// Eight consecutive elements as they lie in memory (zeros when !ok), for loads that are to be in flight together: `arrive` on all of
+// them, then the values.  Converted where they are loaded, the compiler keeps a load next to its first use.
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+template <typename T> struct Raw8 {
+    static constexpr int Q = sizeof(T) / 2;
+    f32x4 q[Q];
+    __device__ __forceinline__ void load(const T* p, bool ok) {
+        const f32x4* src = reinterpret_cast<const f32x4*>(ok ? p : reinterpret_cast<const T*>(g_gate_zeros));
+#pragma unroll
+        for (int i = 0; i < Q; ++i) q[i] = src[i];
+    }
+    __device__ __forceinline__ void arrive() {
+#pragma unroll
+        for (int i = 0; i < Q; ++i) asm volatile("" : "+v"(q[i]));
+    }
+    __device__ __forceinline__ float value(int i) const {
+        if constexpr (Q == 2) return q[i >> 2][i & 3];
+        else {
+            typedef __attribute__((ext_vector_type(8))) T t8;
+            return (float)__builtin_bit_cast(t8, q[0])[i];
+        }
+    }
+};
 // All of v[] has arrived before anything behind this point runs: keeps the scheduler from sinking each
 // load next to its first use (which would pay one memory latency per load instead of one per batch).
-typedef __attribute__((ext_vector_type(4))) float f32x4;
 template <int N> __device__ __forceinline__ void arrive(float (&v)[N][4]) {
     static_assert(N == 8 || N == 16, "batches of 8 or 16");
     f32x4 w[N];

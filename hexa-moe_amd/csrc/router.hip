@@ -23,9 +23,9 @@ constexpr int ROUTER_TB = 64;   // tokens (= lanes) per workgroup of the softmax
 constexpr int ROUTER_LDS_E = 240;   // up to this many experts the workgroup's 64 x E tile is staged in LDS
 
 // insertion of (cv, ci) into a descending list of k entries; strict '>' keeps the lower index on ties
-__device__ __forceinline__ void topk_insert(float (&best_v)[MAX_TOPK], int (&best_i)[MAX_TOPK], int k, float cv, int ci) {
+template <int N> __device__ __forceinline__ void topk_insert(float (&best_v)[N], int (&best_i)[N], int k, float cv, int ci) {
 #pragma unroll
-    for (int j = 0; j < MAX_TOPK; ++j) {
+    for (int j = 0; j < N; ++j) {
         if (j < k && cv > best_v[j]) {
             const float tv = best_v[j]; const int ti = best_i[j];
             best_v[j] = cv; best_i[j] = ci; cv = tv; ci = ti;
@@ -121,10 +121,130 @@ __host__ __device__ constexpr size_t router4_lds_floats(int E, int k, bool hist,
 struct LiK { float* thr; const float* noise; float noise_scale, inv_sigma; };
 __device__ __forceinline__ float normal_cdf(float z) { return 0.5f * erfcf(-z * 0.70710678118654752f); }
 
+// A lane's experts q, q + 4, ...: f(i, e) for each below E -- N of them at most, unrolled (the values can stay in registers), or any number
+// (N = 0)
+template <int N, typename F> __device__ __forceinline__ void lane_experts(int q, int E, F&& f) {
+    if constexpr (N > 0) {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            if (q + ROUTER_G * i < E) f(i, q + ROUTER_G * i);
+    } else {
+        for (int e = q; e < E; e += ROUTER_G) f(0, e);
+    }
+}
+
+// Softmax, top-k, loss and histogram of one token by its four lanes.  N: see lane_experts; KMAX: the longest list.  (144 tokens of 32 experts,
+// top-1: 7000 cycles with the values in LDS between the passes and lists of eight, 3400 so.)
+template <bool LI, int N, int KMAX>
+__device__ __forceinline__ void router4_rows(const Router4Lds& L, int32_t* __restrict__ idx, bool hist, int t0, int rows, int E, int k, const LiK& li) {
+    constexpr bool REGS = N > 0;
+    constexpr int NV = REGS ? N : 1;
+    const int tid = threadIdx.x, r = tid >> 2, q = tid & 3;
+    const int t = t0 + r;
+    const bool ok = r < rows;
+    float* row = L.tile + r * L.P;
+    float v[NV];
+    // The selection is total: a row of NaN scores (NaN or +Inf logits) beats no entry, so the lists start out as
+    // the lanes' own experts in index order and such a token ends up with experts 0..k-1 (torch.topk also returns
+    // valid ids for NaN rows); its NaN then reaches the output through the token's own features and the loss
+    // through the score sums.
+    float bv[KMAX];
+    int bi[KMAX];
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j) { bv[j] = -INFINITY; bi[j] = q + ROUTER_G * j; }
+    // scores of the logits in `from` into `to`
+    auto softmax = [&](const float* from, float* to, auto&& each) {
+        if constexpr (REGS) lane_experts<N>(q, E, [&](int i, int e) { v[i] = from[e]; });
+        float mx = -INFINITY;
+        lane_experts<N>(q, E, [&](int i, int e) { mx = fmaxf(mx, REGS ? v[i] : from[e]); });
+        mx = fmaxf(mx, __shfl_xor(mx, 1));
+        mx = fmaxf(mx, __shfl_xor(mx, 2));
+        float sum = 0.f;
+        lane_experts<N>(q, E, [&](int i, int e) {
+            const float ex = expf((REGS ? v[i] : from[e]) - mx);
+            if (REGS) v[i] = ex;
+            else to[e] = ex;
+            sum += ex;
+        });
+        sum += __shfl_xor(sum, 1);         // (s0 + s1) + (s2 + s3) on every lane of the quad
+        sum += __shfl_xor(sum, 2);
+        const float inv = 1.0f / sum;
+        lane_experts<N>(q, E, [&](int i, int e) {
+            const float sc = (REGS ? v[i] : to[e]) * inv;
+            to[e] = sc;
+            each(e, sc);
+        });
+    };
+    if (ok) softmax(row, row, [&](int e, float sc) { topk_insert(bv, bi, k, sc, e); });   // ascending e, strict '>': the lower index stays ahead on ties
+    else lane_experts<N>(q, E, [&](int, int e) { row[e] = 0.f; });
+    // merge the four lists: k rounds, each takes the best head (greater score; lower index on ties)
+    int pick[KMAX];
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j) {
+        pick[j] = 0;
+        if (j < k) {
+            float hv = bv[0];
+            int hi = bi[0];
+#pragma unroll
+            for (int m = 1; m <= 2; m <<= 1) {
+                const float ov = __shfl_xor(hv, m);
+                const int oi = __shfl_xor(hi, m);
+                if (ov > hv || (ov == hv && oi < hi)) { hv = ov; hi = oi; }
+            }
+            pick[j] = hi;
+            if (hi == bi[0]) {
+#pragma unroll
+                for (int m = 0; m + 1 < KMAX; ++m) { bv[m] = bv[m + 1]; bi[m] = bi[m + 1]; }
+                bv[KMAX - 1] = -INFINITY;
+                bi[KMAX - 1] = 0x7fffffff;
+            }
+        }
+    }
+    if (ok) {
+#pragma unroll
+        for (int j = 0; j < KMAX; ++j)
+            if (j < k && (j & 3) == q) {
+                idx[(size_t)t * k + j] = pick[j];
+                if (hist) atomicAdd(&L.hist[j * E + pick[j]], 1);
+            }
+        if (!LI && q == 0) atomicAdd(&L.cnt[pick[0]], 1.0f);   // exact: at most 64 ones per counter
+    }
+    if (LI) {
+        float* clean = L.clean + r * L.P;
+        if (ok) {
+            int last = 0;
+#pragma unroll
+            for (int j = 0; j < KMAX; ++j)
+                if (j == k - 1) last = pick[j];
+            float thr = clean[last];
+            if (li.noise) thr += li.noise_scale * li.noise[(size_t)t * E + last];
+            if (q == 0) li.thr[t] = thr;
+            softmax(clean, row, [&](int e, float sc) { clean[e] = normal_cdf((sc - thr) * li.inv_sigma); });
+        } else {
+            lane_experts<N>(q, E, [&](int, int e) { clean[e] = 0.f; });
+        }
+    }
+}
+
+// the sum of a column of the tile in token order, its values read 32 at a time
+__device__ __forceinline__ float router4_column(const float* col, int P) {
+    float m = 0.f;
+    for (int r0 = 0; r0 < ROUTER_TB; r0 += 32) {
+        float v[32];
+#pragma unroll
+        for (int i = 0; i < 32; ++i) v[i] = col[(r0 + i) * P];
+#pragma unroll
+        for (int i = 0; i < 32; i += 8) asm volatile("" : "+v"(v[i]), "+v"(v[i + 1]), "+v"(v[i + 2]), "+v"(v[i + 3]), "+v"(v[i + 4]), "+v"(v[i + 5]), "+v"(v[i + 6]), "+v"(v[i + 7]));
+#pragma unroll
+        for (int i = 0; i < 32; ++i) m += v[i];
+    }
+    return m;
+}
+
 // Everything behind the tile of (noisy) logits: softmax, top-k, loss partials, histogram, scores out.  The tile
 // holds rows [t0, t0 + rows) of the workgroup; the counters have been cleared; a barrier separates both from here.
-// The workgroup has at least ROUTER_TB * ROUTER_G threads.
-template <bool LI>
+// The workgroup has at least ROUTER_TB * ROUTER_G threads.  FEW: E <= 64, the lanes keep their scores in registers.
+template <bool LI, bool FEW>
 __device__ __forceinline__ void router4_body(const Router4Lds& L, float* __restrict__ scores, int32_t* __restrict__ idx,
                                              float* __restrict__ part_me, float* __restrict__ part_cnt,
                                              int32_t* __restrict__ hist, int t0, int rows, int E, int k, int nblocks, const LiK& li) {
@@ -136,119 +256,24 @@ __device__ __forceinline__ void router4_body(const Router4Lds& L, float* __restr
     const size_t g0 = (size_t)t0 * E;
     const int total = rows * E;
     if (tid < ROUTER_TB * ROUTER_G) {   // four lanes per token; further wavefronts of the workgroup help with the sums only
-        const int r = tid >> 2, q = tid & 3;
-        const int t = t0 + r;
-        const bool ok = r < rows;
-        float* row = tile + r * P;
-        // The selection is total: a row of NaN scores (NaN or +Inf logits) beats no entry, so the lists start out as
-        // the lanes' own experts in index order and such a token ends up with experts 0..k-1 (torch.topk also returns
-        // valid ids for NaN rows); its NaN then reaches the output through the token's own features and the loss
-        // through the score sums.
-        float bv[MAX_TOPK];
-        int bi[MAX_TOPK];
-    #pragma unroll
-        for (int j = 0; j < MAX_TOPK; ++j) { bv[j] = -INFINITY; bi[j] = q + ROUTER_G * j; }
-        if (ok) {
-            float mx = -INFINITY;
-            for (int e = q; e < E; e += ROUTER_G) mx = fmaxf(mx, row[e]);
-            mx = fmaxf(mx, __shfl_xor(mx, 1));
-            mx = fmaxf(mx, __shfl_xor(mx, 2));
-            float sum = 0.f;
-            for (int e = q; e < E; e += ROUTER_G) {
-                const float ex = expf(row[e] - mx);
-                row[e] = ex;
-                sum += ex;
-            }
-            sum += __shfl_xor(sum, 1);         // (s0 + s1) + (s2 + s3) on every lane of the quad
-            sum += __shfl_xor(sum, 2);
-            const float inv = 1.0f / sum;
-            for (int e = q; e < E; e += ROUTER_G) {
-                const float sc = row[e] * inv;
-                row[e] = sc;
-                topk_insert(bv, bi, k, sc, e);  // ascending e, strict '>': the lower index stays ahead on ties
-            }
+        if constexpr (FEW) {
+            if (E <= 32 && k <= 2) router4_rows<LI, 8, 2>(L, idx, hist != nullptr, t0, rows, E, k, li);
+            else if (k <= 2) router4_rows<LI, 16, 2>(L, idx, hist != nullptr, t0, rows, E, k, li);
+            else router4_rows<LI, 16, MAX_TOPK>(L, idx, hist != nullptr, t0, rows, E, k, li);
         } else {
-            for (int e = q; e < E; e += ROUTER_G) row[e] = 0.f;
-        }
-        // merge the four lists: k rounds, each takes the best head (greater score; lower index on ties)
-        int pick[MAX_TOPK];
-    #pragma unroll
-        for (int j = 0; j < MAX_TOPK; ++j) {
-            pick[j] = 0;
-            if (j < k) {
-                float hv = bv[0];
-                int hi = bi[0];
-    #pragma unroll
-                for (int m = 1; m <= 2; m <<= 1) {
-                    const float ov = __shfl_xor(hv, m);
-                    const int oi = __shfl_xor(hi, m);
-                    if (ov > hv || (ov == hv && oi < hi)) { hv = ov; hi = oi; }
-                }
-                pick[j] = hi;
-                if (hi == bi[0]) {
-    #pragma unroll
-                    for (int m = 0; m + 1 < MAX_TOPK; ++m) { bv[m] = bv[m + 1]; bi[m] = bi[m + 1]; }
-                    bv[MAX_TOPK - 1] = -INFINITY;
-                    bi[MAX_TOPK - 1] = 0x7fffffff;
-                }
-            }
-        }
-        if (ok) {
-    #pragma unroll
-            for (int j = 0; j < MAX_TOPK; ++j)
-                if (j < k && (j & 3) == q) {
-                    idx[(size_t)t * k + j] = pick[j];
-                    if (hist) atomicAdd(&s_hist[j * E + pick[j]], 1);
-                }
-            if (!LI && q == 0) atomicAdd(&s_cnt[pick[0]], 1.0f);   // exact: at most 64 ones per counter
-        }
-        if (LI) {
-            float* clean = L.clean + r * P;
-            if (ok) {
-                int last = 0;
-    #pragma unroll
-                for (int j = 0; j < MAX_TOPK; ++j)
-                    if (j == k - 1) last = pick[j];
-                float thr = clean[last];
-                if (li.noise) thr += li.noise_scale * li.noise[(size_t)t * E + last];
-                if (q == 0) li.thr[t] = thr;
-                float mx = -INFINITY;
-                for (int e = q; e < E; e += ROUTER_G) mx = fmaxf(mx, clean[e]);
-                mx = fmaxf(mx, __shfl_xor(mx, 1));
-                mx = fmaxf(mx, __shfl_xor(mx, 2));
-                float sum = 0.f;
-                for (int e = q; e < E; e += ROUTER_G) {
-                    const float ex = expf(clean[e] - mx);
-                    row[e] = ex;
-                    sum += ex;
-                }
-                sum += __shfl_xor(sum, 1);
-                sum += __shfl_xor(sum, 2);
-                const float inv = 1.0f / sum;
-                for (int e = q; e < E; e += ROUTER_G) {
-                    const float sc = row[e] * inv;
-                    row[e] = sc;
-                    clean[e] = normal_cdf((sc - thr) * li.inv_sigma);
-                }
-            } else {
-                for (int e = q; e < E; e += ROUTER_G) clean[e] = 0.f;
-            }
+            router4_rows<LI, 0, MAX_TOPK>(L, idx, hist != nullptr, t0, rows, E, k, li);
         }
     }
     __syncthreads();
     // per-expert sums over the 64 tokens, in token order; the scores leave coalesced
     for (int e = tid; e < E; e += blockDim.x) {
-        float m = 0.f;
-#pragma unroll 16
-        for (int rr = 0; rr < ROUTER_TB; ++rr) m += tile[rr * P + e];
+        const float m = router4_column(tile + e, P);
         part_me[(size_t)blockIdx.x * E + e] = m;
         if (!LI) part_cnt[(size_t)blockIdx.x * E + e] = s_cnt[e];
     }
     if (LI)
         for (int e = (tid + 128) % blockDim.x; e < E; e += blockDim.x) {      // (other wavefronts than the sums above)
-            float m = 0.f;
-#pragma unroll 16
-            for (int rr = 0; rr < ROUTER_TB; ++rr) m += L.clean[rr * P + e];
+            const float m = router4_column(L.clean + e, P);
             part_cnt[(size_t)blockIdx.x * E + e] = m;
         }
     if (hist)
@@ -308,7 +333,7 @@ __global__ __launch_bounds__(ROUTER_TB * ROUTER_G) void router_fwd4_kernel(
         }
     }
     __syncthreads();
-    router4_body<LI>(L, scores, idx, part_me, part_cnt, hist, t0, rows, E, k, gridDim.x, li);
+    router4_body<LI, false>(L, scores, idx, part_me, part_cnt, hist, t0, rows, E, k, gridDim.x, li);
 }
 
 // The gate's projection and the router in one launch for 16-bit or fp32 token tensors and up to GATE_ROUTER_MAX_E
@@ -320,21 +345,37 @@ __global__ __launch_bounds__(ROUTER_TB * ROUTER_G) void router_fwd4_kernel(
 constexpr int GATE_ROUTER_MAX_E = 64;
 constexpr int GATE_ROUTER_NT = 2 * ROUTER_TB * ROUTER_G;
 //
+// A launch of few tokens is one workgroup's chain, 27500 cycles of it at 144 tokens (384 wide, 32 experts, bf16): operands 7300, products 7000 (two
+// wavefronts of a SIMD, 48 fp32 products of 64 cycles each), partial sums and logits 2500, softmax and lists 3400, the rest merge, sums
+// over the tokens and stores.  wg is the same for every workgroup, and a lane that reads its own row of it fetches 16 bytes of 32 lines an
+// instruction: a trip's 24 pieces of 16 bytes of every row come by asynchronous copy, whole lines at a time, into LDS for the two token
+// blocks.  The token rows, half the bytes and nobody else's, go to registers, all of a trip's loads in flight.  The partial sums take the
+// operands' place in LDS.  Against both operands read by the lanes, a sixth of them in flight at once, and the scores in LDS between the passes
+// with lists of eight: 13.4 -> 11.4 us there, 14.6 -> 12.2 at 2304 tokens, 21.3 -> 19.6 at 18432, 81 -> 71 at 32768 tokens, 1024 wide, 64 experts;
+// fp32 tokens of 8 experts 14.4, 14.7.  Beside workgroups that round (38 to 75 million weights), whose traffic makes every trip to memory
+// longer: 34.5 -> 26.4 at 9216 fp32 tokens, 39 -> 33 at 3600, 768 wide, 43 -> 34 at 18432.
+//
 // Workgroups past the routing ones round fp32 master weights to 16 bits (`round`): the routing workgroups are a chain of
 // latencies that leaves the memory idle, and these are nothing but memory traffic.  ROUND says what the launch rounds:
-// nothing, weights, or the tokens too (x_src into x); two chunks per trip then, because the registers of six would leave the
-// rounding workgroups three wavefronts per SIMD (18432 x 384 tokens: 46 us instead of 43.8).
+// nothing, weights, or the tokens too (x_src into x).
 constexpr int ROUND_NONE = 0, ROUND_WEIGHTS = 1, ROUND_TOKENS = 2;
+constexpr int GR_PIECES = 4 * FWD_NB;                                    // 16-byte pieces of a wg row in a trip
+constexpr int GR_QUARTER = 32 * GR_PIECES * 16, GR_BYTES = 4 * GR_QUARTER;   // of the four quarters of the model dimension
+static_assert(GR_BYTES >= 2 * 4 * 16 * 64 * 4, "the partial sums fit in the operands' place");
+static_assert(GR_QUARTER % 2048 == 0, "copies of 1 KB, half of them by either token block's wavefront");
+// piece p of row r sits in slot (p + r / 2) of its row: rows are 24 slots apart, 16 lanes read 16 different groups of four banks
+__device__ __forceinline__ int gr_turn(int row) { return (row & 15) >> 1; }
 template <typename T, bool LI, int ROUND>
-__global__ __launch_bounds__(GATE_ROUTER_NT) void gate_router_kernel(
+__global__ __launch_bounds__(GATE_ROUTER_NT, 4) void gate_router_kernel(
     float* __restrict__ logits, float* __restrict__ scores, int32_t* __restrict__ idx, float* __restrict__ part_me,
     float* __restrict__ part_cnt, std::conditional_t<ROUND == ROUND_TOKENS, T, const T>* __restrict__ x, const float* __restrict__ x_src,
     const float* __restrict__ wg, const float* __restrict__ noise,
     float noise_scale, int num_tokens, int d, int E, int k, int32_t* __restrict__ hist, int nblocks, LiK li, RoundAllK round) {
     extern __shared__ float sh[];
-    __shared__ float part[2][4][16][64];             // [token block][quarter of d][result register][lane]
+    __shared__ __attribute__((aligned(1024))) char operands[GR_BYTES];
+    float (*part)[4][16][64] = reinterpret_cast<float (*)[4][16][64]>(operands);    // [token block][quarter of d][result register][lane]
     constexpr bool SRC32 = ROUND == ROUND_TOKENS;
-    constexpr int NB = SRC32 ? 2 : FWD_NB;
+    constexpr int NB = FWD_NB;
     if (ROUND != ROUND_NONE && (int)blockIdx.x >= nblocks) {
         round_all_body(round, blockIdx.x - nblocks);
         return;
@@ -357,39 +398,74 @@ __global__ __launch_bounds__(GATE_ROUTER_NT) void gate_router_kernel(
     const int c0 = (chunks * quarter) >> 2, c1 = (chunks * (quarter + 1)) >> 2;
     const bool tok_ok = t0 + 32 * blk + r < num_tokens;
     const size_t xat = (size_t)(tok_ok ? t0 + 32 * blk + r : 0) * d;
-    const T* xrow = x + xat;
+    using X = std::conditional_t<SRC32, float, T>;   // what is read
+    const X* xrow;
+    if constexpr (SRC32) xrow = x_src + xat;
+    else xrow = x + xat;
+    const char* const mine = operands + quarter * GR_QUARTER;
     for (int e0 = 0; e0 < E; e0 += 32) {
         const bool exp_ok = e0 + r < E;
-        const float* wrow = wg + (size_t)(exp_ok ? e0 + r : 0) * d;
         f32x16 acc = zero16();
-        for (int c = c0; c < c1; c += NB) {
-            float xv[NB][8], wv[NB][8];
+        for (int c = 0; c < (chunks + 3) >> 2; c += NB) {            // (the quarters are of one length, or one chunk shorter)
+            if (c > 0) __syncthreads();                              // the trip before has been read
+            int ln = lane;               // (addresses worked out in every trip, not kept over all of them)
+            asm volatile("" : "+v"(ln));
+            const int r = ln & 31, h = ln >> 5;
+            // this wavefront's half of its quarter's rows of wg, and its own token rows
+#pragma unroll
+            for (int i = 0; i < GR_QUARTER / 2048; ++i) {
+                const int at = (blk * (GR_QUARTER / 2048) + i) * 64 + ln, row = at / GR_PIECES, slot = at - row * GR_PIECES;
+                int p = slot - gr_turn(row);
+                if (p < 0) p += GR_PIECES;
+                const int col = (c0 + c) * 16 + p * 4;
+                if (e0 + row >= E) continue;         // (those columns of the logits are nobody's)
+                const bool ok = c0 + c + (p >> 2) < c1 && col < d;
+                const float* src = ok ? wg + (size_t)(e0 + row) * d + col : reinterpret_cast<const float*>(g_gate_zeros);
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                                 (__attribute__((address_space(3))) void*)(operands + quarter * GR_QUARTER + (blk * (GR_QUARTER / 2048) + i) * 1024), 16, 0, 0);
+            }
+            Raw8<X> xv[NB];
 #pragma unroll
             for (int u = 0; u < NB; ++u) {
-                const int piece = 2 * (c + u) + h;
-                const bool ok = c + u < c1 && piece < pieces;
-                if constexpr (SRC32) LoadN<float, 8>::run(x_src + xat + (ok ? piece : 0) * 8, ok && tok_ok, xv[u]);
-                else LoadN<T, 8>::run(xrow + (ok ? piece : 0) * 8, ok && tok_ok, xv[u]);
-                LoadN<float, 8>::run(wrow + (ok ? piece : 0) * 8, ok && exp_ok, wv[u]);
+                const int piece = 2 * (c0 + c + u) + h;
+                const bool ok = c0 + c + u < c1 && piece < pieces;
+                xv[u].load(xrow + (ok ? piece : 0) * 8, ok && tok_ok);
             }
-            if constexpr (SRC32) {      // every piece of the workgroup's rows is some lane's once per block of experts
 #pragma unroll
-                for (int u = 0; u < NB; ++u) {
-                    const int piece = 2 * (c + u) + h;
+            for (int u = 0; u < NB; ++u) xv[u].arrive();
+            __syncthreads();                                         // (every copy has landed, too)
+            f32x4 b[2][2];               // a chunk's values of wg, read while the chunk before it is multiplied
+            auto read = [&](int u) {
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    int slot = 4 * u + 2 * h + q + gr_turn(r);
+                    if (slot >= GR_PIECES) slot -= GR_PIECES;
+                    b[u & 1][q] = *reinterpret_cast<const f32x4*>(mine + (r * GR_PIECES + slot) * 16);
+                }
+            };
+            read(0);
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+                if (u + 1 < NB) read(u + 1);
+                asm volatile("" ::: "memory");       // (no further ahead: their registers)
+                float a[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) a[i] = xv[u].value(i);
+                if constexpr (SRC32) {      // every piece of the workgroup's rows is some lane's once per block of experts
+                    const int piece = 2 * (c0 + c + u) + h;
                     union { uint4 q; T t[8]; } o;
 #pragma unroll
                     for (int i = 0; i < 8; ++i) {
-                        o.t[i] = (T)xv[u][i];
-                        xv[u][i] = (float)o.t[i];
+                        o.t[i] = (T)a[i];
+                        a[i] = (float)o.t[i];
                     }
-                    if (e0 == 0 && c + u < c1 && piece < pieces && tok_ok) *reinterpret_cast<uint4*>(x + xat + (size_t)piece * 8) = o.q;
+                    if (e0 == 0 && c0 + c + u < c1 && piece < pieces && tok_ok) *reinterpret_cast<uint4*>(x + xat + (size_t)piece * 8) = o.q;
                 }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[u & 1][i >> 2][i & 3], acc, 0, 0, 0);
             }
-#pragma unroll
-            for (int u = 0; u < NB; ++u)
-#pragma unroll
-                for (int i = 0; i < 8; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xv[u][i], wv[u][i], acc, 0, 0, 0);
         }
+        __syncthreads();                                             // the operands have been read
 #pragma unroll
         for (int v = 0; v < 16; ++v) part[blk][quarter][v][lane] = acc[v];
         __syncthreads();
@@ -428,7 +504,7 @@ __global__ __launch_bounds__(GATE_ROUTER_NT) void gate_router_kernel(
         }
     }
     __syncthreads();
-    router4_body<LI>(L, scores, idx, part_me, part_cnt, hist, t0, rows, E, k, nblocks, li);
+    router4_body<LI, true>(L, scores, idx, part_me, part_cnt, hist, t0, rows, E, k, nblocks, li);
 }
 
 // The GShard loss from the workgroup partials (see small_bodies.h) as a launch of its own.
