@@ -94,7 +94,7 @@ bool hexa::esmm_slot_sum_takes_extra(const int32_t* route, int w_layout, int T, 
 int hexa::esmm_call(void* out, const void* x, const void* w, const void* bias, const int32_t* route, int m2s,
                     int w_layout, int accumulate, int T, int k, int in_dim, int out_dim, int E, int x_dt, int w_dt,
                     int bias_dt, int out_dt, int act, void* out_act, void* slot_ws, const void* sum_extra,
-                    bool* extra_used, void* stream, bool careful) {
+                    bool* extra_used, void* stream, bool careful, bool act_only) {
     if (extra_used) *extra_used = false;
     if (int rc = check_sizes("hexa_esmm", T, k, E, in_dim, out_dim)) return rc;
     if (!out || !x || !w || !route) HEXA_FAIL(HEXA_ERR_ARG, "hexa_esmm: null pointer");
@@ -114,7 +114,7 @@ int hexa::esmm_call(void* out, const void* x, const void* w, const void* bias, c
     a.out_per_slot = m2s ? 0 : 1;
     a.w_layout = w_layout; a.accumulate = accumulate ? 1 : 0;
     a.x_dt = x_dt; a.w_dt = w_dt; a.bias_dt = bias_dt; a.out_dt = out_dt; a.act = act;
-    a.careful = careful;
+    a.careful = careful; a.act_only = act_only && act == HEXA_ACT_GELU;
     hipStream_t st = (hipStream_t)stream;
     if (x_dt == HEXA_F32) {
         if (w_dt != HEXA_F32 || out_dt != HEXA_F32 || (bias && bias_dt != HEXA_F32))

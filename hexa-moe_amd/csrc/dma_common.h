@@ -348,6 +348,7 @@ struct EsmmK {
     int x_slot_rows, out_slot_rows;
     int accumulate, bias_dt, out_dt, act, group;
     int careful;      // see EsmmArgs::careful
+    int act_only;     // see EsmmArgs::act_only
     int stream_out;   // results are stored with the streaming (non-temporal) hint
     long total;
     void* ws;   // slots > 0 write here ([slot-1][T][N]) when set: the slots are summed afterwards

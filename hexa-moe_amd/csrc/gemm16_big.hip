@@ -35,7 +35,7 @@ constexpr int BIG_ROW_RUN = 4;         // row tiles that are walked together, co
 struct BigK {
     const void* x; const void* w; const void* bias; void* out; void* out_act; void* ws; float* colsum;
     const int32_t* token_ids; const int32_t* offsets;
-    int T, K, N, E, nslots, ntn, x_per_slot, out_per_slot, bias_dt, stream_out;
+    int T, K, N, E, nslots, ntn, x_per_slot, out_per_slot, bias_dt, stream_out, act_only;
     int wg_per_xcd;       // workgroups per XCD (grid = 8 * wg_per_xcd)
 };
 
@@ -77,8 +77,10 @@ __device__ __forceinline__ void global_store128(char* at, u32x4 v, bool streamin
 }
 
 // a copy's wait: at most N (and EXTRA stores, where `lax`) younger operations may be outstanding
-template <int N, int EXTRA> __device__ __forceinline__ void wait_copies(bool more, bool lax) {
+// (half: where only the activation is stored, half as many of them)
+template <int N, int EXTRA, bool HALVES> __device__ __forceinline__ void wait_copies(bool more, bool lax, bool half) {
     if (!more) wait_vmcnt<0>();
+    else if (HALVES && lax && half) wait_vmcnt<N + EXTRA / 2>();
     else if (lax) wait_vmcnt<N + EXTRA>();
     else wait_vmcnt<N>();
 }
@@ -98,6 +100,7 @@ __global__ __launch_bounds__(512, 2) void esmm16_big_kernel(BigK p) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave >> 2, wf = wave & 3;
     const int K = p.K, N = p.N, nk = TAIL ? K / BK + 1 : K / BK;
     const bool streaming = p.stream_out != 0;
+    const bool act_only = ACT == HEXA_ACT_GELU && p.act_only != 0;
 
     // An expert's rows are its lists of all slots, one behind the other: half a tile of its last 256 is empty on average, not half
     // a tile of each list's.  First tile of every expert:
@@ -385,7 +388,7 @@ __global__ __launch_bounds__(512, 2) void esmm16_big_kernel(BigK p) {
             readB(I0(), b0);
             readB(I1(), b1);
             if (more) { issueA(1); next_stage(); }
-            wait_copies<8, STORES>(more, lax);
+            wait_copies<8, STORES, ACT == HEXA_ACT_GELU>(more, lax, act_only);
             lds_wait();
             pinA(); pinB(b0); pinB(b1);
             barrier_nofence();
@@ -399,7 +402,7 @@ __global__ __launch_bounds__(512, 2) void esmm16_big_kernel(BigK p) {
                 if (r + 1 < ntiles) fetch_meta(r + 1);
                 if (COLSUM && r > 0) write_colsum();
             }
-            wait_copies<8, STORES>(more, lax);
+            wait_copies<8, STORES, ACT == HEXA_ACT_GELU>(more, lax, act_only);
             lax = false;
             lds_wait();
             pinA();
@@ -516,7 +519,7 @@ __global__ __launch_bounds__(512, 2) void esmm16_big_kernel(BigK p) {
                 for (int qq = 0; qq < PASSES; ++qq) {
                     const int q = q0 + qq;
                     u32x4 x = val[qq], v = x;
-                    if (ACT != HEXA_ACT_GELU_BWD) store(q, x);
+                    if (ACT != HEXA_ACT_GELU_BWD && !act_only) store(q, x);
                     if (ACT != HEXA_ACT_NONE) {
                         // the activation of the value as stored (rounded): GELU of the result, or GELU' of y1 as a factor of it
                         const u32x4 arg = ACT == HEXA_ACT_GELU ? x : y[b & 1][q];
@@ -645,7 +648,7 @@ int launch_esmm16_big(const EsmmArgs& a, hipStream_t st) {
     pk.T = a.r.T; pk.K = a.in_dim; pk.N = a.out_dim; pk.E = a.r.E; pk.nslots = a.r.k;
     pk.ntn = div_up(a.out_dim, 256);
     pk.x_per_slot = a.x_per_slot; pk.out_per_slot = a.out_per_slot;
-    pk.bias_dt = a.bias_dt; pk.stream_out = option(OPT_ESMM_STREAM) != 2;
+    pk.bias_dt = a.bias_dt; pk.stream_out = option(OPT_ESMM_STREAM) != 2; pk.act_only = a.act_only;
     pk.ws = (!a.out_per_slot && a.r.k > 1) ? a.slot_ws : nullptr;
     const long total_ub = big_tiles_ub(a);
     if (total_ub == 0) return HEXA_OK;

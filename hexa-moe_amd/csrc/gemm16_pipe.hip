@@ -525,7 +525,7 @@ __global__ __launch_bounds__(C::NT + 64 * (PIPE_COPY_WAVES + PIPE_STORE_WAVES)) 
             global_store128(outb, 2 * boff + 16, u32x4{__float_as_uint(lo16<TC>(vw[2])), __float_as_uint(hi16<TC>(vw[2])), __float_as_uint(lo16<TC>(vw[3])), __float_as_uint(hi16<TC>(vw[3]))}, streaming);
             return;
         }
-        global_store128(outb, boff, u32x4{vw[0], vw[1], vw[2], vw[3]}, streaming);
+        if (ACT != HEXA_ACT_GELU || !p.act_only) global_store128(outb, boff, u32x4{vw[0], vw[1], vw[2], vw[3]}, streaming);
         if (COLSUM) {
 #pragma unroll
             for (int u = 0; u < 4; ++u) { cs[2 * u] += lo16<TC>(vw[u]); cs[2 * u + 1] += hi16<TC>(vw[u]); }
@@ -710,7 +710,7 @@ int launch_esmm16_pipe(const EsmmArgs& a, hipStream_t st) {
     p.x_slot_rows = a.x_per_slot ? a.r.T : 0;
     p.out_slot_rows = a.out_per_slot ? a.r.T : 0;
     p.bias_dt = a.bias_dt; p.out_dt = a.out_dt; p.act = a.act;
-    p.stream_out = option(OPT_ESMM_STREAM) != 2; p.colsum = a.colsum; p.group = 0; p.accumulate = a.accumulate;
+    p.stream_out = option(OPT_ESMM_STREAM) != 2; p.colsum = a.colsum; p.group = 0; p.accumulate = a.accumulate; p.act_only = a.act_only;
     p.ws = (!a.out_per_slot && a.r.k > 1) ? a.slot_ws : nullptr;
     p.slot_begin = 0; p.nslots = a.r.k;
     p.total = (long)p.nslots * p.mt_ub * p.ntn;

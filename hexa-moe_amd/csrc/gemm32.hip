@@ -293,7 +293,7 @@ struct Esmm32K {
     const int32_t* token_ids; const int4* tile_info; const int32_t* tile_count;
     int T, K, N, mt_ub, ntn, slot_begin, nslots;
     int x_slot_rows, out_slot_rows;
-    int accumulate, act;
+    int accumulate, act, act_only;
 };
 
 template <bool W_IN_OUT, bool BIG, typename C>
@@ -414,7 +414,7 @@ __global__ __launch_bounds__(C::NT, C::WAVES) void esmm32_kernel(Esmm32K p) {
                     const float4 old = *dst;
                     v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
                 }
-                *dst = v;
+                if (!p.act_only) *dst = v;
                 if (p.act == HEXA_ACT_GELU)
                     *reinterpret_cast<float4*>(p.out_act + off) = make_float4(gelu_full(v.x), gelu_full(v.y), gelu_full(v.z), gelu_full(v.w));
             }
@@ -613,7 +613,7 @@ int launch_esmm32(const EsmmArgs& a, hipStream_t st) {
     p.T = a.r.T; p.K = a.in_dim; p.N = a.out_dim; p.mt_ub = a.r.mt_ub;
     p.x_slot_rows = a.x_per_slot ? a.r.T : 0;
     p.out_slot_rows = a.out_per_slot ? a.r.T : 0;
-    p.act = a.act;
+    p.act = a.act; p.act_only = a.act_only;
     // Summing the slots into one result: with scratch every slot runs in one launch (slot 0 into `out`, the others into
     // the scratch) and a small kernel adds them; without, one launch per slot adds into `out`.
     const bool sum = !a.out_per_slot && a.r.k > 1;

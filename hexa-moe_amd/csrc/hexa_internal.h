@@ -64,6 +64,7 @@ struct EsmmArgs {
     // slots (see esmm16_slot_by_slot): they once ran on the general kernels, which do the same (relative error of y against
     // fp64, 2657 tokens, d 184, top-2, bf16: 2.95e-3; with the rounded product 3.64e-3).
     bool careful = false;
+    bool act_only = false;   // with HEXA_ACT_GELU: nobody reads `out`, kernels may leave it unwritten (the general ones do not)
     bool wide = false;   // the result, rounded to out_dt, is stored as fp32 (pipelined kernel only, see esmm16_wide_supported)
     // optional, with slot_ws on the fast path: one more tensor of the result's shape added by the slot sum
     const void* sum_extra = nullptr;
@@ -90,7 +91,8 @@ struct EssArgs {
 
 int esmm_call(void* out, const void* x, const void* w, const void* bias, const int32_t* route, int m2s, int w_layout,
               int accumulate, int T, int k, int in_dim, int out_dim, int E, int x_dt, int w_dt, int bias_dt, int out_dt,
-              int act, void* out_act, void* slot_ws, const void* sum_extra, bool* extra_used, void* stream, bool careful = false);
+              int act, void* out_act, void* slot_ws, const void* sum_extra, bool* extra_used, void* stream, bool careful = false,
+              bool act_only = false);
 int esmm_gelu_bwd_ess_call(void* out, void* db, const void* x, const void* w, const void* y1, const int32_t* route, int w_layout,
                            int db_accumulate, int T, int k, int in_dim, int out_dim, int E, int x_dt, int w_dt, int db_dt, float* ws,
                            int64_t ws_floats, void* stream, bool careful);

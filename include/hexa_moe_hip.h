@@ -306,6 +306,7 @@ typedef struct hexa_moe_depth_opts {
     int32_t careful;   /* 1: GELU, GELU' and the sums into y and dx take the fp32 product, not the one rounded to act_dt (top_k > 1:
                         * with workspaces that hold an fp32 result of every slot) */
     int32_t no_gate;   /* 1: wg is NULL in every call, and the workspaces leave the router's and the gate's share out */
+    int32_t no_y1;     /* 1: no backward will read y1; a forward of both layers may leave the buffer unwritten */
 } hexa_moe_depth_opts;
 
 /* Which parts of the depth a call runs (0: all of them).  With an activation that the kernels do not fuse, the caller
