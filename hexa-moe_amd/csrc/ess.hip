@@ -100,7 +100,7 @@ __global__ __launch_bounds__(256) void sum_slots_kernel(SumSlotsK p) { sum_slots
 
 template <typename T>
 int launch_sum_slots_t(SumSlotsK p, int dt, hipStream_t st) {
-    if (p.n == 0 || (p.nws == 0 && !p.extra)) return HEXA_OK;
+    if (p.n == 0 || (p.nws == 0 && !p.extra && !p.wide)) return HEXA_OK;
     if ((p.offsets ? p.N : p.n) % Vec16<T>::N) HEXA_FAIL(HEXA_ERR_UNSUPPORTED, "sum_slots: rows must be multiples of the vector width");
     int64_t blocks = (p.n / Vec16<T>::N + 255) / 256;
     if (blocks > 256 * 16) blocks = 256 * 16;
@@ -121,10 +121,11 @@ static int launch_sum_slots_d(const SumSlotsK& p, int dt, hipStream_t st) {
     return dt == HEXA_BF16 ? launch_sum_slots_t<__bf16>(p, dt, st) : launch_sum_slots_t<_Float16>(p, dt, st);
 }
 int launch_sum_slots(void* out, const void* ws, const RouteView& r, int N, bool accumulate, int dt, hipStream_t st, const void* extra) {
-    return launch_sum_slots_d(SumSlotsK{out, ws, (int64_t)r.T * N, r.k - 1, extra, 0, r.offsets, r.token_ids, r.T, r.E, N, accumulate ? 1 : 0}, dt, st);
+    return launch_sum_slots_d(SumSlotsK{out, ws, (int64_t)r.T * N, r.k - 1, extra, 0, r.offsets, r.token_ids, r.T, r.E, N, accumulate ? 1 : 0, nullptr}, dt, st);
 }
-int launch_add(void* out, const void* extra, int64_t n, int dt, hipStream_t st) {
-    return launch_sum_slots_d(SumSlotsK{out, nullptr, n, 0, extra, 0, nullptr, nullptr, 0, 0, 0, 1}, dt, st);
+int launch_add(void* out, const void* extra, int64_t n, int dt, hipStream_t st, float* wide) {
+    if (wide && dt == HEXA_F32) HEXA_FAIL(HEXA_ERR_UNSUPPORTED, "add: only a 16-bit sum is widened");
+    return launch_sum_slots_d(SumSlotsK{out, nullptr, n, 0, extra, 0, nullptr, nullptr, 0, 0, 0, 1, wide}, dt, st);
 }
 
 // out = the fp32 results of every slot, and `extra` (may be null), added in that order and rounded once.  A wavefront per row; rows

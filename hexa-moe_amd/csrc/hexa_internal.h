@@ -167,7 +167,8 @@ int launch_sum_slots(void* out, const void* ws, const RouteView& r, int N, bool 
 // out [T][N] (16-bit) = the slots' fp32 results in ws ([k][T][N]) + extra (of out's type, may be null), rounded once
 constexpr int WIDE_SLOTS_MAX = 32;
 int launch_sum_wide_slots(void* out, const float* ws, const void* extra, const RouteView& r, int N, int dt, hipStream_t s);
-int launch_add(void* out, const void* extra, int64_t n, int dt, hipStream_t s);   // out += extra
+// out += extra (may be null); where `wide` is set the rounded sum goes there as fp32 instead (16-bit out)
+int launch_add(void* out, const void* extra, int64_t n, int dt, hipStream_t s, float* wide = nullptr);
 // routing front end of the depth call: the router also counts, the counting sort's scan launch also finishes the loss,
 // its scatter launch also makes the ESTMM plan (see router.hip, route.hip)
 bool router_hist_supported(int E);

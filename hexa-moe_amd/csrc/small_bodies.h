@@ -311,7 +311,16 @@ __device__ __forceinline__ void sum_slots_body(const SumSlotsK& p, int block) {
         if (__any(len != p.T)) return sum_listed_slots<T>(p, block);
 #pragma unroll
         for (int j = 0; j < V; ++j) o.e[j] = Cvt<T>::from_f(acc[j]);
-        if (i0 + lane < nv) reinterpret_cast<uint4*>(out)[i] = o.u;
+        if (i0 + lane >= nv) continue;
+        if constexpr (V == 8) {
+            if (p.wide) {
+                float4* const to = reinterpret_cast<float4*>(p.wide + i * V);
+                to[0] = make_float4(Cvt<T>::to_f(o.e[0]), Cvt<T>::to_f(o.e[1]), Cvt<T>::to_f(o.e[2]), Cvt<T>::to_f(o.e[3]));
+                to[1] = make_float4(Cvt<T>::to_f(o.e[4]), Cvt<T>::to_f(o.e[5]), Cvt<T>::to_f(o.e[6]), Cvt<T>::to_f(o.e[7]));
+                continue;
+            }
+        }
+        reinterpret_cast<uint4*>(out)[i] = o.u;
     }
 }
 

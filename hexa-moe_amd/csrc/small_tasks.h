@@ -32,6 +32,7 @@ struct SumSlotsK {
     void* out; const void* ws; int64_t n; int nws; const void* extra; int blocks;
     const int32_t* offsets; const int32_t* token_ids;    // of the route (null: every row of every addend was written)
     int T, E, N, accumulate;                             // N: row width; accumulate: out held something before the products
+    float* wide;                                         // where set, the rounded sum goes here as fp32 and out stays as it is (no lists)
 };
 struct GateBwdK { void* dx; float* part; const float* dl; const void* x; const float* wg; int T, d, E, ntasks; };
 struct DwgReduceK { float* dwg; const float* part; int nparts; long n4; };

@@ -41,7 +41,7 @@ class DepthDesc(ctypes.Structure):
 
 class DepthOpts(ctypes.Structure):
     """hexa_moe_depth_opts of include/hexa_moe_hip.h."""
-    _fields_ = [(n, ctypes.c_int32) for n in ("size", "part", "wide_y", "careful", "no_gate", "no_y1")]
+    _fields_ = [(n, ctypes.c_int32) for n in ("size", "part", "wide_y", "careful", "no_gate", "no_y1", "wide_dx")]
 
 
 # name -> (restype, argtypes); kept in one table so the export test can walk it

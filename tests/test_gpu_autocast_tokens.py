@@ -77,3 +77,31 @@ def test_against_fp64(dev, dtype, T, d, E, k):
     names = ("y", "dx", "dwg", "dW1", "dW2", "db1", "db2")
     errs = {n: rel_err(a.grad if n != "y" else a, b)[0] for n, a, b in zip(names, [y, x] + params, [y_ref] + grads)}
     assert all(e <= most for e in errs.values()), errs
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,d,h,E,aux", [
+    (9216, 384, 1536, 32, True), (9216, 384, 1536, 32, False),     # shared launches; without the gate's share nothing else passes over dx
+    (100, 384, 1536, 32, True), (301, 264, 1000, 5, True),         # the gate's share first and dx onto it
+    (3700, 768, 3072, 8, True), (3700, 768, 3072, 8, False),       # separate launches
+    (1, 8, 16, 4, True), (33, 40, 264, 6, False),
+])
+def test_dx_leaves_as_fp32(dev, dtype, T, d, h, E, aux):
+    """The pass that finishes dx widens it: what it stores is the 16-bit value, and what tokens rounded beforehand get."""
+    from hexa_moe import moe as hmoe
+    print(f"dx as fp32: T={T} {d} -> {h} E={E} aux={aux} {dtype}", flush=True)
+    torch.manual_seed(5)
+    m = hmoe.MoE_Cascaded(gate_type={"type": "top", "k": 1, "gate_noise": 0.0, "fp32_gate": True}, model_dim_list=[d], moe_idx_list=[0],
+                          mlp_ratio=h / d, num_global_experts=E, total_depth=1, data_centric=True, activation_fn=F.gelu).to(dev)
+    for p in m.parameters():
+        torch.nn.init.uniform_(p.data, -0.08, 0.08)
+    full, dy = torch.randn(T, d, device=dev), torch.randn(T, d, device=dev).to(dtype)
+    got = []
+    for x in (full, full.to(dtype)):
+        x = x.detach().requires_grad_(True)
+        with torch.autocast("cuda", dtype=dtype):
+            y, l_aux = m(0, x)
+        torch.autograd.backward([y, l_aux] if aux else [y], [dy.to(y.dtype), torch.ones_like(l_aux)] if aux else [dy.to(y.dtype)])
+        torch.cuda.synchronize()
+        got.append(x.grad)
+    assert got[0].dtype == torch.float32 and torch.equal(got[0], got[0].to(dtype).float()) and torch.equal(got[0], got[1].float())
