@@ -179,9 +179,12 @@ int launch_sum_wide_slots(void* out, const float* ws, const void* extra, const R
 
 // out (+)= the sum of `parts` partial results of n values each, in their order
 int launch_fold(void* out, const float* ws, long n, int parts, int dt, int accumulate, hipStream_t st) {
+    // Parts of a weight gradient are bound by memory: 16 bytes of each a thread.  Bias gradients, a few hundred thousand values at most, by
+    // their latency: one value a thread keeps more of them in flight.
+    const int by4 = dt == HEXA_F32 && n % 4 == 0 && n >= ((long)1 << 19) && (((uintptr_t)out | (uintptr_t)ws) & 15) == 0;
     SmallTask f;
-    f.kind = TASK_ESS_FOLD; f.ess_fold = EssFoldK{out, ws, n, parts, dt, accumulate};
-    f.blocks = (int)((n + 255) / 256);
+    f.kind = TASK_ESS_FOLD; f.ess_fold = EssFoldK{out, ws, n, parts, dt, accumulate, by4};
+    f.blocks = by4 ? (int)((n / 4 + 255) / 256) : (int)((n + 255) / 256);
     if (!defer_task(defer_targets().ess_fold, f)) {
         hipLaunchKernelGGL(ess_fold_kernel, dim3(f.blocks), dim3(256), 0, st, f.ess_fold);
         HEXA_CHECK_LAUNCH("ess_fold");

@@ -214,6 +214,22 @@ __device__ __forceinline__ void ess_body(const EssK& p, int block) {
 
 // db (+)= ws[0] + ws[1] + ... in that order
 __device__ __forceinline__ void ess_fold_body(const EssFoldK& p, int block) {
+    if (p.by4) {
+        const long i = ((long)block * 256 + threadIdx.x) * 4;
+        if (i >= p.n) return;
+        float4 part[8], v;
+#pragma unroll
+        for (int z = 0; z < 8; ++z)
+            if (z < p.splits) part[z] = *reinterpret_cast<const float4*>(p.ws + (size_t)z * p.n + i);
+        v = part[0];
+#pragma unroll
+        for (int z = 1; z < 8; ++z)
+            if (z < p.splits) { v.x += part[z].x; v.y += part[z].y; v.z += part[z].z; v.w += part[z].w; }
+        float4* const to = reinterpret_cast<float4*>(reinterpret_cast<float*>(p.db) + i);
+        if (p.accumulate) { const float4 o = *to; v.x += o.x; v.y += o.y; v.z += o.z; v.w += o.w; }
+        *to = v;
+        return;
+    }
     const long i = (long)block * 256 + threadIdx.x;
     if (i >= p.n) return;
     // all parts' loads in flight at once (at most 8 parts), added in part order

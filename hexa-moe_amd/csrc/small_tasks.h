@@ -15,7 +15,7 @@ struct EssK {
     float* ws; int splits;   // splits > 1: workgroup z sums the z-th part of every segment into ws[z][E][N]
     int gx, gy;              // grid: (column strips, experts, splits)
 };
-struct EssFoldK { void* db; const float* ws; long n; int splits, db_dt, accumulate; };
+struct EssFoldK { void* db; const float* ws; long n; int splits, db_dt, accumulate, by4; };     // by4: 4 values a thread (fp32 db, n % 4 == 0)
 struct RouterBwdK {
     float* dlogits; const float* scores; const float* ce; const float* grad_l; int T, E;   // ce: of the importances for the load-importance loss,
     const float* thr; const int32_t* idx; const float* g_load; float inv_sigma; int k;     // which has these too (thr null: GShard loss)
