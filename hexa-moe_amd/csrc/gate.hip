@@ -69,7 +69,10 @@ __global__ __launch_bounds__(256) void gate_fwd_kernel(float* __restrict__ logit
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void gate_bwd_kernel(GateBwdK p) { gate_bwd_body<T>(p, blockIdx.x); }
+__global__ __launch_bounds__(256) void gate_bwd_kernel(GateBwdK p) {
+    __shared__ float4 sums[4 * 3 * 4 * 64];
+    gate_bwd_merged_body<T>(p, blockIdx.x, sums);
+}
 
 __global__ __launch_bounds__(256) void gate_dwg_reduce_kernel(DwgReduceK p) { dwg_reduce_body(p, blockIdx.x); }
 
@@ -80,10 +83,10 @@ GateBwdK gate_bwd_args(void* dx, bool dwg, const float* dl, const void* x, const
     const int nchunks = div_up(T, BWD_TB), groups = div_up(d, 128), eb = div_up(E, 32);
     return GateBwdK{dx, dwg ? ws : nullptr, dl, x, wg, T, d, E, nchunks * ((dx ? groups : 0) + (dwg ? groups * eb : 0))};
 }
-int launch_dwg_reduce(float* dwg, const float* ws, int T, int d, int E, hipStream_t st) {
+int launch_dwg_reduce(float* dwg, const float* ws, int T, int d, int E, hipStream_t st, bool merged) {
     SmallTask r;
     r.kind = TASK_DWG_REDUCE;
-    r.dwg_reduce = DwgReduceK{dwg, ws, div_up(T, BWD_TB), (long)E * d / 4};
+    r.dwg_reduce = DwgReduceK{dwg, ws, div_up(T, merged ? 4 * BWD_TB : BWD_TB), (long)E * d / 4, merged};
     r.blocks = (int)div_up(r.dwg_reduce.n4, 16);
     if (!defer_task(defer_targets().dwg_reduce, r)) {
         hipLaunchKernelGGL(gate_dwg_reduce_kernel, dim3(r.blocks), dim3(256), 0, st, r.dwg_reduce);
@@ -96,10 +99,11 @@ namespace {
 template <typename T>
 int gate_backward_t(void* dx, float* dwg, const float* dl, const void* x, const float* wg, int T_, int d, int E, float* ws,
                     hipStream_t st) {
-    const GateBwdK g = gate_bwd_args(dx, dwg != nullptr, dl, x, wg, T_, d, E, ws);
-    hipLaunchKernelGGL(gate_bwd_kernel<T>, dim3(div_up(g.ntasks, 4)), dim3(256), 0, st, g);
+    GateBwdK g = gate_bwd_args(dx, dwg != nullptr, dl, x, wg, T_, d, E, ws);
+    g.ntasks = g.ntasks / div_up(T_, BWD_TB) * div_up(T_, 4 * BWD_TB);
+    hipLaunchKernelGGL(gate_bwd_kernel<T>, dim3(g.ntasks), dim3(256), 0, st, g);
     HEXA_CHECK_LAUNCH("gate_bwd");
-    return dwg ? launch_dwg_reduce(dwg, ws, T_, d, E, st) : HEXA_OK;
+    return dwg ? launch_dwg_reduce(dwg, ws, T_, d, E, st, true) : HEXA_OK;
 }
 
 }  // namespace
@@ -139,7 +143,7 @@ extern "C" int hexa_gate_backward(void* dx, float* dwg, const float* dlogits, co
     if (T == 0) {   // no tokens: dwg = 0 (a reduction over zero partial sums)
         if (dwg) {
             const long n4 = (long)E * d / 4;
-            hipLaunchKernelGGL(gate_dwg_reduce_kernel, dim3((unsigned)div_up(n4, 16)), dim3(256), 0, st, DwgReduceK{dwg, dwg, 0, n4});
+            hipLaunchKernelGGL(gate_dwg_reduce_kernel, dim3((unsigned)div_up(n4, 16)), dim3(256), 0, st, DwgReduceK{dwg, dwg, 0, n4, 0});
             HEXA_CHECK_LAUNCH("gate_dwg_reduce");
         }
         return HEXA_OK;

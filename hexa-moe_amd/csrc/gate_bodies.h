@@ -169,16 +169,18 @@ __device__ __forceinline__ void gate_dx_task(int chunk, int g, T* __restrict__ d
     }
 }
 
-template <typename T>
+// `sums` (MERGED): 48 KB of LDS, in which the four wavefronts of a workgroup add their chunks' results, in chunk order, to one partial
+// result: wavefront w finishes result registers 4w .. 4w+3 of each accumulator.
+template <typename T, bool MERGED>
 __device__ __forceinline__ void gate_dwg_task(int chunk, int e_block, int g, float* __restrict__ part,
                                               const float* __restrict__ dl, const T* __restrict__ x, int num_tokens,
-                                              int d, int E) {
+                                              int d, int E, float4* sums) {
     const int lane = threadIdx.x & 63;
     const int r = lane & 31, h = lane >> 5;
     const int t0 = chunk * BWD_TB;
     const int e0 = e_block * 32;
     const bool exp_ok = e0 + r < E;
-    float* out = part + (size_t)chunk * E * d;
+    float* out = part + (size_t)(MERGED ? chunk >> 2 : chunk) * E * d;
     constexpr int TRIPS = BWD_TB / 16;      // 8 MFMA steps (16 tokens) per trip
     const int col = g * 128 + 4 * r;
     const bool col_ok = col < d;
@@ -205,7 +207,31 @@ __device__ __forceinline__ void gate_dwg_task(int chunk, int e_block, int g, flo
             for (int j = 0; j < 4; ++j)
                 acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[trip & 1][u], b[trip & 1][u][j], acc[j], 0, 0, 0);
     }
-    if (col_ok) {
+    if constexpr (MERGED) {
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        float4 mine[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 v = make_float4(acc[0][4 * w + q], acc[1][4 * w + q], acc[2][4 * w + q], acc[3][4 * w + q]);
+                if (w == wave) mine[q] = v;
+                else sums[((w * 3 + (wave < w ? wave : wave - 1)) * 4 + q) * 64 + lane] = v;       // [who finishes][whose][q]
+            }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float4* const others = sums + (wave * 3 * 4 + q) * 64 + lane;
+            float4 t = wave == 0 ? mine[q] : others[0];
+#pragma unroll
+            for (int s = 1; s < 4; ++s) {
+                const float4 v = s == wave ? mine[q] : others[(s < wave ? s : s - 1) * 4 * 64];
+                t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
+            }
+            const int e = e0 + 8 * wave + 4 * h + q;
+            if (col_ok && e < E) store4<float>(out + (size_t)e * d + col, t.x, t.y, t.z, t.w);
+        }
+    } else if (col_ok) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             const int e = e0 + 8 * (v >> 2) + 4 * h + (v & 3);
@@ -229,20 +255,49 @@ __device__ __forceinline__ void gate_bwd_body(const GateBwdK& p, int block) {
         gate_dx_task<T>(chunk, role, reinterpret_cast<T*>(p.dx), p.dl, p.wg, p.T, p.d, p.E);
     } else {
         const int q = role - n_dx;
-        gate_dwg_task<T>(chunk, q / groups, q - (q / groups) * groups, p.part, p.dl, reinterpret_cast<const T*>(p.x), p.T, p.d,
-                         p.E);
+        gate_dwg_task<T, false>(chunk, q / groups, q - (q / groups) * groups, p.part, p.dl, reinterpret_cast<const T*>(p.x), p.T, p.d,
+                                p.E, nullptr);
     }
 }
 
-// dwg = sum of the partial results, in a fixed order: a workgroup takes 16 float4 columns; each of its
+// The same products where a workgroup's four wavefronts take the same task of four chunks, one after the other, and leave one partial dwg for
+// them (p.ntasks: workgroups).  At 32768 tokens, 1024 wide, 64 experts the partial results of single chunks are 134 MB, written
+// here and read by the fold.
+template <typename T>
+__device__ __forceinline__ void gate_bwd_merged_body(const GateBwdK& p, int block, float4* sums) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int groups = (p.d + 127) >> 7, e_blocks = (p.E + 31) >> 5;
+    const int n_dx = p.dx ? groups : 0, n_dwg = p.part ? groups * e_blocks : 0;
+    const int four = block / (n_dx + n_dwg), role = block - four * (n_dx + n_dwg), chunk = four * 4 + wave;
+    if (role < n_dx) {
+        gate_dx_task<T>(chunk, role, reinterpret_cast<T*>(p.dx), p.dl, p.wg, p.T, p.d, p.E);
+    } else {
+        const int q = role - n_dx;
+        gate_dwg_task<T, true>(chunk, q / groups, q - (q / groups) * groups, p.part, p.dl, reinterpret_cast<const T*>(p.x), p.T, p.d, p.E, sums);
+    }
+}
+
+// dwg = sum of the partial results, in a fixed order, the same whether a kernel added four chunks each or left them apart: a workgroup takes 16 float4 columns; each of its
 // 16 thread groups sums a contiguous range of the partials, then the 16 group sums are added in order.
 __device__ __forceinline__ void dwg_reduce_body(const DwgReduceK& p, int block) {
     __shared__ float4 sums[16][16];
     const int c = threadIdx.x & 15, grp = threadIdx.x >> 4;
     const long i = (long)block * 16 + c;
-    const int b0 = (int)((long)p.nparts * grp / 16), b1 = (int)((long)p.nparts * (grp + 1) / 16);
+    const int sums_of_four = p.merged ? p.nparts : (p.nparts + 3) / 4;
+    const int b0 = (int)((long)sums_of_four * grp / 16), b1 = (int)((long)sums_of_four * (grp + 1) / 16);
     float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (i < p.n4) {
+    if (i < p.n4 && !p.merged) {
+#pragma unroll 2
+        for (int b = b0; b < b1; ++b) {
+            float4 v[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                v[c] = 4 * b + c < p.nparts ? reinterpret_cast<const float4*>(p.part)[(size_t)(4 * b + c) * p.n4 + i] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int c = 1; c < 4; ++c) { v[0].x += v[c].x; v[0].y += v[c].y; v[0].z += v[c].z; v[0].w += v[c].w; }
+            s.x += v[0].x; s.y += v[0].y; s.z += v[0].z; s.w += v[0].w;
+        }
+    } else if (i < p.n4) {
 #pragma unroll 6
         for (int b = b0; b < b1; ++b) {
             const float4 v = reinterpret_cast<const float4*>(p.part)[(size_t)b * p.n4 + i];

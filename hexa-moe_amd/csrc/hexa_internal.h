@@ -153,7 +153,7 @@ bool backward16_wanted(int T, int k, int hidden, int dim, int dt, double most);
 bool backward16_supported(const EsmmArgs& e, const EstmmArgs& t);
 int launch_backward16(const EsmmArgs* e, const EstmmArgs* t, const GateBwdK* g, bool io, SmallBatch& small, hipStream_t st);
 GateBwdK gate_bwd_args(void* dx, bool dwg, const float* dl, const void* x, const float* wg, int T, int d, int E, float* ws);
-int launch_dwg_reduce(float* dwg, const float* ws, int T, int d, int E, hipStream_t st);
+int launch_dwg_reduce(float* dwg, const float* ws, int T, int d, int E, hipStream_t st, bool merged = false);   // merged: a partial result for every four chunks
 bool estmm16_dma_supported(const EstmmArgs& a);
 int launch_estmm16_dma(const EstmmArgs& a, hipStream_t s);
 int launch_estmm16(const EstmmArgs& a, hipStream_t s);

@@ -35,7 +35,7 @@ struct SumSlotsK {
     float* wide;                                         // where set, the rounded sum goes here as fp32 and out stays as it is (no lists)
 };
 struct GateBwdK { void* dx; float* part; const float* dl; const void* x; const float* wg; int T, d, E, ntasks; };
-struct DwgReduceK { float* dwg; const float* part; int nparts; long n4; };
+struct DwgReduceK { float* dwg; const float* part; int nparts; long n4; int merged; };     // merged: each part is the sum of four chunks
 
 enum SmallKind : unsigned {
     TASK_ESS = 1u, TASK_ESS_FOLD = 2u, TASK_ROUTER_BWD = 4u, TASK_FIXUP = 8u, TASK_COLSUM_FOLD = 16u,

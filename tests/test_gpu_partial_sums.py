@@ -1,4 +1,5 @@
-"""Partial results that a second pass adds: the parts of large fp32 weight gradients, four values a thread."""
+"""Partial results that a second pass adds: the gate's dwg, one for every four chunks of 64 tokens, and the parts of large fp32 weight
+gradients, four values a thread."""
 import pytest
 import torch
 
@@ -6,6 +7,23 @@ from _util import TOL, assert_close, gen, make_routing
 from oracle import hexa_oracle as O
 
 pytestmark = pytest.mark.gpu
+
+
+# tokens: a chunk and four of them, one less and one more; dims and experts: ends of 128 columns and 32 experts
+@pytest.mark.parametrize("T", [1, 63, 65, 192, 255, 256, 257, 512, 1030])
+@pytest.mark.parametrize("d,E", [(8, 1), (136, 33), (120, 65), (256, 32)])
+def test_gate_dwg(dev, T, d, E):
+    from hexa_moe import ops
+    g = gen(T + d)
+    x, wg, dl = torch.randn(T, d, generator=g).bfloat16(), torch.randn(E, d, generator=g), torch.randn(T, E, generator=g)
+    print(f"gate dwg: T={T} d={d} E={E}", flush=True)
+    dx, dwg = ops.gate_backward(dl.to(dev), x.to(dev), wg.to(dev))
+    torch.cuda.synchronize()
+    # fp32 sums of up to 1030 products of order 1: 2^-24 times the root of their number at most, against the largest value
+    assert_close(dwg, dl.double().t() @ x.double(), 2e-6, "gate dwg")
+    assert_close(dx, dl.double() @ wg.double(), 2 ** -8, "gate dx")
+    for need_dx in (True, False):
+        assert torch.equal(ops.gate_backward(dl.to(dev), x.to(dev), wg.to(dev), need_dx=need_dx)[1], dwg)
 
 
 # results just below and above the size from which four values a thread are added; two and eight parts
