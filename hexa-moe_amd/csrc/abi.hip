@@ -276,7 +276,7 @@ int hexa::esmm_gelu_bwd_ess_call(void* out, void* db, const void* x, const void*
     if (!is_dt(x_dt) || !is_dt(w_dt) || !is_dt(db_dt)) HEXA_FAIL(HEXA_ERR_ARG, "hexa_esmm_gelu_bwd_ess: unknown element type");
     int64_t need = 0;
     hexa_esmm_ess_ws_floats(T, k, out_dim, E, &need);
-    if (T > 0 && is_16(x_dt) && w_dt == x_dt && ws && ws_floats >= need && dma_path_enabled()) {
+    if (T > 0 && w_dt == x_dt && ws && ws_floats >= need && (x_dt == HEXA_F32 || (is_16(x_dt) && dma_path_enabled()))) {
         EsmmArgs a;
         a.out = out; a.x = x; a.w = w; a.bias = nullptr; a.out_act = const_cast<void*>(y1); a.slot_ws = nullptr;
         a.r = route_view(route, T, k, E);
@@ -287,9 +287,9 @@ int hexa::esmm_gelu_bwd_ess_call(void* out, void* db, const void* x, const void*
         a.careful = careful;
         if (w_layout != HEXA_W_IN_OUT && w_layout != HEXA_W_OUT_IN)
             HEXA_FAIL(HEXA_ERR_ARG, "hexa_esmm_gelu_bwd_ess: bad w_layout %d", w_layout);
-        if (esmm16_dma_colsum_supported(a)) {
+        if (x_dt == HEXA_F32 ? esmm32_colsum_supported(a) : esmm16_dma_colsum_supported(a)) {
             a.colsum = ws; a.db = db; a.db_dt = db_dt; a.db_accumulate = db_accumulate ? 1 : 0;
-            return launch_esmm16_dma(a, (hipStream_t)stream);
+            return x_dt == HEXA_F32 ? launch_esmm32(a, (hipStream_t)stream) : launch_esmm16_dma(a, (hipStream_t)stream);
         }
     }
     // any other case: the two operators one after the other (same results up to the order of the sums)

@@ -294,6 +294,7 @@ struct Esmm32K {
     int T, K, N, mt_ub, ntn, slot_begin, nslots;
     int x_slot_rows, out_slot_rows;
     int accumulate, act, act_only;
+    float* colsum;        // where set (tiles of HEXA_TILE_ROWS rows): [slot][row tile][column tile][BN] column sums of the stored result
 };
 
 template <bool W_IN_OUT, bool BIG, typename C>
@@ -383,8 +384,13 @@ __global__ __launch_bounds__(C::NT, C::WAVES) void esmm32_kernel(Esmm32K p) {
     zero_acc(acc);
     const bool busy = wr * 32 * C::RB < rows && n0 + wf * 32 * C::FB < N;     // the others have no row or no column of the tile
     multiply_stages<C, W_IN_OUT, false>((K + KD - 1) / KD, busy, smem, sWhole, tid, acc, load);
-    if (!combine<C>(smem, kg, wave, lane, acc) || !busy) return;
+    constexpr bool COLSUM_OK = C::BM == HEXA_TILE_ROWS && C::WR == 2;
+    const bool colsum = COLSUM_OK && p.colsum != nullptr;
+    if (!combine<C>(smem, kg, wave, lane, acc) || (!busy && !colsum)) return;
 
+    float cs[COLSUM_OK ? 16 * C::FB : 1];
+#pragma unroll
+    for (float& c : cs) c = 0.f;
     const bool to_ws = p.ws != nullptr && s > 0;
     float* const outp = to_ws ? p.ws : p.out;
     const bool accumulate = p.accumulate && !to_ws;
@@ -392,7 +398,7 @@ __global__ __launch_bounds__(C::NT, C::WAVES) void esmm32_kernel(Esmm32K p) {
 #pragma unroll
     for (int i = 0; i < C::RB; ++i) {
         const int tok = sTok[(wr * C::RB + i) * 32 + (lane & 31)];
-        if (tok < 0) continue;
+        if (tok < 0 || !busy) continue;
 #pragma unroll
         for (int j = 0; j < C::FB; ++j) {
 #pragma unroll
@@ -415,9 +421,29 @@ __global__ __launch_bounds__(C::NT, C::WAVES) void esmm32_kernel(Esmm32K p) {
                     v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
                 }
                 if (!p.act_only) *dst = v;
+                if constexpr (COLSUM_OK) {
+                    float* const c = cs + j * 16 + 4 * g;
+                    c[0] += v.x; c[1] += v.y; c[2] += v.z; c[3] += v.w;
+                }
                 if (p.act == HEXA_ACT_GELU)
                     *reinterpret_cast<float4*>(p.out_act + off) = make_float4(gelu_full(v.x), gelu_full(v.y), gelu_full(v.z), gelu_full(v.w));
             }
+        }
+    }
+    // Column sums of the tile: the 32 lanes of a row block, then the two wavefronts of a column block.
+    if constexpr (COLSUM_OK) {
+        if (colsum) {
+            __shared__ float sums[2][BN];
+#pragma unroll
+            for (float& c : cs)
+#pragma unroll
+                for (int m = 16; m > 0; m >>= 1) c += __shfl_xor(c, m);
+            if ((lane & 31) == 0) {
+#pragma unroll
+                for (int c = 0; c < 16 * C::FB; ++c) sums[wr][(wf * C::FB + (c >> 4)) * 32 + 8 * ((c >> 2) & 3) + 4 * (lane >> 5) + (c & 3)] = cs[c];
+            }
+            __syncthreads();
+            if (tid < BN) p.colsum[(((size_t)s * p.mt_ub + mt) * p.ntn + nt) * BN + tid] = sums[0][tid] + sums[1][tid];
         }
     }
 }
@@ -602,6 +628,18 @@ bool too_large(size_t rows, size_t cols) { return (rows + 64) * cols * 4 >= ((si
 
 }  // namespace
 
+// 128 x 128 tiles where they come to one for most CUs and the lists fill them: 3000 rows, 1024 -> 2048, 4 experts 101
+// against 125 us of 64 x 64 tiles, 23 x 8 tiles of its fc2 124 against 139, 8192 rows, 2048 -> 512 (64 x 4) 160 both; 64
+// rows an expert 49 against 44, 4000 rows, 2048 -> 512 (31 x 4 tiles) 117 against 101
+static bool esmm32_wide(const EsmmArgs& a, int slots) {
+    return (long)slots * a.r.T / 128 * div_up(a.out_dim, 128) >= 180 && a.r.T >= 100 * a.r.E;
+}
+// Column sums come from the store loop of the 128 x 128 tiles, all slots in one launch: 9216 rows, top-2 of 8 experts, 384 x 1536, a
+// pass over the stored result takes 21.5 us.
+bool esmm32_colsum_supported(const EsmmArgs& a) {
+    return a.act == HEXA_ACT_GELU_BWD && a.out_per_slot && a.r.k <= 8 && a.in_dim % 4 == 0 && a.out_dim % 4 == 0 && esmm32_wide(a, a.r.k);
+}
+
 int launch_esmm32(const EsmmArgs& a, hipStream_t st) {
     if ((a.in_dim & 3) || (a.out_dim & 3))
         HEXA_FAIL(HEXA_ERR_UNSUPPORTED, "esmm (fp32): in_dim and out_dim must be multiples of 4 (got %d, %d)",
@@ -613,7 +651,7 @@ int launch_esmm32(const EsmmArgs& a, hipStream_t st) {
     p.T = a.r.T; p.K = a.in_dim; p.N = a.out_dim; p.mt_ub = a.r.mt_ub;
     p.x_slot_rows = a.x_per_slot ? a.r.T : 0;
     p.out_slot_rows = a.out_per_slot ? a.r.T : 0;
-    p.act = a.act; p.act_only = a.act_only;
+    p.act = a.act; p.act_only = a.act_only; p.colsum = a.colsum;
     // Summing the slots into one result: with scratch every slot runs in one launch (slot 0 into `out`, the others into
     // the scratch) and a small kernel adds them; without, one launch per slot adds into `out`.
     const bool sum = !a.out_per_slot && a.r.k > 1;
@@ -626,10 +664,7 @@ int launch_esmm32(const EsmmArgs& a, hipStream_t st) {
         if (p.mt_ub == 0) continue;
         const bool io = a.w_layout == HEXA_W_IN_OUT;
         const bool big = too_large((size_t)a.r.T * (a.x_per_slot ? a.r.k : 1), a.in_dim) || too_large(a.in_dim, a.out_dim);
-        // 128 x 128 tiles where they come to one for most CUs and the lists fill them: 3000 rows, 1024 -> 2048, 4 experts 101
-        // against 125 us of 64 x 64 tiles, 23 x 8 tiles of its fc2 124 against 139, 8192 rows, 2048 -> 512 (64 x 4) 160 both; 64
-        // rows an expert 49 against 44, 4000 rows, 2048 -> 512 (31 x 4 tiles) 117 against 101
-        const bool wide = (long)p.nslots * a.r.T / 128 * div_up(a.out_dim, 128) >= 180 && a.r.T >= 100 * a.r.E;
+        const bool wide = esmm32_wide(a, p.nslots);
         auto go = [&](auto bg) {
             constexpr bool BIG = decltype(bg)::value;
             return wide ? (io ? launch_esmm32_t<true, BIG, Wide>(p, st) : launch_esmm32_t<false, BIG, Wide>(p, st))
@@ -639,6 +674,7 @@ int launch_esmm32(const EsmmArgs& a, hipStream_t st) {
         if (rc) return rc;
     }
     if (p.ws) return launch_sum_slots(a.out, a.slot_ws, a.r, a.out_dim, a.accumulate, HEXA_F32, st, a.sum_extra);
+    if (a.colsum) return launch_colsum_fold(a, p.mt_ub, HEXA_TILE_ROWS, div_up(a.out_dim, Wide::BN), Wide::BN, st);
     return HEXA_OK;
 }
 

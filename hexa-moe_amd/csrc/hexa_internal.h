@@ -100,6 +100,7 @@ bool esmm_slot_sum_takes_extra(const int32_t* route, int w_layout, int T, int k,
                                int w_dt, int out_dt, const void* slot_ws, bool careful);
 int launch_esmm16(const EsmmArgs& a, hipStream_t s);
 int launch_esmm32(const EsmmArgs& a, hipStream_t s);
+bool esmm32_colsum_supported(const EsmmArgs& a);
 // Tuning / testing knobs: 0 = automatic.  Each one starts from an environment variable (read once) and
 // can be changed at run time with hexa_set_option.
 enum Opt {

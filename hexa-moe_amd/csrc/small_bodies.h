@@ -609,13 +609,15 @@ __device__ __forceinline__ void colsum_fold_body(const ColsumFoldK& p, int block
     for (int s = 0; s < runs; ++s) {
         const int first = sFirst[s], last = min(first + sCount[s], p.mt_ub);
         // eight loads in flight per trip (a busy expert has a dozen tiles; one load per trip would pay the
-        // memory latency a dozen times); the additions stay in tile order
+        // memory latency a dozen times), added in pairs: a chain of eighteen tiles' sums was 10 % less exact in fp32 than a pass
+        // over the stored rows (9216 tokens, top-2 of 8 experts: 1.13e-7 against 1.03e-7 of 64 bits)
         for (int mt = first; mt < last; mt += 8) {
             float v[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) v[u] = p.colsum[(((size_t)s * p.mt_ub + min(mt + u, last - 1)) * p.ntn + nt) * p.bn + nl];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) sum += (mt + u < last) ? v[u] : 0.f;
+            for (int u = 0; u < 8; ++u) v[u] = (mt + u < last) ? v[u] : 0.f;
+            sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
         }
     }
     store_out(p.db, (size_t)e * p.N + n, sum, p.db_dt, p.accumulate != 0);

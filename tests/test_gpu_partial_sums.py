@@ -1,5 +1,5 @@
 """Partial results that a second pass adds: the gate's dwg, one for every four chunks of 64 tokens, and the parts of large fp32 weight
-gradients, four values a thread."""
+gradients, four values a thread; the fp32 bias gradient by column sums of the tiles of dy1."""
 import pytest
 import torch
 
@@ -42,3 +42,27 @@ def test_fp32_weight_gradient_parts(dev, T, E, k, d_in, d_out):
     torch.cuda.synchronize()
     assert_close(got, want, TOL[torch.float32], "estmm")
     assert_close(ops.estmm(dy.to(dev), x.to(dev), route, True, False, out=torch.ones_like(got), accumulate=True), want + 1, TOL[torch.float32], "estmm +=")
+
+
+# 128 x 128 tiles (the rule asks for 180 of them and 100 tokens an expert): columns that end inside a tile and inside a wavefront's 32, lists
+# of no, few and many rows, two slots; one size on the 64 x 64 tiles, whose bias gradient is a pass of its own
+@pytest.mark.parametrize("T,E,k,d_in,d_out,skew", [(3000, 4, 1, 64, 1028, None), (2100, 7, 2, 36, 788, "zipf"), (5000, 3, 1, 132, 640, "one"),
+                                                      (3000, 4, 1, 64, 512, None)])
+def test_fp32_bias_gradient_beside_dy1(dev, T, E, k, d_in, d_out, skew):
+    from hexa_moe import _lib, ops
+    print(f"fp32 column sums: T={T} E={E} k={k} {d_in} -> {d_out} {skew}", flush=True)
+    routing = make_routing(T, E, k, seed=T, skew=skew, empty=2 if skew == "zipf" else 0)
+    _, offsets, token_ids = O.route_build(routing, E)
+    route = ops.route_build(routing.to(dev), E)
+    g = gen(d_in)
+    x, W, y1 = torch.randn(T, d_in, generator=g), torch.randn(E, d_out, d_in, generator=g) / d_in ** 0.5, torch.randn(k, T, d_out, generator=g)
+    t = y1.double()
+    want = O.esmm(x.double(), W.transpose(1, 2).double(), None, token_ids, offsets, False) * \
+        (0.5 * (1 + torch.erf(t / 2 ** 0.5)) + t * torch.exp(-0.5 * t * t) / (2 * torch.pi) ** 0.5)
+    got, db = ops.esmm_gelu_bwd_ess(x.to(dev), W.to(dev), route, _lib.HEXA_W_OUT_IN, y1.to(dev))
+    torch.cuda.synchronize()
+    assert_close(got, want, TOL[torch.float32], "dy1")
+    sums = O.ess(got.double().cpu(), token_ids, offsets, True, E)
+    assert_close(db, sums, TOL[torch.float32], "db")
+    assert torch.equal(db.cpu()[sums.abs().sum(1) == 0], sums[sums.abs().sum(1) == 0].float())       # no rows: zeros
+    assert torch.equal(db, ops.esmm_gelu_bwd_ess(x.to(dev), W.to(dev), route, _lib.HEXA_W_OUT_IN, y1.to(dev))[1])
