@@ -179,7 +179,8 @@ int launch_sum_wide_slots(void* out, const float* ws, const void* extra, const R
 
 // out (+)= the sum of `parts` partial results of n values each, in their order
 int launch_fold(void* out, const float* ws, long n, int parts, int dt, int accumulate, hipStream_t st) {
-    // Parts of a weight gradient are bound by memory: 16 bytes of each a thread.  Bias gradients, a few hundred thousand values at most, by
+    // Parts of a weight gradient are bound by memory: 16 bytes of each a thread (two
+    // gradients of 8 x 1536 x 384 in three parts, 151 MB: 25.3 us, by single values 40.8).  Bias gradients, a few hundred thousand values at most, by
     // their latency: one value a thread keeps more of them in flight.
     const int by4 = dt == HEXA_F32 && n % 4 == 0 && n >= ((long)1 << 19) && (((uintptr_t)out | (uintptr_t)ws) & 15) == 0;
     SmallTask f;

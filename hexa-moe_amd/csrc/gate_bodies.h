@@ -262,7 +262,8 @@ __device__ __forceinline__ void gate_bwd_body(const GateBwdK& p, int block) {
 
 // The same products where a workgroup's four wavefronts take the same task of four chunks, one after the other, and leave one partial dwg for
 // them (p.ntasks: workgroups).  At 32768 tokens, 1024 wide, 64 experts the partial results of single chunks are 134 MB, written
-// here and read by the fold.
+// here and read by the fold: with four chunks to one the launch of fold and slot sum takes 51 us instead of 71, this one 141 instead of
+// 143 (its products 55 us of the chip).
 template <typename T>
 __device__ __forceinline__ void gate_bwd_merged_body(const GateBwdK& p, int block, float4* sums) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

@@ -85,3 +85,20 @@ def test_scratch_of_slots_that_are_added_unrounded(act_dt, careful):
     (rc, fwd, bwd), (rc0, fwd0, bwd0) = ask(careful), ask(0)
     more = T * d * (k * 4 - (k - 1) * 2) if careful and act_dt else 0
     assert rc == rc0 == 0 and (fwd - fwd0, bwd - bwd0) == (more, more)
+
+
+def test_fp32_dx_takes_a_16_bit_one_in_scratch():
+    """Top-1, 16-bit tokens, whole 16-byte pieces; anything else is refused and not ignored."""
+    from hexa_moe import _lib
+    size = ctypes.sizeof(_lib.DepthOpts)
+
+    def ask(T, k, d, act_dt, part=7):
+        desc = _lib.DepthDesc(T, k, 8, d, 64, d, act_dt, act_dt, *[0] * 6, 0, 0.0, 0.0, 0)
+        return [_bytes("hexa_moe_depth_part_ws_bytes", ctypes.byref(desc), ctypes.byref(_lib.DepthOpts(size, part, 0, 0, 0, 0, wide))) for wide in (0, 1)]
+
+    for part in (1, 2, 3, 4, 7):
+        plain, wide = ask(256, 1, 64, 2, part)
+        assert wide[:2] == plain[:2] and wide[2] == plain[2] + (256 * 64 * 2 if part & 2 else 0)
+    for args in ((256, 2, 64, 2), (256, 1, 64, 0), (3, 1, 4, 2)):
+        plain, wide = ask(*args)
+        assert plain[0] == 0 and wide[0] == -2
