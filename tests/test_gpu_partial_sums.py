@@ -66,3 +66,25 @@ def test_fp32_bias_gradient_beside_dy1(dev, T, E, k, d_in, d_out, skew):
     assert_close(db, sums, TOL[torch.float32], "db")
     assert torch.equal(db.cpu()[sums.abs().sum(1) == 0], sums[sums.abs().sum(1) == 0].float())       # no rows: zeros
     assert torch.equal(db, ops.esmm_gelu_bwd_ess(x.to(dev), W.to(dev), route, _lib.HEXA_W_OUT_IN, y1.to(dev))[1])
+
+
+# Lists of 160 and more tiles, values with a mean: what a chain of partial sums would lose.  Both orders of additions modelled on the CPU give
+# 0.7 (20000 rows a list) and 0.7 (65536) of the pass's error; groups of tiles in a chain 1.3 and 2.4.
+@pytest.mark.parametrize("T,E,k", [(65536, 1, 1), (20000, 2, 2)])
+def test_fp32_bias_gradient_of_long_lists(dev, T, E, k):
+    """No less exact than a pass over the stored rows."""
+    from hexa_moe import _lib, ops
+    print(f"fp32 column sums: T={T} E={E} k={k}", flush=True)
+    routing = make_routing(T, E, k, seed=1, skew="one")
+    route = ops.route_build(routing.to(dev), E)
+    g = gen(T)
+    x, W = torch.randn(T, 32, generator=g).to(dev), (torch.randn(E, 512, 32, generator=g) / 32 ** 0.5).to(dev)
+    x[:, 0], W[:, :, 0] = 1.0, 0.1
+    dy1, db = ops.esmm_gelu_bwd_ess(x, W, route, _lib.HEXA_W_OUT_IN, torch.full((k, T, 512), 10.0, device=dev))     # GELU'(10) = 1
+    by_pass = ops.ess(dy1, route, True)
+    torch.cuda.synchronize()
+    want = torch.zeros(E, 512, dtype=torch.float64, device=dev)
+    for s in range(k):
+        want.index_add_(0, routing[:, s].to(dev), dy1[s].double())
+    err = lambda v: ((v.double() - want).norm() / want.norm()).item()      # noqa: E731
+    assert err(db) <= 1.1 * err(by_pass), (err(db), err(by_pass))
