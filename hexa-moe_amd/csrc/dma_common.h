@@ -98,9 +98,10 @@ template <int N, int SPAN, int MAXA> __device__ __forceinline__ void wait_groups
     else wait_groups_of<N, SPAN - 1, MAXA>(more, ahead);
 }
 
-// Workgroup barrier WITHOUT the memory fence of __syncthreads(): the fence would wait for every
-// outstanding copy (vmcnt(0)) and drain the pipeline.  Ordering is by hand: copies are awaited with
-// wait_vmcnt, LDS reads of the previous stage have been consumed by MFMAs before a wavefront arrives.
+// Workgroup barrier WITHOUT the memory fence of __syncthreads().  The fence waits for the LDS accesses that the compiler knows of
+// (lgkmcnt(0)) and holds loads and stores in their place; for asynchronous copies it does not wait, so neither barrier publishes
+// them.  Ordering is by hand: copies are awaited with wait_vmcnt by the wavefront that issued them, LDS reads of the previous
+// stage have been consumed by MFMAs before a wavefront arrives.
 __device__ __forceinline__ void barrier_nofence() {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();

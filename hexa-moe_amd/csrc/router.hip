@@ -9,6 +9,7 @@
 #include "hexa_internal.h"
 #include "small_bodies.h"
 #include "gate_bodies.h"
+#include "dma_common.h"
 
 namespace hexa {
 namespace {
@@ -421,8 +422,7 @@ __global__ __launch_bounds__(GATE_ROUTER_NT, 4) void gate_router_kernel(
                 if (e0 + row >= E) continue;         // (those columns of the logits are nobody's)
                 const bool ok = c0 + c + (p >> 2) < c1 && col < d;
                 const float* src = ok ? wg + (size_t)(e0 + row) * d + col : reinterpret_cast<const float*>(g_gate_zeros);
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                                 (__attribute__((address_space(3))) void*)(operands + quarter * GR_QUARTER + (blk * (GR_QUARTER / 2048) + i) * 1024), 16, 0, 0);
+                dma16(src, operands + quarter * GR_QUARTER + (blk * (GR_QUARTER / 2048) + i) * 1024);
             }
             Raw8<X> xv[NB];
 #pragma unroll
@@ -431,9 +431,10 @@ __global__ __launch_bounds__(GATE_ROUTER_NT, 4) void gate_router_kernel(
                 const bool ok = c0 + c + u < c1 && piece < pieces;
                 xv[u].load(xrow + (ok ? piece : 0) * 8, ok && tok_ok);
             }
+            wait_vmcnt<0>();                                         // this wavefront's copies have landed: the barrier waits for LDS accesses only
 #pragma unroll
             for (int u = 0; u < NB; ++u) xv[u].arrive();
-            __syncthreads();                                         // (every copy has landed, too)
+            __syncthreads();
             f32x4 b[2][2];               // a chunk's values of wg, read while the chunk before it is multiplied
             auto read = [&](int u) {
 #pragma unroll

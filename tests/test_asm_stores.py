@@ -1,4 +1,5 @@
-"""Inline-assembly stores of more than 8 bytes and the wait states behind them."""
+"""Inline-assembly stores of more than 8 bytes and the wait states behind them; asynchronous copies and the waits in front of the barriers
+that publish them."""
 import pathlib
 import re
 
@@ -15,3 +16,14 @@ def test_wide_stores_are_followed_by_wait_states():
                 found += 1
                 assert re.match(r"[^\\]*\\n\\ts_nop [1-9]", text[store.end():]), (path.name, text)
     assert found >= 4
+
+
+def test_copies_are_awaited_before_the_barrier_behind_them():
+    """A barrier does not wait for asynchronous copies into LDS.  In the gate's kernel, which issues them and reads them in one block, a
+    wait of its own stands between."""
+    text = re.sub(r"//[^\n]*", "", (CSRC / "router.hip").read_text())
+    copies = list(re.finditer(r"\bdma16\(|global_load_lds\(", text))
+    assert copies
+    for c in copies:
+        barrier = re.compile(r"__syncthreads\(\)|barrier_nofence\(\)").search(text, c.end())
+        assert barrier and "wait_vmcnt<0>()" in text[c.end():barrier.start()], text[c.start():barrier.start()]
