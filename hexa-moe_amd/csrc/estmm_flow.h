@@ -397,7 +397,7 @@ inline int flow_args(const EstmmArgs& a, FlowK& p) {
     // runs of about nine blocks on one XCD (1024 x 4096: 8 instead of 24, 760 -> 727 us with a skewed load; 384 x 1536: 9 instead of 3, 71 ->
     // 65; 256 x 1024: 6 instead of 2, 56 -> 46)
     const int inside = std::min(p.mtn, p.ntn);
-    p.group = inside * (option(OPT_ESTMM_GROUP) > 0 ? option(OPT_ESTMM_GROUP) : std::max(1, 9 / inside));
+    p.group = inside * run_length(OPT_ESTMM_GROUP, std::max(1, 9 / inside));
     const bool cut = a.plan && a.scratch && a.max_slots >= 2;
     p.plan = cut ? a.plan : nullptr;
     p.scratch = cut ? a.scratch : nullptr;

@@ -599,7 +599,7 @@ int launch_estmm16_pipe(const EstmmArgs& a, hipStream_t st) {
     p.T = a.r.T; p.k = a.r.k; p.E = a.r.E; p.M = a.m_dim; p.N = a.n_dim;
     p.mtn = div_up(a.m_dim, C::BM); p.ntn = div_up(a.n_dim, C::BN);
     // runs of up to three row tiles (with all their column tiles) per XCD: their items share the rows of Q
-    p.group = p.ntn * (option(OPT_ESTMM_GROUP) > 0 ? option(OPT_ESTMM_GROUP) : std::min(3, p.mtn));
+    p.group = p.ntn * run_length(OPT_ESTMM_GROUP, std::min(3, p.mtn));
     p.p_slot_rows = a.p_per_slot ? a.r.T : 0;
     p.q_slot_rows = a.q_per_slot ? a.r.T : 0;
     p.accumulate = a.accumulate;

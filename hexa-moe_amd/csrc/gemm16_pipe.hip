@@ -718,7 +718,7 @@ int launch_esmm16_pipe(const EsmmArgs& a, hipStream_t st) {
     pk.wg_per_xcd = (int)std::min<long>(std::max(1, compute_units() / 8), (p.total + 7) / 8);
     const int grid = 8 * pk.wg_per_xcd;
     pk.offsets = a.r.offsets; pk.E = a.r.E;
-    pk.row_run = option(OPT_ESMM_GROUP) > 0 ? option(OPT_ESMM_GROUP) : (long)a.r.T * 4 >= 3L * C::BM * a.r.E ? PIPE_ROW_RUN : 1;
+    pk.row_run = run_length(OPT_ESMM_GROUP, (long)a.r.T * 4 >= 3L * C::BM * a.r.E ? PIPE_ROW_RUN : 1);
     const bool io = a.w_layout == HEXA_W_IN_OUT;
     if (a.wide && !io) HEXA_FAIL(HEXA_ERR_UNSUPPORTED, "esmm16_pipe: fp32 storage is for weights [in][out]");
     const int act = a.wide ? PIPE_ACT_WIDE : a.act;

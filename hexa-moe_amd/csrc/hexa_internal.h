@@ -125,6 +125,10 @@ enum Opt {
     OPT_COUNT
 };
 int option(int id);
+// An option that says how many row tiles a run has.  Longer runs than MAX_RUN make no difference that a measurement would show, and its
+// products with a result's column tiles stay within the 32 bits that grids and kernels work them out in.
+constexpr int MAX_RUN = 4096;
+inline int run_length(int id, int automatic) { return option(id) > MAX_RUN ? MAX_RUN : option(id) > 0 ? option(id) : automatic; }
 
 bool esmm16_dma_supported(const EsmmArgs& a);
 bool esmm16_dma_colsum_supported(const EsmmArgs& a);

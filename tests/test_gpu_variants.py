@@ -74,3 +74,30 @@ def test_variant(dev, knobs, cfg, dtype, dims):
     assert_close(ops.estmm(xs.to(dev), x.to(dev), route, True, False), want_dw, TOL[dtype], "estmm")
     assert_close(ops.estmm(xs.to(dev), x.to(dev), route, True, False, out_dtype=dtype), want_dw, TOL[dtype], "estmm 16-bit")
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("group", [1, 3, 5, 2 ** 30, 2 ** 31 - 1])
+def test_runs_of_row_tiles(dev, knobs, group):
+    """Runs that divide no list's row tiles, and runs longer than any list, walk every tile once: results of each order are bit for
+    bit those of the automatic one."""
+    from hexa_moe import _lib, ops
+    T, d_in, d_out, E, k, dtype = 5000, 320, 392, 5, 2, torch.bfloat16
+    print(f"runs of {group} row tiles", flush=True)
+    routing = make_routing(T, E, k, seed=6, skew="zipf", empty=1)         # lists of 0 to 20 row tiles
+    route = ops.route_build(routing.to(dev), E)
+    x, W, b = (t.to(dev) for t in make_linear(T, d_in, d_out, E, k, seed=7, dtype=dtype, m2s=False))
+    Wt = W.transpose(1, 2).contiguous()
+    back = (torch.randn(k, T, d_out, generator=gen(8))).to(dtype).to(dev)
+
+    def results():
+        y1, y2 = ops.esmm(x, Wt, b, route, False, _lib.HEXA_W_OUT_IN, gelu=True)
+        dy1, db = ops.esmm_gelu_bwd_ess(x, Wt, route, _lib.HEXA_W_OUT_IN, y1)
+        return [y1, y2, dy1, db, ops.esmm(back, Wt, None, route, True, _lib.HEXA_W_IN_OUT), ops.estmm(back, x, route, True, False)]
+
+    for cfg in ({"pipe": 1}, {"pipe": 2, "esmm_map": 2}):
+        knobs(cfg)
+        want = results()
+        knobs(dict(cfg, esmm_group=group, estmm_group=min(group, 12)))
+        for i, (a, c) in enumerate(zip(want, results())):
+            torch.cuda.synchronize()
+            assert torch.equal(a, c), (cfg, i)
