@@ -307,7 +307,8 @@ typedef struct hexa_moe_depth_opts {
                         * with workspaces that hold an fp32 result of every slot) */
     int32_t no_gate;   /* 1: wg is NULL in every call, and the workspaces leave the router's and the gate's share out */
     int32_t no_y1;     /* 1: no backward will read y1; a forward of both layers may leave the buffer unwritten */
-    int32_t wide_dx;   /* 1: the backward stores dx, rounded to act_dt, as fp32 (16-bit act_dt and top_k 1 only, T * d_in a multiple of 8) */
+    int32_t wide_dx;   /* 1: the backward stores dx, rounded to act_dt, as fp32 (16-bit act_dt and top_k 1 only, T * d_in a multiple of 8,
+                        * dx 16-byte aligned) */
 } hexa_moe_depth_opts;
 
 /* Which parts of the depth a call runs (0: all of them).  With an activation that the kernels do not fuse, the caller

@@ -102,3 +102,16 @@ def test_fp32_dx_takes_a_16_bit_one_in_scratch():
     for args in ((256, 2, 64, 2), (256, 1, 64, 0), (3, 1, 4, 2)):
         plain, wide = ask(*args)
         assert plain[0] == 0 and wide[0] == -2
+
+
+@pytest.mark.parametrize("offset,refused", [(0, False), (16, False), (4, True), (8, True), (15, True)])
+def test_fp32_dx_is_16_byte_aligned(offset, refused):
+    """It is stored 16 bytes at a time.  (No pointer is read: the workspace is said to be empty, which is looked at next.)"""
+    from hexa_moe import _lib
+    lib = _lib.load()
+    desc, opts = _lib.DepthDesc(256, 1, 8, 64, 64, 64, 2, 2, *[0] * 6, 0, 0.0, 0.0, 0), _lib.DepthOpts(ctypes.sizeof(_lib.DepthOpts), 2, 0, 0, 1, 0, 1)
+    any_ = ctypes.c_void_p(4096)
+    rc = lib.hexa_moe_depth_part_backward(ctypes.byref(desc), ctypes.byref(opts), any_, None, any_, None, any_, any_, None, None, None, None, any_, None,
+                                          any_, any_, ctypes.c_void_p(4096 + offset), None, None, None, None, None, any_, any_, 0, None, 0, None)
+    assert rc == -1
+    assert (b"aligned" in lib.hexa_last_error()) == refused, lib.hexa_last_error()
