@@ -618,15 +618,14 @@ extern "C" int hexa_router_ws_floats(int T, int E, int64_t* out) {
 namespace hexa {
 namespace {
 // The LDS tile of the four-lanes-per-token router (with the routing histogram behind it) passes 64 KiB for many
-// experts and a deep top-k: such a launch needs the kernel's dynamic-LDS limit raised first, once per kernel, to the
-// most any supported (E, k) asks for.
-template <typename K> int allow_router_lds(K kernel, size_t bytes) {
+// experts and a deep top-k, and so does the gate's kernel with the FIXED bytes that it declares itself: such a launch needs the kernel's
+// dynamic-LDS limit raised first, once per kernel, to the MOST any supported (E, k) asks for.
+template <auto KERNEL, size_t FIXED, size_t MOST> int allow_router_lds(size_t bytes) {
+    static_assert(FIXED + MOST <= 160 * 1024, "LDS of a CU");
     static bool done = false;   // per kernel
-    if (bytes <= 64 * 1024 || done) return HEXA_OK;
-    constexpr size_t most = sizeof(float) * router4_lds_floats(ROUTER_LDS_E, MAX_TOPK, true, true);
-    static_assert(most <= 160 * 1024, "LDS of a CU");
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)most) != hipSuccess)
-        HEXA_FAIL(HEXA_ERR_LAUNCH, "router: hipFuncSetAttribute(MaxDynamicSharedMemorySize=%d) failed", (int)most);
+    if (FIXED + bytes <= 64 * 1024 || done) return HEXA_OK;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize, (int)MOST) != hipSuccess)
+        HEXA_FAIL(HEXA_ERR_LAUNCH, "router: hipFuncSetAttribute(MaxDynamicSharedMemorySize=%d) failed", (int)MOST);
     done = true;
     return HEXA_OK;
 }
@@ -645,7 +644,8 @@ int launch_router_fwd(float* scores, int32_t* idx, const float* logits, const fl
     const LiK li{thr, noise, noise_scale, inv_sigma};
     if (E <= ROUTER_LDS_E) {
         const size_t lds = sizeof(float) * router4_lds_floats(E, k, hist != nullptr, thr != nullptr);
-        if (int rc = thr ? allow_router_lds(router_fwd4_kernel<true>, lds) : allow_router_lds(router_fwd4_kernel<false>, lds)) return rc;
+        constexpr size_t most = sizeof(float) * router4_lds_floats(ROUTER_LDS_E, MAX_TOPK, true, true);
+        if (int rc = thr ? allow_router_lds<router_fwd4_kernel<true>, 0, most>(lds) : allow_router_lds<router_fwd4_kernel<false>, 0, most>(lds)) return rc;
         if (thr)
             hipLaunchKernelGGL(router_fwd4_kernel<true>, dim3(nb), dim3(ROUTER_TB * ROUTER_G), lds, st, scores, idx, part_me, part_cnt,
                                logits, noise, noise_scale, T, E, k, hist, li);
@@ -674,7 +674,8 @@ int launch_gate_router_t(float* logits, float* scores, int32_t* idx, const void*
                          int T_, int d, int E, int k, float* ws, int32_t* hist, const LiK& li, RoundAllK* round, hipStream_t st) {
     const int nb = div_up(T_, ROUTER_TB);
     const size_t lds = sizeof(float) * router4_lds_floats(E, k, hist != nullptr, LI);
-    if (int rc = allow_router_lds(gate_router_kernel<T, LI, ROUND>, lds)) return rc;
+    constexpr size_t most = sizeof(float) * router4_lds_floats(GATE_ROUTER_MAX_E, MAX_TOPK, true, LI);
+    if (int rc = allow_router_lds<gate_router_kernel<T, LI, ROUND>, GR_BYTES, most>(lds)) return rc;
     RoundAllK r{};
     if (round) r = *round;
     r.blocks = (int)((r.n + GATE_ROUTER_NT * 8 * ROUND_STEPS - 1) / (GATE_ROUTER_NT * 8 * ROUND_STEPS));
