@@ -363,6 +363,7 @@ constexpr int ROUND_NONE = 0, ROUND_WEIGHTS = 1, ROUND_TOKENS = 2;
 constexpr int GR_PIECES = 4 * FWD_NB;                                    // 16-byte pieces of a wg row in a trip
 constexpr int GR_QUARTER = 32 * GR_PIECES * 16, GR_BYTES = 4 * GR_QUARTER;   // of the four quarters of the model dimension
 static_assert(GR_BYTES >= 2 * 4 * 16 * 64 * 4, "the partial sums fit in the operands' place");
+static_assert(GR_BYTES >= 4 * ROUTER_TB * router_pitch(GATE_ROUTER_MAX_E), "the logits without the noise fit in the operands' place");
 static_assert(GR_QUARTER % 2048 == 0, "copies of 1 KB, half of them by either token block's wavefront");
 // piece p of row r sits in slot (p + r / 2) of its row: rows are 24 slots apart, 16 lanes read 16 different groups of four banks
 __device__ __forceinline__ int gr_turn(int row) { return (row & 15) >> 1; }
@@ -381,7 +382,8 @@ __global__ __launch_bounds__(GATE_ROUTER_NT, 4) void gate_router_kernel(
         round_all_body(round, blockIdx.x - nblocks);
         return;
     }
-    const Router4Lds L(sh, E, LI);
+    Router4Lds L(sh, E, false);
+    if (LI) L.clean = reinterpret_cast<float*>(operands);    // (behind the projection; with a place of its own 64 experts left one workgroup a CU)
     const int P = L.P;
     float* tile = L.tile;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -673,8 +675,8 @@ template <typename T, bool LI, int ROUND>
 int launch_gate_router_t(float* logits, float* scores, int32_t* idx, const void* x, const float* x_src, const float* wg, const float* noise, float noise_scale,
                          int T_, int d, int E, int k, float* ws, int32_t* hist, const LiK& li, RoundAllK* round, hipStream_t st) {
     const int nb = div_up(T_, ROUTER_TB);
-    const size_t lds = sizeof(float) * router4_lds_floats(E, k, hist != nullptr, LI);
-    constexpr size_t most = sizeof(float) * router4_lds_floats(GATE_ROUTER_MAX_E, MAX_TOPK, true, LI);
+    const size_t lds = sizeof(float) * router4_lds_floats(E, k, hist != nullptr, false);
+    constexpr size_t most = sizeof(float) * router4_lds_floats(GATE_ROUTER_MAX_E, MAX_TOPK, true, false);
     if (int rc = allow_router_lds<gate_router_kernel<T, LI, ROUND>, GR_BYTES, most>(lds)) return rc;
     RoundAllK r{};
     if (round) r = *round;
