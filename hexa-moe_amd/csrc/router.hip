@@ -352,8 +352,8 @@ constexpr int GATE_ROUTER_NT = 2 * ROUTER_TB * ROUTER_G;
 // instruction: a trip's 24 pieces of 16 bytes of every row come by asynchronous copy, whole lines at a time, into LDS for the two token
 // blocks.  The token rows, half the bytes and nobody else's, go to registers, all of a trip's loads in flight.  The partial sums take the
 // operands' place in LDS.  Against both operands read by the lanes, a sixth of them in flight at once, and the scores in LDS between the passes
-// with lists of eight: 13.4 -> 11.4 us there, 14.6 -> 12.2 at 2304 tokens, 21.3 -> 19.6 at 18432, 81 -> 71 at 32768 tokens, 1024 wide, 64 experts;
-// fp32 tokens of 8 experts 14.4, 14.7.  Beside workgroups that round (38 to 75 million weights), whose traffic makes every trip to memory
+// with lists of eight: 13.4 -> 11.4 us there, 14.6 -> 12.2 at 2304 tokens, 21.3 -> 19.6 at 18432, 81 -> 71 at 32768 tokens, 1024 wide, 64 experts.
+// Beside workgroups that round (38 to 75 million weights), whose traffic makes every trip to memory
 // longer: 34.5 -> 26.4 at 9216 fp32 tokens, 39 -> 33 at 3600, 768 wide, 43 -> 34 at 18432.
 //
 // Workgroups past the routing ones round fp32 master weights to 16 bits (`round`): the routing workgroups are a chain of
@@ -362,19 +362,35 @@ constexpr int GATE_ROUTER_NT = 2 * ROUTER_TB * ROUTER_G;
 constexpr int ROUND_NONE = 0, ROUND_WEIGHTS = 1, ROUND_TOKENS = 2;
 constexpr int GR_PIECES = 4 * FWD_NB;                                    // 16-byte pieces of a wg row in a trip
 constexpr int GR_QUARTER = 32 * GR_PIECES * 16, GR_BYTES = 4 * GR_QUARTER;   // of the four quarters of the model dimension
-static_assert(GR_BYTES >= 2 * 4 * 16 * 64 * 4, "the partial sums fit in the operands' place");
-static_assert(GR_BYTES >= 4 * ROUTER_TB * router_pitch(GATE_ROUTER_MAX_E), "the logits without the noise fit in the operands' place");
+// Where wg's values come from.  DIRECT: few experts are few lines an instruction, and every lane reads its own row: no barrier between trips, no
+// chunk multiplied that a quarter does not have.  STAGED: through LDS as above, trips cut where a quarter's chunks end.  WHOLE: no trip is cut
+// (384, 768, 1152 columns); for rounded tokens an instance of its own, because beside cut trips it spills 28 registers and the cuts cost it 0.7 to
+// 1 us of 13 to 17.  us of the launch, DIRECT | STAGED, 8 experts.  bf16, 144 and 9216 tokens: 128 wide 7.0, 8.3 | 8.7, 9.8; 768 wide 12.6,
+// 14.5 | 15.5, 16.6; 1024 wide 15.2, 15.9 | 19.6, 20.8; 16 experts 15.5, 16.4 | 20.3, 21.3; 32 experts, 384 wide 11.7, 13.3 | 10.7, 12.3.  Rounded tokens, 144, 18432
+// and 32768 of them: 128 wide 8.5, 12.2, 12.9 | 8.7, 13.9, 15.8; 512 wide 14.8, 25.8, 27.3 | 17.0, 27.1, 29.8; 768 wide 20.1, 34.9, 49.5 | 21.9,
+// 37.5, 43.5; 12 experts, 512 wide 15.7, 26.0, 28.5 | 17.1, 27.5, 29.8, 768 wide 22.1, 36.9, 58.9 | 23.4, 38.5, 49.2.
+constexpr int GR_DIRECT = 0, GR_STAGED = 1, GR_WHOLE = 2;
+constexpr int GR_DIRECT_E = 16;
+constexpr int GR_AHEAD = 2;              // chunks in registers: one is under way while the other is multiplied
+inline int gate_router_mode(int d, int E, bool tokens) {
+    if (E <= (tokens && d > 512 ? GR_DIRECT_E / 2 : GR_DIRECT_E)) return GR_DIRECT;
+    return tokens && d % (4 * FWD_NB * 16) == 0 ? GR_WHOLE : GR_STAGED;
+}
+constexpr int GR_DIRECT_BYTES = 2 * 4 * 16 * 64 * 4;                     // the partial sums
+static_assert(GR_BYTES >= GR_DIRECT_BYTES, "the partial sums fit in the operands' place");
+static_assert(GR_BYTES >= 4 * ROUTER_TB * router_pitch(GATE_ROUTER_MAX_E) && GR_DIRECT_BYTES >= 4 * ROUTER_TB * router_pitch(GR_DIRECT_E),
+              "the logits without the noise fit in the operands' place");
 static_assert(GR_QUARTER % 2048 == 0, "copies of 1 KB, half of them by either token block's wavefront");
 // piece p of row r sits in slot (p + r / 2) of its row: rows are 24 slots apart, 16 lanes read 16 different groups of four banks
 __device__ __forceinline__ int gr_turn(int row) { return (row & 15) >> 1; }
-template <typename T, bool LI, int ROUND>
+template <typename T, bool LI, int ROUND, int MODE>
 __global__ __launch_bounds__(GATE_ROUTER_NT, 4) void gate_router_kernel(
     float* __restrict__ logits, float* __restrict__ scores, int32_t* __restrict__ idx, float* __restrict__ part_me,
     float* __restrict__ part_cnt, std::conditional_t<ROUND == ROUND_TOKENS, T, const T>* __restrict__ x, const float* __restrict__ x_src,
     const float* __restrict__ wg, const float* __restrict__ noise,
     float noise_scale, int num_tokens, int d, int E, int k, int32_t* __restrict__ hist, int nblocks, LiK li, RoundAllK round) {
     extern __shared__ float sh[];
-    __shared__ __attribute__((aligned(1024))) char operands[GR_BYTES];
+    __shared__ __attribute__((aligned(1024))) char operands[MODE == GR_DIRECT ? GR_DIRECT_BYTES : GR_BYTES];
     float (*part)[4][16][64] = reinterpret_cast<float (*)[4][16][64]>(operands);    // [token block][quarter of d][result register][lane]
     constexpr bool SRC32 = ROUND == ROUND_TOKENS;
     constexpr int NB = FWD_NB;
@@ -406,9 +422,84 @@ __global__ __launch_bounds__(GATE_ROUTER_NT, 4) void gate_router_kernel(
     if constexpr (SRC32) xrow = x_src + xat;
     else xrow = x + xat;
     const char* const mine = operands + quarter * GR_QUARTER;
-    for (int e0 = 0; e0 < E; e0 += 32) {
+    for (int e0 = 0; e0 < (MODE == GR_DIRECT ? 1 : E); e0 += 32) {
         const bool exp_ok = e0 + r < E;
         f32x16 acc = zero16();
+        // this lane's piece of a chunk as values; rounded tokens are stored, too: every piece of the workgroup's rows is some lane's once per block of
+        // experts.  (The caller says which piece: from its own trip's h, see there.)
+        auto values = [&](const Raw8<X>& from, int piece, bool ok, float (&a)[8]) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) a[i] = from.value(i);
+            if constexpr (SRC32) {
+                union { uint4 q; T t[8]; } o;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    o.t[i] = (T)a[i];
+                    a[i] = (float)o.t[i];
+                }
+                if (e0 == 0 && ok && piece < pieces && tok_ok) *reinterpret_cast<uint4*>(x + xat + (size_t)piece * 8) = o.q;
+            }
+        };
+        if constexpr (MODE == GR_DIRECT && SRC32) {
+            // Two chunks of an fp32 row are a line of 128 bytes and asked for together.  (One at a time and one ahead, as below, with a workgroup's lines as
+            // large as the L1: 83 us instead of 71 at 32768 tokens, 1024 wide, 8 experts.)
+            const float* const wrow = wg + (size_t)(exp_ok ? r : 0) * d;
+            for (int c = c0; c < c1; c += 2) {
+                Raw8<X> xv[2];
+                Raw8<float> wv[2];
+                float a[2][8];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int piece = 2 * (c + u) + h;
+                    const bool ok = c + u < c1 && piece < pieces;
+                    xv[u].load(xrow + (ok ? piece : 0) * 8, ok && tok_ok);
+                    wv[u].load(wrow + (ok ? piece : 0) * 8, ok && exp_ok);
+                }
+#pragma unroll
+                for (int u = 0; u < 2; ++u) values(xv[u], 2 * (c + u) + h, c + u < c1, a[u]);
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][i], wv[u].value(i), acc, 0, 0, 0);
+            }
+        } else if constexpr (MODE == GR_DIRECT) {
+            // (lanes without an expert or a token read another's: their column or row of the logits is nobody's)
+            const X* const xblock = x + (size_t)t0 * d;
+            const unsigned wat = (exp_ok ? r : 0) * d, tat = (tok_ok ? 32 * blk + r : 0) * d;
+            Raw8<X> xv[GR_AHEAD];
+            Raw8<float> wv[GR_AHEAD];
+            auto fetch = [&](int u, int chunk) {
+                chunk = min(chunk, c1 - 1);
+                const unsigned at = (chunk * 2 + (2 * chunk + h < pieces ? h : 0)) * 8;
+                wv[u].load(wg + (wat + at), true);
+                xv[u].load(xblock + (tat + at), true);
+            };
+            auto multiply = [&](int u, int chunk) {
+                wv[u].arrive();
+                xv[u].arrive();
+                float a[8];
+                values(xv[u], 2 * chunk + h, true, a);
+                const bool there = 2 * chunk + h < pieces;           // (the last chunk may have one piece)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(there ? a[i] : 0.f, there ? wv[u].value(i) : 0.f, acc, 0, 0, 0);
+            };
+            if (c0 < c1) {
+#pragma unroll
+                for (int u = 0; u < GR_AHEAD; ++u) fetch(u, c0 + u);
+                int c = c0;
+                for (; c + GR_AHEAD <= c1; c += GR_AHEAD) {
+#pragma unroll
+                    for (int u = 0; u < GR_AHEAD; ++u) {
+                        multiply(u, c + u);
+                        fetch(u, c + u + GR_AHEAD);
+                        asm volatile("" ::: "memory");
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < GR_AHEAD - 1; ++u)
+                    if (c + u < c1) multiply(u, c + u);
+            }
+        } else {
         for (int c = 0; c < (chunks + 3) >> 2; c += NB) {            // (the quarters are of one length, or one chunk shorter)
             if (c > 0) __syncthreads();                              // the trip before has been read
             int ln = lane;               // (addresses worked out in every trip, not kept over all of them)
@@ -421,9 +512,8 @@ __global__ __launch_bounds__(GATE_ROUTER_NT, 4) void gate_router_kernel(
                 int p = slot - gr_turn(row);
                 if (p < 0) p += GR_PIECES;
                 const int col = (c0 + c) * 16 + p * 4;
-                if (e0 + row >= E) continue;         // (those columns of the logits are nobody's)
-                const bool ok = c0 + c + (p >> 2) < c1 && col < d;
-                const float* src = ok ? wg + (size_t)(e0 + row) * d + col : reinterpret_cast<const float*>(g_gate_zeros);
+                if (e0 + row >= E || c0 + c + (p >> 2) >= c1) continue;     // (those columns of the logits are nobody's, those chunks not multiplied)
+                const float* src = col < d ? wg + (size_t)(e0 + row) * d + col : reinterpret_cast<const float*>(g_gate_zeros);
                 dma16(src, operands + quarter * GR_QUARTER + (blk * (GR_QUARTER / 2048) + i) * 1024);
             }
             Raw8<X> xv[NB];
@@ -446,27 +536,23 @@ __global__ __launch_bounds__(GATE_ROUTER_NT, 4) void gate_router_kernel(
                     b[u & 1][q] = *reinterpret_cast<const f32x4*>(mine + (r * GR_PIECES + slot) * 16);
                 }
             };
-            read(0);
+            auto multiply = [&](auto all) {                          // all: the quarter has chunks for the whole trip
+                read(0);
 #pragma unroll
-            for (int u = 0; u < NB; ++u) {
-                if (u + 1 < NB) read(u + 1);
-                asm volatile("" ::: "memory");       // (no further ahead: their registers)
-                float a[8];
+                for (int u = 0; u < NB; ++u) {
+                    if (!decltype(all)::value && c0 + c + u >= c1) break;
+                    if (u + 1 < NB) read(u + 1);
+                    asm volatile("" ::: "memory");       // (no further ahead: their registers)
+                    float a[8];
+                    values(xv[u], 2 * (c0 + c + u) + h, true, a);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) a[i] = xv[u].value(i);
-                if constexpr (SRC32) {      // every piece of the workgroup's rows is some lane's once per block of experts
-                    const int piece = 2 * (c0 + c + u) + h;
-                    union { uint4 q; T t[8]; } o;
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        o.t[i] = (T)a[i];
-                        a[i] = (float)o.t[i];
-                    }
-                    if (e0 == 0 && c0 + c + u < c1 && piece < pieces && tok_ok) *reinterpret_cast<uint4*>(x + xat + (size_t)piece * 8) = o.q;
+                    for (int i = 0; i < 8; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[u & 1][i >> 2][i & 3], acc, 0, 0, 0);
                 }
-#pragma unroll
-                for (int i = 0; i < 8; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[u & 1][i >> 2][i & 3], acc, 0, 0, 0);
-            }
+            };
+            if constexpr (MODE == GR_WHOLE) multiply(std::true_type());
+            else if (!SRC32 && c0 + c + NB <= c1) multiply(std::true_type());
+            else multiply(std::false_type());
+        }
         }
         __syncthreads();                                             // the operands have been read
 #pragma unroll
@@ -671,21 +757,30 @@ bool gate_router_supported(int d, int E, int x_dt) {
     return E <= GATE_ROUTER_MAX_E && (d % 8) == 0 && (x_dt == HEXA_F32 || x_dt == HEXA_BF16 || x_dt == HEXA_F16);
 }
 namespace {
-template <typename T, bool LI, int ROUND>
-int launch_gate_router_t(float* logits, float* scores, int32_t* idx, const void* x, const float* x_src, const float* wg, const float* noise, float noise_scale,
+template <typename T, bool LI, int ROUND, int MODE>
+int launch_gate_router_k(float* logits, float* scores, int32_t* idx, const void* x, const float* x_src, const float* wg, const float* noise, float noise_scale,
                          int T_, int d, int E, int k, float* ws, int32_t* hist, const LiK& li, RoundAllK* round, hipStream_t st) {
     const int nb = div_up(T_, ROUTER_TB);
     const size_t lds = sizeof(float) * router4_lds_floats(E, k, hist != nullptr, false);
-    constexpr size_t most = sizeof(float) * router4_lds_floats(GATE_ROUTER_MAX_E, MAX_TOPK, true, false);
-    if (int rc = allow_router_lds<gate_router_kernel<T, LI, ROUND>, GR_BYTES, most>(lds)) return rc;
+    constexpr size_t fixed = MODE == GR_DIRECT ? GR_DIRECT_BYTES : GR_BYTES;
+    constexpr size_t most = sizeof(float) * router4_lds_floats(MODE == GR_DIRECT ? GR_DIRECT_E : GATE_ROUTER_MAX_E, MAX_TOPK, true, false);
+    if (int rc = allow_router_lds<gate_router_kernel<T, LI, ROUND, MODE>, fixed, most>(lds)) return rc;
     RoundAllK r{};
     if (round) r = *round;
     r.blocks = (int)((r.n + GATE_ROUTER_NT * 8 * ROUND_STEPS - 1) / (GATE_ROUTER_NT * 8 * ROUND_STEPS));
     using X = std::conditional_t<ROUND == ROUND_TOKENS, T*, const T*>;
-    hipLaunchKernelGGL((gate_router_kernel<T, LI, ROUND>), dim3(nb + r.blocks), dim3(GATE_ROUTER_NT), lds, st, logits, scores, idx, ws,
+    hipLaunchKernelGGL((gate_router_kernel<T, LI, ROUND, MODE>), dim3(nb + r.blocks), dim3(GATE_ROUTER_NT), lds, st, logits, scores, idx, ws,
                        ws + (size_t)nb * E, (X)x, x_src, wg, noise, noise_scale, T_, d, E, k, hist, nb, li, r);
     HEXA_CHECK_LAUNCH("gate_router");
     return HEXA_OK;
+}
+template <typename T, bool LI, int ROUND, typename... Args>
+int launch_gate_router_t(int d, int E, Args... args) {
+    const int mode = gate_router_mode(d, E, ROUND == ROUND_TOKENS);
+    if (mode == GR_DIRECT) return launch_gate_router_k<T, LI, ROUND, GR_DIRECT>(args...);
+    if constexpr (ROUND == ROUND_TOKENS)
+        if (mode == GR_WHOLE) return launch_gate_router_k<T, LI, ROUND, GR_WHOLE>(args...);
+    return launch_gate_router_k<T, LI, ROUND, GR_STAGED>(args...);
 }
 }  // namespace
 int launch_gate_router(float* logits, float* scores, int32_t* idx, const void* x, const float* x_src, const float* wg, const float* noise,
@@ -693,8 +788,8 @@ int launch_gate_router(float* logits, float* scores, int32_t* idx, const void* x
                        RoundAllK* round, hipStream_t st) {
     const LiK li{thr, noise, noise_scale, inv_sigma};
 #define HEXA_GATE_ROUTER(TYPE, S)                                                                                                     \
-    return thr ? launch_gate_router_t<TYPE, true, S>(logits, scores, idx, x, x_src, wg, noise, noise_scale, T, d, E, k, ws, hist, li, round, st) \
-               : launch_gate_router_t<TYPE, false, S>(logits, scores, idx, x, x_src, wg, noise, noise_scale, T, d, E, k, ws, hist, li, round, st)
+    return thr ? launch_gate_router_t<TYPE, true, S>(d, E, logits, scores, idx, x, x_src, wg, noise, noise_scale, T, d, E, k, ws, hist, li, round, st) \
+               : launch_gate_router_t<TYPE, false, S>(d, E, logits, scores, idx, x, x_src, wg, noise, noise_scale, T, d, E, k, ws, hist, li, round, st)
     if (x_dt == HEXA_F32) HEXA_GATE_ROUTER(float, ROUND_NONE);
     const bool bf = x_dt == HEXA_BF16;
     if (bf && x_src) HEXA_GATE_ROUTER(__bf16, ROUND_TOKENS);
