@@ -365,16 +365,20 @@ constexpr int GR_QUARTER = 32 * GR_PIECES * 16, GR_BYTES = 4 * GR_QUARTER;   // 
 // Where wg's values come from.  DIRECT: few experts are few lines an instruction, and every lane reads its own row: no barrier between trips, no
 // chunk multiplied that a quarter does not have.  STAGED: through LDS as above, trips cut where a quarter's chunks end.  WHOLE: no trip is cut
 // (384, 768, 1152 columns); for rounded tokens an instance of its own, because beside cut trips it spills 28 registers and the cuts cost it 0.7 to
-// 1 us of 13 to 17.  us of the launch, DIRECT | STAGED, 8 experts.  bf16, 144 and 9216 tokens: 128 wide 7.0, 8.3 | 8.7, 9.8; 768 wide 12.6,
-// 14.5 | 15.5, 16.6; 1024 wide 15.2, 15.9 | 19.6, 20.8; 16 experts 15.5, 16.4 | 20.3, 21.3; 32 experts, 384 wide 11.7, 13.3 | 10.7, 12.3.  Rounded tokens, 144, 18432
-// and 32768 of them: 128 wide 8.5, 12.2, 12.9 | 8.7, 13.9, 15.8; 512 wide 14.8, 25.8, 27.3 | 17.0, 27.1, 29.8; 768 wide 20.1, 34.9, 49.5 | 21.9,
-// 37.5, 43.5; 12 experts, 512 wide 15.7, 26.0, 28.5 | 17.1, 27.5, 29.8, 768 wide 22.1, 36.9, 58.9 | 23.4, 38.5, 49.2.
+// 1 us of 13 to 17.  us of the launch, DIRECT | STAGED, 8 experts, 144, 3600 and 18432 tokens.  bf16 tokens: 128 wide 8.0, 8.7, 11.8 | 9.2, 9.9, 12.4; 768 wide
+// 14.2, 15.3, 24.8 | 16.9, 17.8, 27.1; 1024 wide 16.4, 17.9, 29.5 | 21.0, 22.1, 33.9; 16 experts, 512 wide 12.2, 13.0, 20.2 | 14.9, 15.9, 22.8; 32 experts, 384 wide,
+// 144 and 9216 tokens 11.7, 13.3 | 10.7, 12.3.  Rounded tokens beside 8 experts' weights, d x 4d: 128 wide 8.8, 10.3, 14.1 | 10.4, 11.6, 15.7; 512
+// wide 20.1, 19.5, 28.4 | 23.1, 22.4, 29.6; 640 wide 24.2, 25.3, 42.7 | 26.3, 26.9, 41.2; 1024 wide 46.4, 46.6, 68.7 | 43.2, 44.2, 63.7; 4 experts, 1024 wide 29.9,
+// 31.5, 58.8 | 32.7, 33.4, 59.5.  Against WHOLE: 384 wide 16.3, 16.6, 23.3 | 16.8, 17.2, 23.2, 16 experts 19.6, 19.6, 26.2 | 19.3, 19.4, 24.1; 768 wide 29.2, 33.4,
+// 51.1 | 28.3, 31.1, 48.2; 1152 wide 53.7, 53.9, 80.6 | 47.7, 49.2, 74.2.
 constexpr int GR_DIRECT = 0, GR_STAGED = 1, GR_WHOLE = 2;
 constexpr int GR_DIRECT_E = 16;
 constexpr int GR_AHEAD = 2;              // chunks in registers: one is under way while the other is multiplied
 inline int gate_router_mode(int d, int E, bool tokens) {
-    if (E <= (tokens && d > 512 ? GR_DIRECT_E / 2 : GR_DIRECT_E)) return GR_DIRECT;
-    return tokens && d % (4 * FWD_NB * 16) == 0 ? GR_WHOLE : GR_STAGED;
+    if (!tokens) return E <= GR_DIRECT_E ? GR_DIRECT : GR_STAGED;
+    const bool whole = d % (4 * FWD_NB * 16) == 0;
+    if (E <= GR_DIRECT_E && (whole ? E <= 8 && d <= 512 : d <= 512 || (d <= 1024 && E * d <= 5120))) return GR_DIRECT;
+    return whole ? GR_WHOLE : GR_STAGED;
 }
 constexpr int GR_DIRECT_BYTES = 2 * 4 * 16 * 64 * 4;                     // the partial sums
 static_assert(GR_BYTES >= GR_DIRECT_BYTES, "the partial sums fit in the operands' place");
@@ -394,6 +398,7 @@ __global__ __launch_bounds__(GATE_ROUTER_NT, 4) void gate_router_kernel(
     float (*part)[4][16][64] = reinterpret_cast<float (*)[4][16][64]>(operands);    // [token block][quarter of d][result register][lane]
     constexpr bool SRC32 = ROUND == ROUND_TOKENS;
     constexpr int NB = FWD_NB;
+    constexpr bool WHOLE = MODE == GR_WHOLE;         // every quarter is whole trips, every chunk two pieces: nothing is asked for
     if (ROUND != ROUND_NONE && (int)blockIdx.x >= nblocks) {
         round_all_body(round, blockIdx.x - nblocks);
         return;
@@ -437,7 +442,7 @@ __global__ __launch_bounds__(GATE_ROUTER_NT, 4) void gate_router_kernel(
                     o.t[i] = (T)a[i];
                     a[i] = (float)o.t[i];
                 }
-                if (e0 == 0 && ok && piece < pieces && tok_ok) *reinterpret_cast<uint4*>(x + xat + (size_t)piece * 8) = o.q;
+                if (e0 == 0 && ok && (WHOLE || piece < pieces) && tok_ok) *reinterpret_cast<uint4*>(x + xat + (size_t)piece * 8) = o.q;
             }
         };
         if constexpr (MODE == GR_DIRECT && SRC32) {
@@ -512,15 +517,15 @@ __global__ __launch_bounds__(GATE_ROUTER_NT, 4) void gate_router_kernel(
                 int p = slot - gr_turn(row);
                 if (p < 0) p += GR_PIECES;
                 const int col = (c0 + c) * 16 + p * 4;
-                if (e0 + row >= E || c0 + c + (p >> 2) >= c1) continue;     // (those columns of the logits are nobody's, those chunks not multiplied)
-                const float* src = col < d ? wg + (size_t)(e0 + row) * d + col : reinterpret_cast<const float*>(g_gate_zeros);
+                if (e0 + row >= E || (!WHOLE && c0 + c + (p >> 2) >= c1)) continue;     // (those columns of the logits are nobody's, those chunks not multiplied)
+                const float* src = WHOLE || col < d ? wg + (size_t)(e0 + row) * d + col : reinterpret_cast<const float*>(g_gate_zeros);
                 dma16(src, operands + quarter * GR_QUARTER + (blk * (GR_QUARTER / 2048) + i) * 1024);
             }
             Raw8<X> xv[NB];
 #pragma unroll
             for (int u = 0; u < NB; ++u) {
                 const int piece = 2 * (c0 + c + u) + h;
-                const bool ok = c0 + c + u < c1 && piece < pieces;
+                const bool ok = WHOLE || (c0 + c + u < c1 && piece < pieces);
                 xv[u].load(xrow + (ok ? piece : 0) * 8, ok && tok_ok);
             }
             wait_vmcnt<0>();                                         // this wavefront's copies have landed: the barrier waits for LDS accesses only
@@ -549,7 +554,7 @@ __global__ __launch_bounds__(GATE_ROUTER_NT, 4) void gate_router_kernel(
                     for (int i = 0; i < 8; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[u & 1][i >> 2][i & 3], acc, 0, 0, 0);
                 }
             };
-            if constexpr (MODE == GR_WHOLE) multiply(std::true_type());
+            if constexpr (WHOLE) multiply(std::true_type());
             else if (!SRC32 && c0 + c + NB <= c1) multiply(std::true_type());
             else multiply(std::false_type());
         }

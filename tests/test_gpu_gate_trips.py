@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 
 # 8 to 384 columns are one trip of one to six chunks, 392 two (the second of one chunk for some quarters and none for others), 1160 four.  Up to 16 experts
-# (rounded tokens, above 512 columns: 8) have no trips: a quarter of no, one, an even and an odd number of chunks, a last chunk of one piece
+# have no trips (rounded tokens: where columns and experts are few): a quarter of no, one, an even and an odd number of chunks, a last chunk of one piece
 DIMS = [8, 16, 24, 40, 64, 72, 104, 128, 136, 192, 200, 256, 264, 320, 384, 392, 448, 512, 520, 768, 776, 1024, 1160]
 
 
